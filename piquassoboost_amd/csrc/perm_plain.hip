@@ -259,17 +259,17 @@ void plain_sweep_kernel(PlainParams p) {
     // ---- grid reduction: last block sums the per-block partials ----
     __shared__ bool is_last;
     if (threadIdx.x == 0) {
-        partials[blockIdx.x] = v;
-        __threadfence();
+        ddc_store_through(&partials[blockIdx.x], v);
+        wait_stores();
         const unsigned done = atomicAdd(counter, 1u);
         is_last = (done == gridDim.x - 1);
     }
     __syncthreads();
     if (is_last) {
-        __threadfence();
         ddc s = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
         for (unsigned b = threadIdx.x; b < gridDim.x; b += blockDim.x) {
-            const ddc q = partials[b];
+            const ddc q = ddc_load_through(&partials[b]);
             ddc_add(s, q);
         }
         s = block_reduce(s, red);
@@ -391,18 +391,18 @@ __global__ __launch_bounds__(256) void plain_exact_kernel(ExactParams p) {
         u128 s = 0;
         const int nw = (blockDim.x + kWave - 1) / kWave;
         for (int w = 0; w < nw; ++w) s += red[w];
-        p.partials[2 * blockIdx.x] = (unsigned long long)s;
-        p.partials[2 * blockIdx.x + 1] = (unsigned long long)(s >> 64);
-        __threadfence();
+        store_through(&p.partials[2 * blockIdx.x], (unsigned long long)s);
+        store_through(&p.partials[2 * blockIdx.x + 1], (unsigned long long)(s >> 64));
+        wait_stores();
         const unsigned done = atomicAdd(p.counter, 1u);
         is_last = (done == gridDim.x - 1);
     }
     __syncthreads();
     if (is_last && threadIdx.x == 0) {
-        __threadfence();
         u128 s = 0;
+#pragma unroll 8
         for (unsigned b = 0; b < gridDim.x; ++b)
-            s += ((u128)p.partials[2 * b + 1] << 64) | p.partials[2 * b];
+            s += ((u128)load_through(&p.partials[2 * b + 1]) << 64) | load_through(&p.partials[2 * b]);
         p.out[0] = (unsigned long long)s;
         p.out[1] = (unsigned long long)(s >> 64);
         *p.counter = 0u;
