@@ -99,50 +99,29 @@ __device__ __forceinline__ void add_row(double (&cr)[NC], double (&ci)[NC],
     }
 }
 
-// colsum += s * row, s = +/-1 per lane.
+// LDS of a block's seeds.  Rows are an odd number of 16-byte elements apart, so that
+// lanes reading eight different rows of `lanes` at one column hit different banks.
 template <int NC>
-__device__ __forceinline__ void add_row_signed(double (&cr)[NC], double (&ci)[NC],
-                                               const double2* __restrict__ row, double s) {
-#pragma unroll
-    for (int j = 0; j < NC; ++j) {
-        const double2 v = row[j];
-        cr[j] = fma(s, v.x, cr[j]);
-        ci[j] = fma(s, v.y, ci[j]);
-    }
-}
+struct SeedLds {
+    static constexpr int P = NC | 1;
+    double2 rows[(NC + 1) * P];  // A
+    double2 lanes[16 * P];       // the lane rows' sums for lane bits 0-2 (8 rows), then bits 3-5
+    double2 base[4 * P];         // per wave: anchor, walk and group rows at its seed
+};
 
+// One wave's run of the sweep over the R rows of the +-2A table at Mb: the lane's
+// part of the sum, without the lane sign.  Every wave of the block calls it (barriers).
 template <int NC>
-// Up to 32 columns the sweep fits in 168 VGPRs: ask for three waves per SIMD
-// so that scalar-load and FP64 latencies of one wave hide behind the others.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NC <= 32 ? 3 : 1)))
-void plain_sweep_kernel(PlainParams p) {
-    __shared__ ddc red[256 / kWave];
-    // batch of equal-size matrices: blockIdx.y is the matrix, gridDim.x blocks each
-    const unsigned task = blockIdx.y;
-    ddc* const partials = p.partials + (size_t)task * gridDim.x;
-    unsigned* const counter = p.counter + task;
-    double* const out = p.out + 6 * (size_t)task;
-
-    const int lane = threadIdx.x & (kWave - 1);
-    // the wave index as a scalar: the run bounds, walk positions and row offsets
-    // derived from it are then uniform for the compiler too (scalar loads, SGPR
-    // operands), not only in fact
-    const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / kWave) +
-                         __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) / kWave;
-
-    const int R = p.R;
-    const int K = p.K;  // walk bits:  rows R-K .. R-1
-    const int B = p.B;  // lane bits:  rows R-K-B .. R-K-1
-    const int H = p.H;  // group bits: rows 1 .. R-1-K-B
+__device__ __forceinline__ void sweep_run(const char* __restrict__ Mb, const int R, const int K, const int B,
+                                          const int H, const int64_t wave, const int64_t nwaves, const int lane,
+                                          SeedLds<NC>& lds, double& tr, double& ti) {
+    // K walk bits: rows R-K .. R-1; B lane bits: rows R-K-B .. R-K-1; H group bits: rows 1 .. R-1-K-B
     const unsigned rowb = NC * sizeof(double2);
     // byte offsets of the +2A / -2A rows: row r of +2A at r*rowb, of -2A at (R+r)*rowb
-    const char* __restrict__ Mb = reinterpret_cast<const char*>(p.M2 + (size_t)task * p.m2_stride);
     const unsigned neg = (unsigned)R * rowb;
     const unsigned low_p = (unsigned)(R - 1) * rowb;  // +2A[R-1]
     const unsigned low_m = neg + low_p;               // -2A[R-1]
     const unsigned W = 1u << K;
-    const bool lane_on = lane < (1 << B);
 
     // contiguous run [tau0, tau1) of the walk index tau = group * 2^K + t for
     // this wave, in units of (even, odd) step pairs, so that every resident
@@ -153,41 +132,68 @@ void plain_sweep_kernel(PlainParams p) {
     const int64_t tau0 = (units * wave / nwaves) * step;
     const int64_t tau1 = (units * (wave + 1) / nwaves) * step;
 
-    double tr = 0.0, ti = 0.0;  // lane total, lane sign applied at the end
-    if (tau0 < tau1) {
-        const int64_t g0 = tau0 >> K;
-        unsigned t0 = (unsigned)(tau0 & (int64_t)(W - 1));  // even when K >= 1
-        // ---- seed at (g0, t0): delta_0 = +1, walk row R-1-b is -1 iff bit b of
-        // the Gray code t0 ^ (t0 >> 1), lane row R-1-K-b is -1 iff bit b of the
-        // lane, group row R-1-K-B-h is -1 iff bit h of g0.  Built from the
-        // +/-2A rows and halved (scaling by 2 is exact, so this equals seeding
-        // from A as BBFGPermanentCalculator.hpp:143-167).
-        double cr[NC], ci[NC];
-#pragma unroll
-        for (int j = 0; j < NC; ++j) {
-            const double2 v = reinterpret_cast<const double2*>(Mb)[j];
-            cr[j] = v.x;
-            ci[j] = v.y;
+    // ---- seed at (g0, t0): delta_0 = +1, walk row R-1-b is -1 iff bit b of the Gray
+    // code t0 ^ (t0 >> 1), lane row R-1-K-b is -1 iff bit b of the lane, group row
+    // R-1-K-B-h is -1 iff bit h of g0 (BBFGPermanentCalculator.hpp:143-167).  The
+    // block stages A in LDS once; a lane per column sums the wave-uniform rows, the
+    // lane rows' 2 x 8 partial sums are formed once per block, and a lane's column
+    // sum is the sum of three.  (Adding the rows one after another, each fetched with
+    // scalar loads as in the walk, took 24 us of the 38 us of an n = 20 permanent:
+    // 3072 waves x 20 rows through the scalar caches.)
+    constexpr int P = SeedLds<NC>::P;
+    const int64_t g0 = tau0 >> K;
+    unsigned t0 = (unsigned)(tau0 & (int64_t)(W - 1));  // even when K >= 1
+    const unsigned gray0 = t0 ^ (t0 >> 1);
+    for (int e = threadIdx.x; e < R * NC; e += blockDim.x) {
+        const int i = e / NC;
+        const double2 v = reinterpret_cast<const double2*>(Mb)[e];
+        lds.rows[i * P + e - i * NC] = make_double2(0.5 * v.x, 0.5 * v.y);  // exact
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < 16 * NC; e += blockDim.x) {
+        const int k = e / NC, j = e - k * NC;
+        double2 v = make_double2(0.0, 0.0);
+        for (int b = 0; b < 3; ++b) {
+            const int bit = (k >= 8 ? 3 : 0) + b;
+            if (bit < B) {
+                const double s = ((k >> b) & 1) ? -1.0 : 1.0;
+                const double2 a = lds.rows[(R - 1 - K - bit) * P + j];
+                v.x = fma(s, a.x, v.x);
+                v.y = fma(s, a.y, v.y);
+            }
         }
-        const unsigned gray0 = t0 ^ (t0 >> 1);
-        for (int i = R - K; i < R; ++i) {
-            const unsigned off = (((gray0 >> (R - 1 - i)) & 1u) ? neg : 0u) + (unsigned)i * rowb;
-            add_row<NC>(cr, ci, reinterpret_cast<const double2*>(Mb + off));
-        }
-        for (int b = 0; b < B; ++b) {
-            const int row = R - 1 - K - b;
-            const double s = ((lane >> b) & 1) ? -1.0 : 1.0;
-            add_row_signed<NC>(cr, ci, reinterpret_cast<const double2*>(Mb + (size_t)row * rowb), s);
+        lds.lanes[k * P + j] = v;
+    }
+    double2* const base = lds.base + (threadIdx.x / kWave) * P;
+    if (lane < NC) {
+        double2 v = lds.rows[lane];
+        for (int b = 0; b < K; ++b) {
+            const double s = ((gray0 >> b) & 1u) ? -1.0 : 1.0;
+            const double2 a = lds.rows[(R - 1 - b) * P + lane];
+            v.x = fma(s, a.x, v.x);
+            v.y = fma(s, a.y, v.y);
         }
         for (int h = 0; h < H; ++h) {
-            const int row = R - 1 - K - B - h;
-            const unsigned off = (((g0 >> h) & 1) ? neg : 0u) + (unsigned)row * rowb;
-            add_row<NC>(cr, ci, reinterpret_cast<const double2*>(Mb + off));
+            const double s = ((g0 >> h) & 1) ? -1.0 : 1.0;
+            const double2 a = lds.rows[(R - 1 - K - B - h) * P + lane];
+            v.x = fma(s, a.x, v.x);
+            v.y = fma(s, a.y, v.y);
         }
+        base[lane] = v;
+    }
+    __syncthreads();
+
+    tr = 0.0;  // lane total, lane sign applied at the end
+    ti = 0.0;
+    if (tau0 < tau1) {
+        double cr[NC], ci[NC];
+        const double2* const lo = lds.lanes + (lane & 7) * P;
+        const double2* const hi = lds.lanes + (8 + (lane >> 3)) * P;
 #pragma unroll
         for (int j = 0; j < NC; ++j) {
-            cr[j] *= 0.5;
-            ci[j] *= 0.5;
+            const double2 u = base[j], v = lo[j], w = hi[j];
+            cr[j] = u.x + (v.x + w.x);
+            ci[j] = u.y + (v.y + w.y);
         }
 
         for (int64_t g = g0;;) {
@@ -250,6 +256,33 @@ void plain_sweep_kernel(PlainParams p) {
             }
         }
     }
+}
+
+template <int NC>
+// Up to 32 columns the sweep fits in 168 VGPRs: ask for three waves per SIMD
+// so that scalar-load and FP64 latencies of one wave hide behind the others.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NC <= 32 ? 3 : 1)))
+void plain_sweep_kernel(PlainParams p) {
+    __shared__ ddc red[256 / kWave];
+    __shared__ SeedLds<NC> seeds;
+    // batch of equal-size matrices: blockIdx.y is the matrix, gridDim.x blocks each
+    const unsigned task = blockIdx.y;
+    ddc* const partials = p.partials + (size_t)task * gridDim.x;
+    unsigned* const counter = p.counter + task;
+    double* const out = p.out + 6 * (size_t)task;
+
+    const int lane = threadIdx.x & (kWave - 1);
+    // the wave index as a scalar: the run bounds, walk positions and row offsets
+    // derived from it are then uniform for the compiler too (scalar loads, SGPR
+    // operands), not only in fact
+    const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / kWave) +
+                         __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) / kWave;
+    const char* __restrict__ Mb = reinterpret_cast<const char*>(p.M2 + (size_t)task * p.m2_stride);
+
+    double tr, ti;
+    sweep_run<NC>(Mb, p.R, p.K, p.B, p.H, wave, nwaves, lane, seeds, tr, ti);
+    const bool lane_on = lane < (1 << p.B);
     const double ls = (__popc((unsigned)lane) & 1) ? -1.0 : 1.0;
     tr = lane_on ? ls * tr : 0.0;
     ti = lane_on ? ls * ti : 0.0;
