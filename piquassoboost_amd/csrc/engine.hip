@@ -69,7 +69,7 @@ static int set_device_locked(int dev) {
     e = hipGetDeviceProperties(&prop, dev);
     if (e != hipSuccess) return hip_fail(e, "hipGetDeviceProperties");
     g_dev.cus = prop.multiProcessorCount;
-    for (int i = 0; i <= PQB_MAX_COLS; ++i) g_dev.blocks_per_cu[i] = 0;
+    for (int i = 0; i <= PQB_MAX_COLS; ++i) g_dev.blocks_per_cu[0][i] = g_dev.blocks_per_cu[1][i] = 0;
     g_dev.device = dev;
     return PQB_OK;
 }
@@ -105,16 +105,17 @@ int bind_device(int dev, int* device, int* cus) {
     return PQB_OK;
 }
 
-int64_t resident_waves(int nc) {
+int64_t resident_waves(int nc, bool expanded) {
     if (nc < 1 || nc > PQB_MAX_COLS) return 0;
     std::lock_guard<std::mutex> lk(g_dev.mu);
-    if (g_dev.blocks_per_cu[nc] == 0) {
+    int& per_cu = g_dev.blocks_per_cu[expanded][nc];
+    if (per_cu == 0) {
         int nb = 0;
-        hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, plain_kernel_fn(nc), kBlock, 0);
+        hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, plain_kernel_fn(nc, expanded), kBlock, 0);
         if (e != hipSuccess || nb <= 0) nb = 1;
-        g_dev.blocks_per_cu[nc] = nb;
+        per_cu = nb;
     }
-    return (int64_t)g_dev.blocks_per_cu[nc] * (kBlock / kWave) * g_dev.cus;
+    return (int64_t)per_cu * (kBlock / kWave) * g_dev.cus;
 }
 
 // ---------------------------------------------------------------- contexts --
@@ -277,6 +278,54 @@ PlainPlan make_plain_plan(int R, int NC, int64_t waves_resident) {
     return pl;
 }
 
+// The expanded sweep does 10 n instead of 12 n FP64 instructions per pair of sign
+// vectors; its table costs a launch, and device matrices a second sweep launch for the
+// ones that keep all rows.  From 2^24 sign vectors on that pays (all rows / expanded,
+// us, device entries, one box): 1 x 24 50.3 / 53.0, 1 x 25 89 / 86, 1 x 26 169 / 153,
+// 1 x 30 2929 / 2495; 16 x 20 43.2 / 45.5, 64 x 20 138 / 120, 256 x 20 502 / 422;
+// 4 x 22 46.8 / 48.8, 8 x 22 82.7 / 76.6; 512 x 16 61.1 / 60.0, 2048 x 14 65.7 / 61.4.
+// Below 14 columns a table of n^2 quotients per matrix costs more than the walk of
+// 2^(n-2) vectors saves (8192 x 12: 64.7 / 90.3).
+bool plain_expandable(int R, int C, int64_t count) {
+    return R == C && C >= kExpandedMinCols && count >= ((int64_t)1 << std::max(0, 25 - C));
+}
+
+// +-2A of an R x C matrix with row stride ld.
+static void fill_m2(const double* A, int R, int C, int64_t ld, double* t) {
+    const size_t rc = (size_t)R * C;
+    for (int i = 0; i < R; ++i)
+        for (int j = 0; j < C; ++j) {
+            const double re = A[2 * (i * ld + j)], im = A[2 * (i * ld + j) + 1];
+            const size_t q = (size_t)i * C + j;
+            t[2 * q] = 2.0 * re;
+            t[2 * q + 1] = 2.0 * im;
+            t[2 * (q + rc)] = -2.0 * re;
+            t[2 * (q + rc) + 1] = -2.0 * im;
+        }
+}
+
+PlainParams plain_params(const PlainPlan& pl, int R, const double2* m2, int64_t m2_stride, ddc* partials,
+                         unsigned* counter, double* out) {
+    PlainParams p;
+    p.M2 = m2;
+    p.m2_stride = m2_stride;
+    p.R = R;
+    p.K = pl.K;
+    p.B = pl.B;
+    p.H = pl.H;
+    p.by_flag = 0;
+    p.partials = partials;
+    p.counter = counter;
+    p.out = out;
+    p.scale = std::ldexp(1.0, -(R - 1));
+    return p;
+}
+
+static void pack_rows(const double* A, int R, int C, int64_t ld, double* t) {
+    for (int i = 0; i < R; ++i)
+        std::memcpy(t + 2 * (size_t)i * C, A + 2 * i * ld, (size_t)C * sizeof(double2));
+}
+
 // Integer route eligibility.  Fills `ai` (packed R x C int32) when the matrix
 // is integer valued and real, and returns log2 of an upper bound on the sweep's
 // sum S = sum_delta (prod delta) prod_j (sum_i delta_i a_ij) (or -inf when S is
@@ -328,6 +377,8 @@ static bool integer_matrix(const double* A, int64_t R, int64_t C, int64_t ld, st
 }
 
 static bool exact_fits(long double log2_bound) { return log2_bound < 126.5L; }
+
+static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
 typedef __int128 i128;
 
@@ -391,43 +442,35 @@ static int run_exact_locked(Engine& E, const std::vector<int>& ai, int R, int C,
 
 // FP64 route.  The caller holds the lease of E.
 static int run_plain_locked(Engine& E, const double* A, int R, int C, int64_t ld, double* out) {
-    const PlainPlan pl = make_plain_plan(R, C, E.resident_waves_locked(C));
-    const size_t m2_elems = (size_t)2 * R * C;
-    const size_t m2_bytes = m2_elems * sizeof(double2);
+    const bool expanded = plain_expandable(R, C, 1) && plain_expand_row(A, C, ld) >= 0;
+    const int rows = expanded ? R - 1 : R;
+    const PlainPlan pl = make_plain_plan(rows, C, E.resident_waves_locked(C, expanded));
+    const size_t a_bytes = (size_t)R * C * sizeof(double2), m2_bytes = 2 * a_bytes;
     const size_t part_off = kCounterBytes;
     const size_t part_bytes = (size_t)pl.blocks * sizeof(ddc);
-    const size_t out_off = part_off + ((part_bytes + 255) / 256) * 256;
+    const size_t out_off = part_off + round256(part_bytes);
     const size_t m2_off = out_off + 256;
-    int st = E.ensure_buffers_locked(m2_off + m2_bytes, m2_bytes + 256);
+    const size_t a_off = m2_off + round256(m2_bytes);
+    // the upload: the +-2A table, or the matrix whose expanded table a kernel builds
+    const size_t up_bytes = expanded ? a_bytes : m2_bytes;
+    int st = E.ensure_buffers_locked(a_off + a_bytes, up_bytes + 256);
     if (st) return st;
     double* h = static_cast<double*>(E.hbuf);
-    for (int i = 0; i < R; ++i) {
-        for (int j = 0; j < C; ++j) {
-            const double re = A[2 * (i * ld + j)], im = A[2 * (i * ld + j) + 1];
-            const size_t k = (size_t)i * C + j;
-            h[2 * k] = 2.0 * re;
-            h[2 * k + 1] = 2.0 * im;
-            h[2 * (k + (size_t)R * C)] = -2.0 * re;
-            h[2 * (k + (size_t)R * C) + 1] = -2.0 * im;
-        }
-    }
+    if (expanded) pack_rows(A, R, C, ld, h);
+    else fill_m2(A, R, C, ld, h);
     char* d = static_cast<char*>(E.dbuf);
-    hipError_t e = hipMemcpyAsync(d + m2_off, h, m2_bytes, hipMemcpyHostToDevice, E.stream);
+    unsigned* counter = reinterpret_cast<unsigned*>(d);
+    double2* m2 = reinterpret_cast<double2*>(d + m2_off);
+    hipError_t e = hipMemcpyAsync(d + (expanded ? a_off : m2_off), h, up_bytes, hipMemcpyHostToDevice, E.stream);
     if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync");
-    PlainParams p;
-    p.M2 = reinterpret_cast<const double2*>(d + m2_off);
-    p.m2_stride = (int64_t)m2_elems;
-    p.R = R;
-    p.K = pl.K;
-    p.B = pl.B;
-    p.H = pl.H;
-    p.partials = reinterpret_cast<ddc*>(d + part_off);
-    p.counter = reinterpret_cast<unsigned*>(d);
-    p.out = reinterpret_cast<double*>(d + out_off);
-    p.scale = std::ldexp(1.0, -(R - 1));
-    e = launch_plain(C, p, pl.blocks, pl.block, 1, E.stream);
+    if (expanded) e = launch_plain_expand(reinterpret_cast<const double2*>(d + a_off), m2, C, 1, counter, E.stream);
+    if (e == hipSuccess)
+        e = launch_plain(C, expanded,
+                         plain_params(pl, R, m2, 2 * R * C, reinterpret_cast<ddc*>(d + part_off), counter,
+                                      reinterpret_cast<double*>(d + out_off)),
+                         pl.blocks, pl.block, 1, E.stream);
     if (e != hipSuccess) return drain_fail(E, e, "plain sweep launch");
-    double* hout = h + 2 * m2_elems;
+    double* hout = h + up_bytes / sizeof(double);
     e = hipMemcpyAsync(hout, d + out_off, 6 * sizeof(double), hipMemcpyDeviceToHost, E.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(E.stream);
     if (e != hipSuccess) return hip_fail(e, "plain sweep");
@@ -503,8 +546,6 @@ int plain_entry(const double* A, int64_t rows, int64_t cols, int64_t ld, int alg
     return run_plain_locked(E, A, R, C, ld, out);
 }
 
-static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
-
 // ------------------------------------------------------------- list entry --
 //
 // Plain permanents of a list of host matrices (any mix of shapes).  Each
@@ -520,27 +561,37 @@ static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 struct ListItem {
     int64_t idx;
     int R, C;
+    bool expanded;
 };
 
 static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld, std::vector<ListItem>& items,
                             double* out) {
     if (items.empty()) return PQB_OK;
+    for (ListItem& it : items)
+        it.expanded = plain_expandable(it.R, it.C, 1) && plain_expand_row(A[it.idx], it.C, ld[it.idx]) >= 0;
     std::stable_sort(items.begin(), items.end(), [](const ListItem& a, const ListItem& b) {
-        return a.R != b.R ? a.R < b.R : a.C < b.C;
+        return a.R != b.R ? a.R < b.R : (a.C != b.C ? a.C < b.C : a.expanded < b.expanded);
     });
     struct Group {
         size_t first, count;
+        int R, C;
+        bool expanded;
         PlainPlan pl;
+        size_t up_off;            // byte offset in the upload: +-2A tables, or (expanded) the matrices
         size_t part_off, m2_off;  // device byte offsets of the group's partials and tables
     };
     std::vector<Group> groups;
     for (size_t k = 0; k < items.size();) {
+        const ListItem& f = items[k];
         size_t e = k;
-        while (e < items.size() && items[e].R == items[k].R && items[e].C == items[k].C) ++e;
+        while (e < items.size() && items[e].R == f.R && items[e].C == f.C && items[e].expanded == f.expanded) ++e;
         Group g;
         g.first = k;
         g.count = e - k;
-        g.pl = make_plain_plan(items[k].R, items[k].C, E.resident_waves_locked(items[k].C));
+        g.R = f.R;
+        g.C = f.C;
+        g.expanded = f.expanded;
+        g.pl = make_plain_plan(f.expanded ? f.R - 1 : f.R, f.C, E.resident_waves_locked(f.C, f.expanded));
         groups.push_back(g);
         k = e;
     }
@@ -553,61 +604,58 @@ static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld
         g.part_off = off;
         off += round256(g.count * (size_t)g.pl.blocks * sizeof(ddc));
     }
-    size_t m2_total = 0;
+    // the upload holds the +-2A tables of the all-rows groups, used in place, and the
+    // matrices of the expanded ones, whose tables a kernel builds behind it
+    const size_t up_base = off;
+    size_t up_total = 0;
     for (Group& g : groups) {
-        g.m2_off = off + m2_total;
-        m2_total += g.count * (size_t)2 * items[g.first].R * items[g.first].C * sizeof(double2);
+        g.up_off = up_total;
+        g.m2_off = up_base + up_total;
+        up_total += round256(g.count * (size_t)g.R * g.C * sizeof(double2) * (g.expanded ? 1 : 2));
     }
-    const size_t m2_base = off;
-    int st = E.ensure_buffers_locked(m2_base + m2_total, m2_total + n * 6 * sizeof(double));
+    off += up_total;
+    for (Group& g : groups)
+        if (g.expanded) {
+            g.m2_off = off;
+            off += round256(g.count * (size_t)2 * g.R * g.C * sizeof(double2));
+        }
+    int st = E.ensure_buffers_locked(off, up_total + n * 6 * sizeof(double));
     if (st) return st;
     double* h = static_cast<double*>(E.hbuf);
     for (const Group& g : groups) {
-        const int R = items[g.first].R, C = items[g.first].C;
-        const size_t rc = (size_t)R * C;
-        double* hg = h + (g.m2_off - m2_base) / sizeof(double);
+        const size_t rc = (size_t)g.R * g.C;
+        double* hg = h + g.up_off / sizeof(double);
         for (size_t k = 0; k < g.count; ++k) {
-            const ListItem& it = items[g.first + k];
-            const double* a = A[it.idx];
-            const int64_t l = ld[it.idx];
-            double* t = hg + 4 * rc * k;  // +2A then -2A, complex interleaved
-            for (int i = 0; i < R; ++i)
-                for (int j = 0; j < C; ++j) {
-                    const double re = a[2 * (i * l + j)], im = a[2 * (i * l + j) + 1];
-                    const size_t q = (size_t)i * C + j;
-                    t[2 * q] = 2.0 * re;
-                    t[2 * q + 1] = 2.0 * im;
-                    t[2 * (q + rc)] = -2.0 * re;
-                    t[2 * (q + rc) + 1] = -2.0 * im;
-                }
+            const int64_t i = items[g.first + k].idx;
+            if (g.expanded) pack_rows(A[i], g.R, g.C, ld[i], hg + 2 * rc * k);
+            else fill_m2(A[i], g.R, g.C, ld[i], hg + 4 * rc * k);
         }
     }
     char* d = static_cast<char*>(E.dbuf);
-    hipError_t e = hipMemsetAsync(d + cnt_off, 0, n * sizeof(unsigned), E.stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(d + m2_base, h, m2_total, hipMemcpyHostToDevice, E.stream);
+    unsigned* counters = reinterpret_cast<unsigned*>(d + cnt_off);
+    hipError_t e = hipMemsetAsync(counters, 0, n * sizeof(unsigned), E.stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(d + up_base, h, up_total, hipMemcpyHostToDevice, E.stream);
     if (e != hipSuccess) return drain_fail(E, e, "list upload");
     constexpr size_t kMaxGridY = 65535;
     for (const Group& g : groups) {
-        const int R = items[g.first].R, C = items[g.first].C;
-        const int64_t m2n = (int64_t)2 * R * C;
+        double2* const m2 = reinterpret_cast<double2*>(d + g.m2_off);
+        const int64_t m2n = (int64_t)2 * g.R * g.C;
+        if (g.expanded) {
+            e = launch_plain_expand(reinterpret_cast<const double2*>(d + up_base + g.up_off), m2, g.C,
+                                    (int64_t)g.count, counters + g.first, E.stream);
+            if (e != hipSuccess) return drain_fail(E, e, "prep launch");
+        }
         for (size_t o = 0; o < g.count; o += kMaxGridY) {
             const size_t nt = std::min(kMaxGridY, g.count - o);
-            PlainParams p;
-            p.M2 = reinterpret_cast<const double2*>(d + g.m2_off) + (o * (size_t)m2n);
-            p.m2_stride = m2n;
-            p.R = R;
-            p.K = g.pl.K;
-            p.B = g.pl.B;
-            p.H = g.pl.H;
-            p.partials = reinterpret_cast<ddc*>(d + g.part_off) + o * (size_t)g.pl.blocks;
-            p.counter = reinterpret_cast<unsigned*>(d + cnt_off) + g.first + o;
-            p.out = reinterpret_cast<double*>(d + out_off) + 6 * (g.first + o);
-            p.scale = std::ldexp(1.0, -(R - 1));
-            e = launch_plain(C, p, g.pl.blocks, g.pl.block, (int)nt, E.stream);
+            const PlainParams p = plain_params(
+                g.pl, g.R, m2 + o * (size_t)m2n, m2n,
+                reinterpret_cast<ddc*>(d + g.part_off) + o * (size_t)g.pl.blocks, counters + g.first + o,
+                reinterpret_cast<double*>(d + out_off) + 6 * (g.first + o));
+            e = launch_plain(g.C, g.expanded, p, g.pl.blocks, g.pl.block, (int)nt, E.stream);
             if (e != hipSuccess) return drain_fail(E, e, "list sweep launch");
         }
     }
-    double* hout = h + m2_total / sizeof(double);
+    double* hout = h + up_total / sizeof(double);
     e = hipMemcpyAsync(hout, d + out_off, n * 6 * sizeof(double), hipMemcpyDeviceToHost, E.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(E.stream);
     if (e != hipSuccess) return drain_fail(E, e, "list sweep");
@@ -645,7 +693,7 @@ int list_entry(const double* const* A, const int64_t* rows, const int64_t* cols,
         if (precision == PQB_PREC_EXACT && !exact_ok)
             return bad(i, PQB_ERR_EXACT, is_int ? "exact mode: the permanent may exceed the 128-bit range"
                                                 : "exact mode needs a real integer-valued matrix");
-        const ListItem it{i, (int)rows[i], (int)cols[i]};
+        const ListItem it{i, (int)rows[i], (int)cols[i], false};
         if (exact_ok)
             exact.emplace_back(i, std::move(ai));
         else if (precision == PQB_PREC_INF)
@@ -708,16 +756,44 @@ int plain_device_check(int64_t count, int64_t rows, int64_t cols) {
     return PQB_OK;
 }
 
-// Launch plan of a batch of `count` equal-size matrices: the single-matrix
-// plan for the resident waves divided among the matrices.
-int plain_device_blocks(int64_t count, int R, int C, PlainPlan* plan, int64_t* blocks_per_matrix) {
+// Launch plans of a batch of `count` equal-size matrices: the single-matrix plan for
+// the resident waves divided among the matrices, of the sweep over all rows and (where
+// the matrices may be expanded) of the expanded one.  Each matrix takes one of the two
+// and the partials have room for either.
+static int plain_device_plan(int64_t count, int R, int C, PlainPlan* pl, PlainPlan* xp,
+                             int64_t* blocks_per_matrix) {
     const int st = bind_device(-1, nullptr, nullptr);
     if (st) return st;
-    const int64_t wr = resident_waves(C);
-    const PlainPlan pl = make_plain_plan(R, C, std::max<int64_t>(1, wr / count));
-    if (pl.blocks > kMaxBlocks) return fail(PQB_ERR_SIZE, "launch plan exceeds the workspace layout");
-    if (plan) *plan = pl;
-    *blocks_per_matrix = pl.blocks;
+    *pl = make_plain_plan(R, C, std::max<int64_t>(1, resident_waves(C, false) / count));
+    *blocks_per_matrix = pl->blocks;
+    if (plain_expandable(R, C, count)) {
+        *xp = make_plain_plan(R - 1, C, std::max<int64_t>(1, resident_waves(C, true) / count));
+        *blocks_per_matrix = std::max(pl->blocks, xp->blocks);
+    }
+    if (*blocks_per_matrix > kMaxBlocks) return fail(PQB_ERR_SIZE, "launch plan exceeds the workspace layout");
+    return PQB_OK;
+}
+
+// The launches of `count` packed R x C device matrices: tables, then the sweep over all
+// rows, then (plan xp given) the expanded one; counters zero before, zero after.
+int plain_device_launch(const double2* dA, int64_t count, int R, int C, const PlainPlan& pl, const PlainPlan* xp,
+                        double2* m2, ddc* partials, unsigned* counters, double* d_out, hipStream_t st) {
+    const int64_t m2n = (int64_t)2 * R * C;
+    hipError_t e = xp ? launch_plain_expand(dA, m2, C, count, counters, st)
+                      : launch_plain_prep(dA, m2, R * C, count, st);
+    if (e != hipSuccess) return hip_fail(e, "prep launch");
+    constexpr int64_t kMaxGridY = 65535;
+    for (const PlainPlan* q : {&pl, xp}) {
+        if (!q) continue;
+        for (int64_t off = 0; off < count; off += kMaxGridY) {
+            const int64_t nt = std::min(kMaxGridY, count - off);
+            PlainParams p = plain_params(*q, R, m2 + off * m2n, m2n, partials + off * q->blocks, counters + off,
+                                         d_out + 6 * off);
+            p.by_flag = xp ? 1 : 0;
+            e = launch_plain(C, q == xp, p, q->blocks, q->block, (int)nt, st);
+            if (e != hipSuccess) return hip_fail(e, "plain sweep launch");
+        }
+    }
     return PQB_OK;
 }
 
@@ -727,9 +803,9 @@ int plain_device_run(const double* dA, int64_t count, int64_t rows, int64_t cols
     int s = plain_device_check(count, rows, cols);
     if (s) return s;
     const int R = (int)rows, C = (int)cols;
-    PlainPlan pl;
+    PlainPlan pl, xp;
     int64_t bpm = 0;
-    s = plain_device_blocks(count, R, C, &pl, &bpm);
+    s = plain_device_plan(count, R, C, &pl, &xp, &bpm);
     if (s) return s;
     if (single) bpm = kMaxBlocks;  // the documented single-matrix layout
     if (work_bytes < plain_device_bytes(count, rows, cols, bpm)) return fail(PQB_ERR_ARG, "workspace too small");
@@ -737,27 +813,8 @@ int plain_device_run(const double* dA, int64_t count, int64_t rows, int64_t cols
     unsigned* counters = reinterpret_cast<unsigned*>(w);
     ddc* partials = reinterpret_cast<ddc*>(w + round256((size_t)count * sizeof(unsigned)));
     double2* m2 = reinterpret_cast<double2*>(reinterpret_cast<char*>(partials) + (size_t)count * bpm * sizeof(ddc));
-    const int64_t m2n = (int64_t)2 * R * C;
-    hipError_t e = launch_plain_prep(reinterpret_cast<const double2*>(dA), m2, R * C, count, st);
-    if (e != hipSuccess) return hip_fail(e, "prep launch");
-    constexpr int64_t kMaxGridY = 65535;
-    for (int64_t off = 0; off < count; off += kMaxGridY) {
-        const int64_t nt = std::min(kMaxGridY, count - off);
-        PlainParams p;
-        p.M2 = m2 + off * m2n;
-        p.m2_stride = m2n;
-        p.R = R;
-        p.K = pl.K;
-        p.B = pl.B;
-        p.H = pl.H;
-        p.partials = partials + off * pl.blocks;
-        p.counter = counters + off;
-        p.out = d_out + 6 * off;
-        p.scale = std::ldexp(1.0, -(R - 1));
-        e = launch_plain(C, p, pl.blocks, pl.block, (int)nt, st);
-        if (e != hipSuccess) return hip_fail(e, "plain sweep launch");
-    }
-    return PQB_OK;
+    return plain_device_launch(reinterpret_cast<const double2*>(dA), count, R, C, pl,
+                               plain_expandable(R, C, count) ? &xp : nullptr, m2, partials, counters, d_out, st);
 }
 
 // Repeated-row permanent: a batch of one task (batch.hip applies the
@@ -850,7 +907,8 @@ int pqb_perm_batch_device_workspace(int64_t count, int64_t rows, int64_t cols, s
     int st = plain_device_check(count, rows, cols);
     if (st) return st;
     int64_t bpt = 0;
-    st = plain_device_blocks(count, (int)rows, (int)cols, nullptr, &bpt);
+    PlainPlan pl, xp;
+    st = plain_device_plan(count, (int)rows, (int)cols, &pl, &xp, &bpt);
     if (st) return st;
     *bytes = plain_device_bytes(count, rows, cols, bpt);
     return PQB_OK;
@@ -870,7 +928,7 @@ int pqb_plain_plan(int64_t rows, int64_t cols, int64_t waves_resident, int64_t* 
     if (wr <= 0) {
         const int st = bind_device(-1, nullptr, nullptr);
         if (st) return st;
-        wr = resident_waves((int)cols);
+        wr = resident_waves((int)cols, false);
     }
     const PlainPlan pl = make_plain_plan((int)rows, (int)cols, wr);
     plan[0] = pl.K;

@@ -50,7 +50,7 @@ struct ScratchDevice {
     bool ready = false;
     char* ptr = nullptr;  // device address of this GPU's `scratch`
     int cus = 0;
-    int blocks_per_cu[PQB_MAX_COLS + 1] = {0};
+    int blocks_per_cu[2][PQB_MAX_COLS + 1] = {};  // [expanded]
 };
 
 std::mutex g_scratch_mu;
@@ -71,7 +71,7 @@ __global__ void noalloc_prep_kernel(const double2* __restrict__ A, double2* __re
 
 // Set-up of the current device, once: the device address of `scratch`, the CU
 // count and (per column count, on first use) the resident blocks of the sweep.
-int scratch_device(int nc, ScratchDevice** out, int64_t* waves_resident) {
+int scratch_device(int nc, bool expandable, ScratchDevice** out, int64_t (&waves_resident)[2]) {
     int dev = -1;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
@@ -90,13 +90,16 @@ int scratch_device(int nc, ScratchDevice** out, int64_t* waves_resident) {
         s.cus = cus;
         s.ready = true;
     }
-    if (s.blocks_per_cu[nc] == 0) {
-        int nb = 0;
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, plain_kernel_fn(nc), kBlock, 0);
-        if (e != hipSuccess || nb <= 0) nb = 1;
-        s.blocks_per_cu[nc] = nb;
+    for (int x = 0; x <= (expandable ? 1 : 0); ++x) {
+        int& per_cu = s.blocks_per_cu[x][nc];
+        if (per_cu == 0) {
+            int nb = 0;
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, plain_kernel_fn(nc, x != 0), kBlock, 0);
+            if (e != hipSuccess || nb <= 0) nb = 1;
+            per_cu = nb;
+        }
+        waves_resident[x] = (int64_t)per_cu * (kBlock / kWave) * s.cus;
     }
-    *waves_resident = (int64_t)s.blocks_per_cu[nc] * (kBlock / kWave) * s.cus;
     *out = &s;
     return PQB_OK;
 }
@@ -113,12 +116,15 @@ static int noalloc_entry(const double* dA, int64_t rows, int64_t cols, double* d
                                       std::to_string(PQB_MAX_COLS));
     const int R = (int)rows, C = (int)cols;
     ScratchDevice* s = nullptr;
-    int64_t wr = 0;
-    int rc = scratch_device(C, &s, &wr);
+    const bool expandable = plain_expandable(R, C, 1);
+    int64_t wr[2] = {1, 1};
+    int rc = scratch_device(C, expandable, &s, wr);
     if (rc) return rc;
-    // the launch plan of pqb_perm_device for one matrix: the values agree bit for bit
-    const PlainPlan pl = make_plain_plan(R, C, std::max<int64_t>(1, wr));
-    if (pl.blocks > kMaxBlocks)
+    // the launch plans of pqb_perm_device for one matrix: the values agree bit for bit
+    const PlainPlan pl = make_plain_plan(R, C, std::max<int64_t>(1, wr[0]));
+    PlainPlan xp;
+    if (expandable) xp = make_plain_plan(R - 1, C, std::max<int64_t>(1, wr[1]));
+    if (std::max(pl.blocks, xp.blocks) > kMaxBlocks)
         return fail(PQB_ERR_SIZE, "launch plan exceeds the static scratch buffer (" + std::to_string(kMaxBlocks) +
                                       " partials)");
     const size_t table = (size_t)2 * R * C * sizeof(double2);
@@ -126,24 +132,17 @@ static int noalloc_entry(const double* dA, int64_t rows, int64_t cols, double* d
     unsigned* counter = reinterpret_cast<unsigned*>(s->ptr);
     ddc* partials = reinterpret_cast<ddc*>(s->ptr + kScratchCounter);
     double2* m2 = reinterpret_cast<double2*>(s->ptr + kScratchCounter + kScratchPartials);
+    if (expandable)  // the table kernel writes the counter too
+        return plain_device_launch(reinterpret_cast<const double2*>(dA), 1, R, C, pl, &xp, m2, partials, counter,
+                                   d_out, st);
     const int n = R * C;
     const int bd = 256;
     hipLaunchKernelGGL(noalloc_prep_kernel, dim3((unsigned)((n + bd - 1) / bd)), dim3(bd), 0, st,
                        reinterpret_cast<const double2*>(dA), m2, n, counter);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "prep launch");
-    PlainParams p;
-    p.M2 = m2;
-    p.m2_stride = (int64_t)2 * n;
-    p.R = R;
-    p.K = pl.K;
-    p.B = pl.B;
-    p.H = pl.H;
-    p.partials = partials;
-    p.counter = counter;
-    p.out = d_out;
-    p.scale = std::ldexp(1.0, -(R - 1));
-    e = launch_plain(C, p, pl.blocks, pl.block, 1, st);
+    e = launch_plain(C, false, plain_params(pl, R, m2, (int64_t)2 * n, partials, counter, d_out), pl.blocks, pl.block,
+                     1, st);
     if (e != hipSuccess) return hip_fail(e, "plain sweep launch");
     return PQB_OK;
 }

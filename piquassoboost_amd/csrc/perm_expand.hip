@@ -1,0 +1,182 @@
+// Tables of the expanded plain sweep: perm(A) of a square matrix by expansion
+// along one row r,
+//
+//     perm(A) = sum_j a_rj perm(A without row r and column j)
+//             = (prod_j a_rj) sum_j perm(S without column j),   S_ij = a_ij / a_rj, i != r,
+//
+// so that the sign-vector sum runs over the n-1 rows of S and each vector's term
+// is the coefficient of x in prod_j (c_j + x), c = the column sums of S: half as
+// many vectors as the sum over all n rows (BBFGPermanentCalculator.hpp:87-235),
+// at 10 n instead of 2 x 6 n FP64 instructions per pair of them
+// (add_expanded_term in perm_plain.hip).
+//
+// One block per matrix.  The row with the largest smallest entry is expanded;
+// a matrix keeps the all-rows table when
+//  * a row without an entry below 2^-16 of the matrix's largest and outside
+//    [2^-20, 2^20] does not exist (zeros, sparse rows): the scaled column sums
+//    are then below 40 x 2^16.5, their products over 40 columns and the sum over
+//    2^39 vectors below 2^950, and the product of the scales is above 2^-800;
+//  * an entry is not finite or beyond 2^20;
+//  * every entry is a (Gaussian) integer: small integer matrices sum without
+//    rounding, which a division would lose.
+// Quotients are formed in double-double and rounded once, the product of the
+// scales is kept in double-double, so the scaling adds half an ulp per entry.
+//
+// This unit is compiled without contraction: the exact product splits would
+// otherwise be fused away.
+
+#include <cmath>
+
+#include "pqb_device.h"
+#include "pqb_kernels.h"
+
+namespace pqb {
+
+namespace {
+
+struct dd {
+    double h, l;
+};
+
+__device__ __forceinline__ dd dd_prod(double a, double b) {
+    const double p = a * b;
+    return {p, __builtin_fma(a, b, -p)};
+}
+
+__device__ __forceinline__ dd dd_sum(dd a, dd b) {
+    dd_add(a.h, a.l, b.h, b.l);
+    return a;
+}
+
+__device__ __forceinline__ dd dd_times(dd a, dd b) {
+    const dd p = dd_prod(a.h, b.h);
+    dd r;
+    fast_two_sum(p.h, p.l + (a.h * b.l + a.l * b.h), r.h, r.l);
+    return r;
+}
+
+__device__ __forceinline__ ddc ddc_times(const ddc& a, const ddc& b) {
+    const dd rr = dd_times({a.hr, a.lr}, {b.hr, b.lr}), ii = dd_times({a.hi, a.li}, {b.hi, b.li});
+    const dd ri = dd_times({a.hr, a.lr}, {b.hi, b.li}), ir = dd_times({a.hi, a.li}, {b.hr, b.lr});
+    const dd re = dd_sum(rr, {-ii.h, -ii.l}), im = dd_sum(ri, ir);
+    return {re.h, re.l, im.h, im.l};
+}
+
+// x / y rounded to double (x, y double-double, y.h != 0)
+__device__ __forceinline__ double dd_quot(dd x, dd y) {
+    const double q = x.h / y.h;
+    const dd qy = dd_prod(q, y.h);
+    // x - q y, leading parts cancel
+    const double r = ((x.h - qy.h) - qy.l) + x.l - q * y.l;
+    return q + r / y.h;
+}
+
+constexpr double kLargest = 0x1p20, kSmallest = 0x1p-20, kSpread = 0x1p-16;
+
+}  // namespace
+
+__global__ __launch_bounds__(256) void plain_expand_kernel(const double2* __restrict__ A, double2* __restrict__ M2,
+                                                           int n, int64_t m2_stride, unsigned* counters) {
+    __shared__ double row_min[kMaxCols];
+    __shared__ double row_max[kMaxCols];
+    __shared__ int row_flags[kMaxCols];  // bit 0: an entry not finite or too large; bit 1: one not an integer
+    __shared__ int pivot;
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    const int64_t task = blockIdx.x;
+    A += task * n * n;
+    M2 += task * m2_stride;
+
+    for (int i = wid; i < n; i += 4) {  // a wave per row (n <= 40 <= 64 lanes)
+        double lo = __builtin_inf(), hi = 0.0;
+        bool bad = false, frac = false;
+        if (lane < n) {
+            const double2 v = A[i * n + lane];
+            const double x = fabs(v.x), y = fabs(v.y);
+            bad = !(x <= kLargest && y <= kLargest);
+            frac = !(v.x == rint(v.x) && v.y == rint(v.y));
+            lo = hi = x > y ? x : y;
+        }
+        for (int m = kWave / 2; m >= 1; m >>= 1) {
+            lo = fmin(lo, __shfl_xor(lo, m, kWave));
+            hi = fmax(hi, __shfl_xor(hi, m, kWave));
+        }
+        const bool any_bad = __any(bad), any_frac = __any(frac);
+        if (lane == 0) {
+            row_min[i] = lo;
+            row_max[i] = hi;
+            row_flags[i] = (any_bad ? 1 : 0) | (any_frac ? 2 : 0);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int best = 0, flags = 0;
+        double hi = 0.0;
+        for (int i = 0; i < n; ++i) {
+            if (row_min[i] > row_min[best]) best = i;
+            hi = fmax(hi, row_max[i]);
+            flags |= row_flags[i];
+        }
+        const bool fits = flags == 2 && row_min[best] >= kSmallest && row_min[best] >= kSpread * hi;
+        pivot = fits ? best : -1;
+        counters[task] = fits ? kExpandedFlag : 0u;
+    }
+    __syncthreads();
+    const int r = pivot;
+    if (r < 0) {
+        for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
+            const double2 v = A[e];
+            M2[e] = make_double2(2.0 * v.x, 2.0 * v.y);
+            M2[n * n + e] = make_double2(-2.0 * v.x, -2.0 * v.y);
+        }
+        return;
+    }
+    const int m = (n - 1) * n;
+    for (int e = threadIdx.x; e < m; e += blockDim.x) {
+        const int k = e / n, j = e - k * n;
+        const double2 a = A[(k < r ? k : k + 1) * n + j];
+        const double2 b = A[r * n + j];
+        const dd den = dd_sum(dd_prod(b.x, b.x), dd_prod(b.y, b.y));
+        const double2 q = make_double2(2.0 * dd_quot(dd_sum(dd_prod(a.x, b.x), dd_prod(a.y, b.y)), den),
+                                       2.0 * dd_quot(dd_sum(dd_prod(a.y, b.x), dd_prod(-a.x, b.y)), den));
+        M2[e] = q;
+        M2[m + e] = make_double2(-q.x, -q.y);
+    }
+    if (wid == 0) {  // the product of the scales, after the table
+        ddc f = {1.0, 0.0, 0.0, 0.0};
+        if (lane < n) f = ddc_from(A[r * n + lane].x, A[r * n + lane].y);
+        for (int s = 1; s < kWave; s <<= 1) f = ddc_times(f, ddc_shfl_xor(f, s));
+        if (lane == 0) *reinterpret_cast<ddc*>(M2 + 2 * m) = f;
+    }
+}
+
+int plain_expand_row(const double* A, int n, int64_t ld) {
+    int best = -1;
+    double best_min = -1.0, hi = 0.0;
+    bool frac = false;
+    for (int i = 0; i < n; ++i) {
+        double lo = __builtin_inf();
+        for (int j = 0; j < n; ++j) {
+            const double re = A[2 * (i * ld + j)], im = A[2 * (i * ld + j) + 1];
+            const double x = std::fabs(re), y = std::fabs(im);
+            if (!(x <= kLargest && y <= kLargest)) return -1;
+            frac = frac || re != std::rint(re) || im != std::rint(im);
+            const double v = x > y ? x : y;
+            lo = v < lo ? v : lo;
+            hi = v > hi ? v : hi;
+        }
+        if (lo > best_min) {
+            best_min = lo;
+            best = i;
+        }
+    }
+    return frac && best_min >= kSmallest && best_min >= kSpread * hi ? best : -1;
+}
+
+hipError_t launch_plain_expand(const double2* A, double2* M2, int n, int64_t count, unsigned* counters,
+                               hipStream_t st) {
+    hipLaunchKernelGGL(plain_expand_kernel, dim3((unsigned)count), dim3(256), 0, st, A, M2, n, (int64_t)2 * n * n,
+                       counters);
+    return hipGetLastError();
+}
+
+}  // namespace pqb

@@ -30,6 +30,12 @@
 //   (wave, block, grid) is summed in double-double, and the last block to
 //   finish reduces the per-block partials and writes the result.
 //
+// The expanded form of a square matrix (perm_expand.hip; template argument EXPANDED) is
+// swept the same way over one row fewer, with the coefficient of x in prod_l (c_l + x) as
+// its term: 10*NC-12 FP64 instructions for what takes two Gray steps, 12*NC-8, of the
+// sweep over all rows.  n = 30, sustained: 2.93 ms all rows, 2.43 ms expanded (the FP64
+// issue rate and the clock the card's power allows bound both).
+//
 // A second kernel evaluates the same sum exactly for integer matrices, with
 // integer column sums and products/sums modulo 2^128 (two's complement
 // wrap-around); the true sum 2^(R-1) perm is recovered exactly whenever
@@ -99,6 +105,58 @@ __device__ __forceinline__ void add_row(double (&cr)[NC], double (&ci)[NC],
     }
 }
 
+// acc += sum_j prod_{l != j} c_l, the coefficient of x in prod_l (c_l + x).  Two
+// chains of linear polynomials p0 + p1 x over half of the columns each; a column
+// multiplies a chain by (c + x): p1 <- p1 c + p0 (4 FMAs, the addition is free),
+// p0 <- p0 c (4).  The chains' product is fused into the accumulation (8 FMAs).
+template <int NC>
+__device__ __forceinline__ void add_expanded_term(const double (&cr)[NC], const double (&ci)[NC], double& ar,
+                                                  double& ai) {
+    static_assert(NC >= 4, "two columns per chain");
+    constexpr int H = NC / 2;
+    double p0r[2], p0i[2], p1r[2], p1i[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int lo = q * H;
+        p0r[q] = cr[lo];
+        p0i[q] = ci[lo];
+        p1r[q] = cr[lo] + cr[lo + 1];
+        p1i[q] = ci[lo] + ci[lo + 1];
+        cmul(p0r[q], p0i[q], cr[lo + 1], ci[lo + 1]);
+    }
+#pragma unroll
+    for (int k = 2; k < NC - H; ++k) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            if (q == 0 && k >= H) continue;
+            const double xr = cr[q * H + k], xi = ci[q * H + k];
+            double tr = fma(p1r[q], xr, p0r[q]);
+            double ti = fma(p1r[q], xi, p0i[q]);
+            tr = fma(-p1i[q], xi, tr);
+            ti = fma(p1i[q], xr, ti);
+            cmul(p0r[q], p0i[q], xr, xi);
+            p1r[q] = tr;
+            p1i[q] = ti;
+        }
+    }
+    ar = fma(p0r[0], p1r[1], ar);
+    ai = fma(p0r[0], p1i[1], ai);
+    ar = fma(-p0i[0], p1i[1], ar);
+    ai = fma(p0i[0], p1r[1], ai);
+    ar = fma(p1r[0], p0r[1], ar);
+    ai = fma(p1r[0], p0i[1], ai);
+    ar = fma(-p1i[0], p0i[1], ar);
+    ai = fma(p1i[0], p0r[1], ai);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int NC, bool EXPANDED>
+__device__ __forceinline__ void add_sweep_term(const double (&cr)[NC], const double (&ci)[NC], double& ar,
+                                               double& ai) {
+    if constexpr (EXPANDED) add_expanded_term<NC>(cr, ci, ar, ai);
+    else add_term<NC>(cr, ci, ar, ai);
+}
+
 // LDS of a block's seeds.  Rows are an odd number of 16-byte elements apart, so that
 // lanes reading eight different rows of `lanes` at one column hit different banks.
 template <int NC>
@@ -111,7 +169,7 @@ struct SeedLds {
 
 // One wave's run of the sweep over the R rows of the +-2A table at Mb: the lane's
 // part of the sum, without the lane sign.  Every wave of the block calls it (barriers).
-template <int NC>
+template <int NC, bool EXPANDED>
 __device__ __forceinline__ void sweep_run(const char* __restrict__ Mb, const int R, const int K, const int B,
                                           const int H, const int64_t wave, const int64_t nwaves, const int lane,
                                           SeedLds<NC>& lds, double& tr, double& ti) {
@@ -204,11 +262,11 @@ __device__ __forceinline__ void sweep_run(const char* __restrict__ Mb, const int
                 (int)((tau1 - gbase >= (int64_t)W) ? W : (unsigned)(tau1 - gbase)));
             double pr = 0.0, pi = 0.0, mr = 0.0, mi = 0.0;
             // t = t0: even Gray index
-            add_term<NC>(cr, ci, pr, pi);
+            add_sweep_term<NC, EXPANDED>(cr, ci, pr, pi);
             if (K >= 1) {
                 // t = t0 + 1: walk bit 0 (row R-1) goes to delta = -1 iff bit 1 of t0 is 0
                 add_row<NC>(cr, ci, reinterpret_cast<const double2*>(Mb + (((t0 >> 1) & 1u) ? low_p : low_m)));
-                add_term<NC>(cr, ci, mr, mi);
+                add_sweep_term<NC, EXPANDED>(cr, ci, mr, mi);
                 // one (even, odd) step pair: the even step flips walk row ctz(t),
                 // the odd step row R-1
                 auto pair = [&](unsigned t) __attribute__((always_inline)) {
@@ -216,16 +274,17 @@ __device__ __forceinline__ void sweep_run(const char* __restrict__ Mb, const int
                     const unsigned nb = ((t >> b) ^ (t >> (b + 1))) & 1u;
                     const unsigned off = (nb ? neg : 0u) + (unsigned)(R - 1 - (int)b) * rowb;
                     add_row<NC>(cr, ci, reinterpret_cast<const double2*>(Mb + off));
-                    add_term<NC>(cr, ci, pr, pi);
+                    add_sweep_term<NC, EXPANDED>(cr, ci, pr, pi);
                     const unsigned off0 = ((t >> 1) & 1u) ? low_p : low_m;
                     add_row<NC>(cr, ci, reinterpret_cast<const double2*>(Mb + off0));
-                    add_term<NC>(cr, ci, mr, mi);
+                    add_sweep_term<NC, EXPANDED>(cr, ci, mr, mi);
                 };
                 // Two pairs per iteration: the second pair's even row is then issued
                 // during the first pair's odd product instead of after the loop's
                 // back-edge (n=30: 2.876 against 2.909 ms, same sums).  At 32 columns
-                // the two-pair body does not fit 168 VGPRs.
-                constexpr unsigned kPairs = NC == 32 ? 1u : 2u;
+                // the two-pair body does not fit 168 VGPRs; nor does the expanded sweep's
+                // (13 sizes spill), whose products are longer than the loads take anyway.
+                constexpr unsigned kPairs = NC == 32 || EXPANDED ? 1u : 2u;
                 unsigned t = t0 + 2;
                 if constexpr (kPairs == 2u) {
                     for (; t + 2 < t_stop; t += 4) {
@@ -258,7 +317,39 @@ __device__ __forceinline__ void sweep_run(const char* __restrict__ Mb, const int
     }
 }
 
-template <int NC>
+// (hr + lr) + i (hi + li) times the double-double complex f, for the scale of an
+// expanded sweep: products split exactly, the cross terms in FP64.  The empty asm
+// keeps each rounded product out of contraction, so that its FMA is its error.
+__device__ __forceinline__ void two_prod(double a, double b, double& p, double& e) {
+    p = a * b;
+    asm volatile("" : "+v"(p));
+    e = fma(a, b, -p);
+}
+
+__device__ __forceinline__ void dd_mul(double ah, double al, double bh, double bl, double& h, double& l) {
+    double p, e;
+    two_prod(ah, bh, p, e);
+    e = fma(ah, bl, fma(al, bh, e));
+    fast_two_sum(p, e, h, l);
+}
+
+__device__ __forceinline__ ddc ddc_mul(const ddc& a, const ddc& f) {
+    ddc r;
+    double h, l;
+    dd_mul(a.hr, a.lr, f.hr, f.lr, r.hr, r.lr);
+    dd_mul(a.hi, a.li, f.hi, f.li, h, l);
+    dd_add(r.hr, r.lr, -h, -l);
+    dd_mul(a.hr, a.lr, f.hi, f.li, r.hi, r.li);
+    dd_mul(a.hi, a.li, f.hr, f.lr, h, l);
+    dd_add(r.hi, r.li, h, l);
+    return r;
+}
+
+// EXPANDED: the sweep over the R-1 rows of a square matrix's expanded table, else over
+// all R rows.  Two kernels and not one with both sweeps: registers are allocated for
+// the whole kernel, and the pair did not fit (28 VGPRs spilled at 30 columns; 156 and
+// 162 VGPRs without a spill apart).
+template <int NC, bool EXPANDED>
 // Up to 32 columns the sweep fits in 168 VGPRs: ask for three waves per SIMD
 // so that scalar-load and FP64 latencies of one wave hide behind the others.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NC <= 32 ? 3 : 1)))
@@ -280,8 +371,16 @@ void plain_sweep_kernel(PlainParams p) {
     const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) / kWave;
     const char* __restrict__ Mb = reinterpret_cast<const char*>(p.M2 + (size_t)task * p.m2_stride);
 
+    // Where the tables were built on the GPU the launcher does not know their form and
+    // launches this kernel, then the expanded one; each leaves the other's matrices alone.
+    // (Blocks of this launch only change the counter's low bits until the last of them
+    // resets the word.)
+    if (p.by_flag) {
+        const unsigned c = (unsigned)__builtin_amdgcn_readfirstlane((int)*counter);
+        if (((c & kExpandedFlag) != 0) != EXPANDED) return;
+    }
     double tr, ti;
-    sweep_run<NC>(Mb, p.R, p.K, p.B, p.H, wave, nwaves, lane, seeds, tr, ti);
+    sweep_run<NC, EXPANDED>(Mb, EXPANDED ? p.R - 1 : p.R, p.K, p.B, p.H, wave, nwaves, lane, seeds, tr, ti);
     const bool lane_on = lane < (1 << p.B);
     const double ls = (__popc((unsigned)lane) & 1) ? -1.0 : 1.0;
     tr = lane_on ? ls * tr : 0.0;
@@ -294,7 +393,7 @@ void plain_sweep_kernel(PlainParams p) {
     if (threadIdx.x == 0) {
         ddc_store_through(&partials[blockIdx.x], v);
         wait_stores();
-        const unsigned done = atomicAdd(counter, 1u);
+        const unsigned done = atomicAdd(counter, 1u) & ~kExpandedFlag;
         is_last = (done == gridDim.x - 1);
     }
     __syncthreads();
@@ -307,7 +406,13 @@ void plain_sweep_kernel(PlainParams p) {
         }
         s = block_reduce(s, red);
         if (threadIdx.x == 0) {
-            s = ddc_scale(s, p.scale);
+            if constexpr (EXPANDED) {
+                // one row fewer was summed over (2^-(R-2)); the columns' scales follow the table
+                const ddc f = *reinterpret_cast<const ddc*>(Mb + (size_t)2 * (p.R - 1) * NC * sizeof(double2));
+                s = ddc_mul(ddc_scale(s, 2.0 * p.scale), f);
+            } else {
+                s = ddc_scale(s, p.scale);
+            }
             out[0] = s.hr + s.lr;
             out[1] = s.hi + s.li;
             out[2] = s.hr;
@@ -444,9 +549,9 @@ __global__ __launch_bounds__(256) void plain_exact_kernel(ExactParams p) {
 
 // ------------------------------------------------------------ dispatch --
 
-template <int NC>
+template <int NC, bool EXPANDED>
 static hipError_t launch_plain_nc(const PlainParams& p, int nblocks, int bdim, int ntasks, hipStream_t st) {
-    hipLaunchKernelGGL(plain_sweep_kernel<NC>, dim3(nblocks, ntasks), dim3(bdim), 0, st, p);
+    hipLaunchKernelGGL((plain_sweep_kernel<NC, EXPANDED>), dim3(nblocks, ntasks), dim3(bdim), 0, st, p);
     return hipGetLastError();
 }
 
@@ -461,30 +566,32 @@ static hipError_t launch_exact_nc(const ExactParams& p, int nblocks, int bdim, h
     return hipGetLastError();
 }
 
-template <int NC>
-static const void* plain_fn_nc() {
-    return reinterpret_cast<const void*>(&plain_sweep_kernel<NC>);
-}
-
 #define PQB_NC_CASES(X) \
     X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) \
     X(17) X(18) X(19) X(20) X(21) X(22) X(23) X(24) X(25) X(26) X(27) X(28) X(29) X(30)    \
     X(31) X(32) X(33) X(34) X(35) X(36) X(37) X(38) X(39) X(40)
 
-hipError_t launch_plain(int nc, const PlainParams& p, int nblocks, int bdim, int ntasks, hipStream_t st) {
+hipError_t launch_plain(int nc, bool expanded, const PlainParams& p, int nblocks, int bdim, int ntasks,
+                        hipStream_t st) {
     switch (nc) {
-#define PQB_CASE(N) \
-    case N: return launch_plain_nc<N>(p, nblocks, bdim, ntasks, st);
+#define PQB_CASE(N)                                                                                        \
+    case N:                                                                                                \
+        if constexpr (N >= kExpandedMinCols)                                                               \
+            if (expanded) return launch_plain_nc<N, true>(p, nblocks, bdim, ntasks, st);                   \
+        return expanded ? hipErrorInvalidValue : launch_plain_nc<N, false>(p, nblocks, bdim, ntasks, st);
         PQB_NC_CASES(PQB_CASE)
 #undef PQB_CASE
         default: return hipErrorInvalidValue;
     }
 }
 
-const void* plain_kernel_fn(int nc) {
+const void* plain_kernel_fn(int nc, bool expanded) {
     switch (nc) {
-#define PQB_CASE(N) \
-    case N: return plain_fn_nc<N>();
+#define PQB_CASE(N)                                                                                          \
+    case N:                                                                                                  \
+        if constexpr (N >= kExpandedMinCols)                                                                 \
+            if (expanded) return reinterpret_cast<const void*>(&plain_sweep_kernel<N, true>);                \
+        return expanded ? nullptr : reinterpret_cast<const void*>(&plain_sweep_kernel<N, false>);
         PQB_NC_CASES(PQB_CASE)
 #undef PQB_CASE
         default: return nullptr;

@@ -26,6 +26,18 @@ struct PlainPlan {
 
 PlainPlan make_plain_plan(int R, int NC, int64_t waves_resident);
 
+// Whether `count` R x C matrices are worth expanding (perm_expand.hip) where their
+// entries allow it.
+bool plain_expandable(int R, int C, int64_t count);
+
+struct ddc;
+struct PlainParams;
+PlainParams plain_params(const PlainPlan& pl, int R, const double2* m2, int64_t m2_stride, ddc* partials,
+                         unsigned* counter, double* out);
+// The launches of device matrices (engine.hip); xp: plan of the expanded sweep or NULL.
+int plain_device_launch(const double2* dA, int64_t count, int R, int C, const PlainPlan& pl, const PlainPlan* xp,
+                        double2* m2, ddc* partials, unsigned* counters, double* d_out, hipStream_t st);
+
 // One planned repeated-row permanent (see batch.hip).
 struct TaskPlan {
     bool trivial = false;      // decided without a sweep: value (tre, tim)
@@ -64,7 +76,7 @@ struct DeviceState {
     std::mutex mu;
     int device = -1;
     int cus = 0;
-    int blocks_per_cu[PQB_MAX_COLS + 1] = {0};
+    int blocks_per_cu[2][PQB_MAX_COLS + 1] = {};  // [expanded]
 };
 extern DeviceState g_dev;
 
@@ -72,7 +84,7 @@ extern DeviceState g_dev;
 // none) and reports it; a change of device releases every context's resources.
 int bind_device(int dev, int* device, int* cus);
 // Resident waves of the plain sweep for `nc` columns on the bound device.
-int64_t resident_waves(int nc);
+int64_t resident_waves(int nc, bool expanded);
 
 struct BatchBuffers;  // persistent-batch buffers and captured graphs (batch.hip)
 
@@ -95,7 +107,7 @@ struct Engine {
     // stream and device binding (first use, or after a device change); lock held
     int ensure_init_locked();
     int ensure_buffers_locked(size_t dneed, size_t hneed);
-    int64_t resident_waves_locked(int nc) { return resident_waves(nc); }
+    int64_t resident_waves_locked(int nc, bool expanded = false) { return resident_waves(nc, expanded); }
     void release_locked();  // stream, buffers and graphs (device change)
 };
 

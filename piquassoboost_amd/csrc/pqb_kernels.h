@@ -13,16 +13,26 @@ struct ddc;
 // (blockIdx.y = matrix index; a single matrix is a grid of height 1).
 struct PlainParams {
     const double2* M2;   // per matrix 2R x NC, packed: rows [0,R) = +2A, rows [R,2R) = -2A
+                         // expanded matrices: the 2(R-1) x NC table of the scaled rows,
+                         // then the product of the scales (ddc); see perm_expand.hip
     int64_t m2_stride;   // elements between consecutive matrices' M2 (2 R NC)
     int R;               // rows
     int K;               // Gray bits walked inside a chunk (rows R-K .. R-1)
     int B;               // lane bits (rows R-K-B .. R-K-1), B <= 6
     int H;               // group bits (rows 1 .. R-1-K-B), K + B + H = R - 1
+                         // (expanded: R - 1 rows, K + B + H = R - 2)
+    int by_flag;         // 1: only the matrices whose counter flag says this kernel
     ddc* partials;       // one dd complex per block, gridDim.x per matrix
-    unsigned* counter;   // one per matrix, zero on entry; the last block restores it to zero
+    unsigned* counter;   // one per matrix, zero on entry (or kExpandedFlag, from the prep kernel);
+                         // the last block restores it to zero
     double* out;         // 6 per matrix: [re, im, hi_re, lo_re, hi_im, lo_im]
     double scale;        // 2^-(R-1)
 };
+
+// Square matrices from this size on may be swept in expanded form (perm_expand.hip);
+// plain_expand_kernel decides per matrix and sets this bit of the matrix's counter.
+constexpr int kExpandedMinCols = 14;
+constexpr unsigned kExpandedFlag = 0x80000000u;
 
 // Exact integer sweep (sum kept modulo 2^128).
 struct ExactParams {
@@ -136,10 +146,18 @@ hipError_t launch_grad_reduce(const GradReduceParams& p, hipStream_t st);
 // perm = sum_j a_0j G_0j per matrix (A, G packed count x n x n)
 hipError_t launch_grad_perm(const double2* A, const double2* G, double2* perm, int n, int count, hipStream_t st);
 
-hipError_t launch_plain(int nc, const PlainParams& p, int nblocks, int bdim, int ntasks, hipStream_t st);
+// expanded: the sweep of expanded tables (square, nc >= kExpandedMinCols)
+hipError_t launch_plain(int nc, bool expanded, const PlainParams& p, int nblocks, int bdim, int ntasks,
+                        hipStream_t st);
+// Tables and counters of `count` packed n x n matrices, M2 stride 2 n n.
+hipError_t launch_plain_expand(const double2* A, double2* M2, int n, int64_t count, unsigned* counters,
+                               hipStream_t st);
 hipError_t launch_plain_prep(const double2* A, double2* M2, int n, int64_t count, hipStream_t st);
 hipError_t launch_plain_exact(int nc, const ExactParams& p, int nblocks, int bdim, hipStream_t st);
-const void* plain_kernel_fn(int nc);
+const void* plain_kernel_fn(int nc, bool expanded);
+// The row an n x n host matrix (row stride ld) is expanded along, -1 for none: the
+// choice plain_expand_kernel makes.
+int plain_expand_row(const double* A, int n, int64_t ld);
 
 constexpr int kMaxCols = 40;
 
