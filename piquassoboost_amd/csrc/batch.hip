@@ -52,15 +52,17 @@ static uint64_t binom_u64(int n, int k) {
     return c;
 }
 
-// Gray steps of the repeated sweep for multiplicities v (nonzero entries).
-static long double sweep_steps(const std::vector<int64_t>& v) {
-    if (v.empty()) return 0.0L;
+// Gray steps of the repeated sweep for multiplicities v (nonzero entries; at most 2^40,
+// exact in a double.  Not long double: an x87 operation takes ~70 ns on the GPU hosts, and
+// planning 4096 tasks in it cost milliseconds).
+static double sweep_steps(const std::vector<int64_t>& v) {
+    if (v.empty()) return 0.0;
     size_t mi = 0;
     for (size_t i = 1; i < v.size(); ++i)
         if (v[i] < v[mi]) mi = i;
-    long double s = (long double)v[mi];
+    double s = (double)v[mi];
     for (size_t i = 0; i < v.size(); ++i)
-        if (i != mi) s *= (long double)(v[i] + 1);
+        if (i != mi) s *= (double)(v[i] + 1);
     return s;
 }
 
@@ -79,31 +81,138 @@ struct PlanScratch {
 };
 }  // namespace
 
-int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int64_t* rmult,
-              const int64_t* cmult, uint64_t target_L, TaskPlan& P, bool plain) {
-    P = TaskPlan();
-    thread_local PlanScratch sc;
-    std::vector<int64_t>& ri = sc.ri;
-    std::vector<int64_t>& rm = sc.rm;
-    std::vector<int64_t>& ci = sc.ci;
-    std::vector<int64_t>& cm = sc.cm;
-    ri.clear();
-    rm.clear();
-    ci.clear();
-    cm.clear();
-    int64_t N = 0, Nc = 0;
+// Occupied rows and columns and their multiplicities into the thread's scratch.
+static void compact_occupations(int64_t rows, int64_t cols, const int64_t* rmult, const int64_t* cmult,
+                                PlanScratch& sc, int64_t* N, int64_t* Nc) {
+    sc.ri.clear();
+    sc.rm.clear();
+    sc.ci.clear();
+    sc.cm.clear();
+    *N = *Nc = 0;
     for (int64_t i = 0; i < rows; ++i)
         if (rmult[i] > 0) {
-            ri.push_back(i);
-            rm.push_back(rmult[i]);
-            N += rmult[i];
+            sc.ri.push_back(i);
+            sc.rm.push_back(rmult[i]);
+            *N += rmult[i];
         }
     for (int64_t j = 0; j < cols; ++j)
         if (cmult[j] > 0) {
-            ci.push_back(j);
-            cm.push_back(cmult[j]);
-            Nc += cmult[j];
+            sc.ci.push_back(j);
+            sc.cm.push_back(cmult[j]);
+            *Nc += cmult[j];
         }
+}
+
+static PlanScratch& plan_scratch() {
+    thread_local PlanScratch sc;
+    return sc;
+}
+
+// FP64 instructions of one Gray step (add_wterm, add_wcoeff in perm_repeated.hip).
+static double step_cost(int degree, int ns) {
+    if (degree == 0) return 6.0 * ns - 1.0;
+    // 2 per column sum and for the weight; 4 per coefficient and column, without the
+    // coefficients that are still zero or one, or can no longer reach x^D
+    const int d = degree;
+    return 2.0 * ns + 2.0 + 4.0 * (d + 1) * (ns - 1) - 2.0 * d * d - 2.0 * d * (d + 1);
+}
+
+// Sweeps below this many steps keep all rows: they take microseconds either way, and the
+// expanded ones need the launch that divides their columns.
+constexpr double kExpandMinSteps = 4096.0;
+
+// The sweep of a repeated-row task (A: the rows x cols matrix, its occupied rows and
+// columns in `sc`).  Without expansion: the orientation with fewer Gray steps.  A row of
+// multiplicity D can be expanded instead of walked: with every column divided by its entry
+// of that row, the row's D copies contribute the coefficient of x^D in the product of the
+// (column sums + x), so its radix D + 1 leaves the walk for a term of about 4 (D + 1) + 2
+// instead of 6 FP64 instructions per column -- of the D + 1 steps it replaces, 0.80, 0.72,
+// 0.67 of the instructions at D = 1, 2, 3 and 26 columns, 0.78, 0.68, 0.61 at 16.  The
+// cheapest orientation and multiplicity whose entries allow it is taken; the conditions
+// are those of the plain sweep (perm_expand.hip): a row without an entry below 2^-16 of
+// the matrix's largest, all of it inside [2^-20, 2^20], entries finite and not all whole
+// numbers.
+static SweepChoice choose_sweep(const double* A, int64_t ld, const PlanScratch& sc, bool expand) {
+    SweepChoice c;
+    const double sr = sweep_steps(sc.rm), st = sweep_steps(sc.cm);
+    c.transpose = st < sr;
+    c.steps = std::min(sr, st);
+    const int NS = (int)std::accumulate(sc.rm.begin(), sc.rm.end(), (int64_t)0);
+    if (!expand || c.steps < kExpandMinSteps || NS < kExpandedMinSlots) return c;
+
+    struct Candidate {
+        double cost, steps;
+        bool transpose;
+        int degree;
+    };
+    Candidate cand[2 * kMaxDegree];
+    int nc = 0;
+    const double kept = c.steps * step_cost(0, NS);
+    for (int t = 0; t < 2; ++t) {
+        const std::vector<int64_t>& m = t ? sc.cm : sc.rm;
+        if (m.size() < 2) continue;
+        for (int d = 1; d <= kMaxDegree; ++d) {
+            const auto at = std::find(m.begin(), m.end(), (int64_t)d);
+            if (at == m.end()) continue;
+            // steps of the other rows: their smallest is the anchor
+            int64_t lo = -1;
+            double s = 1.0;
+            for (auto k = m.begin(); k != m.end(); ++k)
+                if (k != at) {
+                    lo = lo < 0 ? *k : std::min(lo, *k);
+                    s *= (double)(*k + 1);
+                }
+            s = s / (double)(lo + 1) * (double)lo;
+            const double cost = s * step_cost(d, NS);
+            if (cost < kept) cand[nc++] = Candidate{cost, s, t != 0, d};
+        }
+    }
+    if (nc == 0) return c;
+    std::sort(cand, cand + nc, [](const Candidate& a, const Candidate& b) { return a.cost < b.cost; });
+
+    constexpr double kLargest = 0x1p20, kSmallest = 0x1p-20, kSpread = 0x1p-16;
+    const size_t R = sc.ri.size(), C = sc.ci.size();
+    double row_min[kMaxSlots], col_min[kMaxSlots], hi = 0.0;
+    std::fill(row_min, row_min + R, HUGE_VAL);
+    std::fill(col_min, col_min + C, HUGE_VAL);
+    bool frac = false;
+    for (size_t r = 0; r < R; ++r)
+        for (size_t k = 0; k < C; ++k) {
+            const double* a = A + 2 * (sc.ri[r] * ld + sc.ci[k]);
+            const double x = std::fabs(a[0]), y = std::fabs(a[1]);
+            if (!(x <= kLargest && y <= kLargest)) return c;
+            frac = frac || a[0] != std::rint(a[0]) || a[1] != std::rint(a[1]);
+            const double v = std::max(x, y);
+            row_min[r] = std::min(row_min[r], v);
+            col_min[k] = std::min(col_min[k], v);
+            hi = std::max(hi, v);
+        }
+    if (!frac) return c;
+    const double least = std::max(kSmallest, kSpread * hi);
+    for (int q = 0; q < nc; ++q) {
+        const std::vector<int64_t>& m = cand[q].transpose ? sc.cm : sc.rm;
+        const double* mins = cand[q].transpose ? col_min : row_min;
+        int best = -1;
+        for (size_t k = 0; k < m.size(); ++k)
+            if (m[k] == cand[q].degree && mins[k] >= least && (best < 0 || mins[k] > mins[best])) best = (int)k;
+        if (best < 0) continue;
+        c.transpose = cand[q].transpose;
+        c.degree = cand[q].degree;
+        c.row = (cand[q].transpose ? sc.ci : sc.ri)[(size_t)best];
+        c.steps = cand[q].steps;
+        return c;
+    }
+    return c;
+}
+
+// choice: the sweep (NULL: without expansion).
+int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int64_t* rmult,
+              const int64_t* cmult, uint64_t target_L, TaskPlan& P, const SweepChoice* choice, bool plain) {
+    P = TaskPlan();
+    PlanScratch& sc = plan_scratch();
+    const std::vector<int64_t>&ri = sc.ri, &rm = sc.rm, &ci = sc.ci, &cm = sc.cm;
+    int64_t N = 0, Nc = 0;
+    compact_occupations(rows, cols, rmult, cmult, sc, &N, &Nc);
     // plain: a rows x cols matrix with every multiplicity 1 and rows <= cols + 1
     // (the BBFG sum of BBFGPermanentCalculator.hpp:87-235, which is not
     // transpose invariant when rows != cols)
@@ -114,7 +223,12 @@ int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int
     }
     if (Nc > kMaxSlots || (!plain && N > kMaxSlots))
         return fail(PQB_ERR_SIZE, "more than " + std::to_string(kMaxSlots) + " photons");
-    const bool transpose = !plain && sweep_steps(cm) < sweep_steps(rm);
+    SweepChoice own;
+    if (!choice) {
+        if (!plain) own = choose_sweep(A, ld, sc, false);
+        choice = &own;
+    }
+    const bool transpose = choice->transpose;
     // element (r, c) of the oriented compact matrix
     auto elem = [&](int64_t r, int64_t c, double* re, double* im) {
         // oriented row r / column c -> original row i, column j
@@ -125,6 +239,7 @@ int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int
     };
     const std::vector<int64_t>& row_m = transpose ? cm : rm;
     const std::vector<int64_t>& col_m = transpose ? rm : cm;
+    const std::vector<int64_t>& row_i = transpose ? ci : ri;
 
     // column slots
     std::vector<int64_t>& slot_col = sc.slot_col;
@@ -133,15 +248,29 @@ int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int
         for (int64_t k = 0; k < col_m[c]; ++k) slot_col.push_back((int64_t)c);
     const int NS = (int)slot_col.size();
 
-    // anchor: smallest multiplicity, first occurrence
-    size_t anchor = 0;
-    for (size_t r = 1; r < row_m.size(); ++r)
-        if (row_m[r] < row_m[anchor]) anchor = r;
+    // the expanded row, and the anchor: of the others the smallest multiplicity, first occurrence
+    size_t expanded = row_m.size();
+    if (choice->degree > 0)
+        for (size_t r = 0; r < row_m.size(); ++r)
+            if (row_i[r] == choice->row) expanded = r;
+    size_t anchor = expanded == 0 ? 1 : 0;
+    for (size_t r = anchor + 1; r < row_m.size(); ++r)
+        if (r != expanded && row_m[r] < row_m[anchor]) anchor = r;
     std::vector<Digit>& digits = sc.digits;
     digits.clear();
     for (size_t r = 0; r < row_m.size(); ++r) {
+        if (r == expanded) continue;
         const int64_t m = (r == anchor) ? row_m[r] - 1 : row_m[r];
         if (m > 0) digits.push_back({(int64_t)r, (int)m});
+    }
+    P.degree = choice->degree;
+    P.scale = std::ldexp(1.0, -(int)(N - 1));
+    if (P.degree > 0) {  // the columns' scales follow on the GPU (rep_expand_kernel)
+        P.scale = std::ldexp(1.0, -(int)(N - P.degree - 1));
+        for (int d = 2; d <= P.degree; ++d) P.scale *= d;
+        P.xrow.assign((size_t)NS * 2, 0.0);
+        for (int s = 0; s < NS; ++s)
+            elem((int64_t)expanded, slot_col[(size_t)s], &P.xrow[2 * (size_t)s], &P.xrow[2 * (size_t)s + 1]);
     }
     // low / high split: largest radices first into the walk while it fits
     std::vector<size_t>& ord = sc.ord;
@@ -170,9 +299,9 @@ int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int
                 high.push_back(digits[k]);
             }
         }
-        long double nch = 1.0L;
-        for (const Digit& d : high) nch *= (long double)(d.m + 1);
-        if (nch < 4.0e9L) {
+        double nch = 1.0;
+        for (const Digit& d : high) nch *= (double)(d.m + 1);
+        if (nch < 4.0e9) {
             P.nchunks = (uint64_t)nch;
             // rows of A: anchor, low digits in walk order, high digits
             std::vector<Digit>& order_rows = sc.order_rows;
@@ -211,7 +340,6 @@ int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int
             for (const Digit& d : low) P.low_radix.push_back(d.m + 1);
             P.hrad.clear();
             for (const Digit& d : high) P.hrad.push_back((uint32_t)(d.m + 1));
-            P.scale = std::ldexp(1.0, -(int)(N - 1));
             return PQB_OK;
         }
         target_L *= 4;  // too many chunks for 32-bit chunk indices: walk more per chunk
@@ -507,7 +635,7 @@ static std::atomic<int64_t> g_walk[PQB_MAX_COLS + 1] = {};
 // Target walk length for a task of S steps when the batch holds `total`
 // steps: long walks amortise the per-chunk seed, but there must be enough
 // chunks to keep every resident lane busy.
-static uint64_t choose_L(long double S, long double total, int64_t lanes, bool fp64) {
+static uint64_t choose_L(double S, double total, int64_t lanes, bool fp64, double step = 1.0) {
     // A lane's time is (its chunks) x (walk + per-chunk cost: the item fetch, the
     // mixed-radix decomposition of the chunk index and the seed, tens of FP64 steps
     // with many chunk digits).  With little work per lane one chunk each; in the FP64
@@ -518,14 +646,18 @@ static uint64_t choose_L(long double S, long double total, int64_t lanes, bool f
     // FP64 step, so there the seed is cheap and short walks stay (n = 16: 0.046 ms
     // against 0.19 ms with the floor).  Larger batches take 4 chunks per lane so that
     // uneven items balance.
-    const long double per_lane = std::max(total, S) / (long double)std::max<int64_t>(lanes, 1);
-    const long double chunks_per_lane = per_lane < 1024.0L ? 1.0L : 4.0L;
-    long double want_chunks =
-        std::max<long double>(chunks_per_lane * (long double)lanes * S / std::max(total, S), 1.0L);
-    long double L = S / want_chunks;
-    L = std::min(L, S / 64.0L);  // at least one chunk per lane of a wave
-    if (fp64 && per_lane < 1024.0L) L = std::max(L, std::min(128.0L, 4.0L * S / (long double)std::max<int64_t>(lanes, 1)));
-    L = std::min<long double>(std::max<long double>(L, 16.0L), 2048.0L);
+    const double per_lane = std::max(total, S) / (double)std::max<int64_t>(lanes, 1);
+    const double chunks_per_lane = per_lane < 1024.0 ? 1.0 : 4.0;
+    double want_chunks =
+        std::max<double>(chunks_per_lane * (double)lanes * S / std::max(total, S), 1.0);
+    double L = S / want_chunks;
+    L = std::min(L, S / 64.0);  // at least one chunk per lane of a wave
+    // `step`: cost of a step in steps of the sweep over all rows; an expanded task's chunk
+    // is as long in time, not in steps (30 photons, degree 3: 24-step chunks 68.4 us,
+    // 36-step ones 72.3 us)
+    if (fp64 && per_lane < 1024.0)
+        L = std::max(L, std::min(128.0, 4.0 * S / (double)std::max<int64_t>(lanes, 1)) / step);
+    L = std::min<double>(std::max<double>(L, 16.0), 2048.0);
     return (uint64_t)L;
 }
 
@@ -537,6 +669,7 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     out6.assign(nt * 6, 0.0);
     // sweeps to run
     std::vector<size_t> live;
+    bool any_expanded = false;
     int min_ns = 1 << 30, max_ns = 0;
     for (size_t i = 0; i < nt; ++i) {
         if (plans[i].trivial) {
@@ -547,6 +680,7 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
             continue;
         }
         live.push_back(i);
+        any_expanded = any_expanded || plans[i].degree > 0;
         min_ns = std::min(min_ns, plans[i].NS);
         max_ns = std::max(max_ns, plans[i].NS);
     }
@@ -617,10 +751,11 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     for (size_t k = 0; k < live.size(); ++k) {
         const TaskPlan& P = plans[live[k]];
         const uint64_t per_item = std::min(per_item_of(P), cap);
+        const uint64_t chunk_cost = P.L * (uint64_t)step_cost(P.degree, P.NS);
         task_items[k].first = (uint32_t)items.size();
         for (uint64_t c0 = 0; c0 < P.nchunks; c0 += per_item) {
             const uint64_t cnt = std::min<uint64_t>(per_item, P.nchunks - c0);
-            const uint64_t cost = ((cnt + walkers - 1) / walkers) * P.L * (uint64_t)(P.NS + 4);
+            const uint64_t cost = ((cnt + walkers - 1) / walkers) * chunk_cost;
             if (cost != last_cost) {
                 const auto r = class_of.emplace(cost, (unsigned)class_cost.size());
                 if (r.second) class_cost.push_back(cost);
@@ -653,7 +788,7 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     table_off.reserve(64);
     std::string key;
     std::vector<std::pair<size_t, size_t>> tables;  // (offset, task whose radices it walks)
-    std::vector<size_t> a_off(live.size()), b_off(live.size()), t_off(live.size());
+    std::vector<size_t> a_off(live.size()), b_off(live.size()), x_off(live.size()), t_off(live.size());
     size_t nd = 0;
     for (size_t k = 0; k < live.size(); ++k) {
         const TaskPlan& P = plans[live[k]];
@@ -661,6 +796,8 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         nd = align256(nd + P.A.size() * sizeof(double));
         b_off[k] = nd;
         nd = align256(nd + P.base.size() * sizeof(double));
+        x_off[k] = nd;
+        nd = align256(nd + P.xrow.size() * sizeof(double));
         key.assign(P.low_radix.begin(), P.low_radix.end());
         auto it = table_off.find(key);
         if (it == table_off.end()) {
@@ -701,7 +838,10 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         t.nitems = task_items[k].second;
         t.out_index = (uint32_t)k;
         t.nchunks = (uint32_t)P.nchunks;
-        t.scale = P.scale;
+        t.degree = P.degree;
+        t.rows = P.R;
+        t.xrow = reinterpret_cast<const double2*>(d + B.off_data + x_off[k]);
+        t.scale[0] = P.scale;
         for (int hd = 0; hd < P.nhigh; ++hd) {
             t.hrow[hd] = (uint32_t)(1 + P.nlow + hd);
             t.hrad[hd] = P.hrad[(size_t)hd];
@@ -709,6 +849,8 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         T[k] = t;
         std::memcpy(h + B.off_data + a_off[(size_t)k], P.A.data(), P.A.size() * sizeof(double));
         std::memcpy(h + B.off_data + b_off[(size_t)k], P.base.data(), P.base.size() * sizeof(double));
+        if (P.degree > 0)
+            std::memcpy(h + B.off_data + x_off[(size_t)k], P.xrow.data(), P.xrow.size() * sizeof(double));
     }
     });
     host_parallel((int64_t)tables.size(), 4, [&](int64_t lo, int64_t hi) {
@@ -724,6 +866,10 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
 
     hipError_t e = hipMemcpyAsync(d, h, B.off_data + nd, hipMemcpyHostToDevice, E.stream);
     if (e != hipSuccess) return hip_fail(e, "batch upload");
+    if (any_expanded) {  // outside the graph: it divides the uploaded rows in place, once
+        e = launch_rep_expand(reinterpret_cast<RepTask*>(d + B.off_tasks), (int64_t)live.size(), E.stream);
+        if (e != hipSuccess) return drain_fail(E, e, "prep launch");
+    }
     hipGraphExec_t gx = nullptr;
     st = batch_graph_locked(E, range, &gx);
     if (st) {
@@ -792,7 +938,7 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
     if (precision == PQB_PREC_EXACT) return fail(PQB_ERR_ARG, "exact mode is available for the plain permanent only");
     const bool dd = precision == PQB_PREC_INF;
     std::vector<TaskPlan> plans((size_t)ntasks);
-    std::vector<long double> steps((size_t)ntasks, 0.0L);
+    std::vector<SweepChoice> choices((size_t)ntasks);
     std::vector<int> photons((size_t)ntasks, 0);
     // Validation and planning are per task and independent: large batches run
     // them on host threads (4096 tasks are milliseconds of host work either
@@ -816,12 +962,11 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
                     plans[(size_t)i].tre = v;
                     continue;
                 }
-                std::vector<int64_t> rm(tasks[i].row_mult, tasks[i].row_mult + tasks[i].rows);
-                std::vector<int64_t> cm(tasks[i].col_mult, tasks[i].col_mult + tasks[i].cols);
-                rm.erase(std::remove(rm.begin(), rm.end(), 0), rm.end());
-                cm.erase(std::remove(cm.begin(), cm.end(), 0), cm.end());
-                steps[(size_t)i] = std::min(sweep_steps(rm), sweep_steps(cm));
-                photons[(size_t)i] = (int)std::accumulate(rm.begin(), rm.end(), (int64_t)0);
+                PlanScratch& sc = plan_scratch();
+                int64_t n = 0, nc = 0;
+                compact_occupations(tasks[i].rows, tasks[i].cols, tasks[i].row_mult, tasks[i].col_mult, sc, &n, &nc);
+                choices[(size_t)i] = choose_sweep(tasks[i].A, tasks[i].ld, sc, !dd);
+                photons[(size_t)i] = (int)n;
             } catch (const std::exception& ex) {
                 pst[(size_t)i] = PQB_ERR_DEVICE;
                 perr[(size_t)i] = std::string("internal error: ") + ex.what();
@@ -833,10 +978,10 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
             t_err = (ntasks > 1 ? "task " + std::to_string(i) + ": " : std::string()) + perr[(size_t)i];
             return pst[(size_t)i];
         }
-    long double total = 0.0L;
+    double total = 0.0;
     int max_photons = 1;  // = the largest slot count of the batch
     for (int64_t i = 0; i < ntasks; ++i) {
-        total += steps[(size_t)i];
+        total += choices[(size_t)i].steps;
         max_photons = std::max(max_photons, photons[(size_t)i]);
     }
     bool any_sweep = false;
@@ -856,7 +1001,7 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
     const int dd_range = rep_dd_range_for(max_photons);
     const int64_t lanes = dd ? (int64_t)batch_grid_locked(E, dd_range) * (kBlock / kWave) * rep_dd_walkers(dd_range)
                              : (int64_t)batch_grid_locked(E, 2) * kBlock;
-    const bool large_batch = total >= 1024.0L * (long double)lanes;  // steps per lane
+    const bool large_batch = total >= 1024.0 * (double)lanes;  // steps per lane
     auto plan_range = [&](int64_t lo, int64_t hi) {
         for (int64_t i = lo; i < hi; ++i) {
             if (plans[(size_t)i].trivial) continue;
@@ -870,10 +1015,12 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
                 (!dd && large_batch && photons >= 0 && photons <= PQB_MAX_COLS) ? g_walk[photons].load() : 0;
             const uint64_t L = L_override > 0 ? (uint64_t)L_override
                                : tuned > 0    ? (uint64_t)tuned
-                                              : choose_L(steps[(size_t)i], total, lanes, !dd);
+                                              : choose_L(choices[(size_t)i].steps, total, lanes, !dd,
+                                                         step_cost(choices[(size_t)i].degree, (int)photons) /
+                                                             step_cost(0, (int)photons));
             try {  // nothing may escape a worker thread
                 pst[(size_t)i] = plan_task(tasks[i].A, tasks[i].rows, tasks[i].cols, tasks[i].ld,
-                                           tasks[i].row_mult, tasks[i].col_mult, L, plans[(size_t)i]);
+                                           tasks[i].row_mult, tasks[i].col_mult, L, plans[(size_t)i], &choices[(size_t)i]);
                 if (pst[(size_t)i]) perr[(size_t)i] = t_err;  // t_err is per thread
             } catch (const std::exception& ex) {
                 pst[(size_t)i] = PQB_ERR_DEVICE;
@@ -902,11 +1049,11 @@ int run_plain_dd_list_locked(Engine& E, const double* const* A, const int* R, co
     std::vector<TaskPlan> plans((size_t)n);
     for (int64_t k = 0; k < n; ++k) {
         const std::vector<int64_t> rm((size_t)R[k], 1), cm((size_t)C[k], 1);
-        const long double S = std::ldexp(1.0L, R[k] - 1);
+        const double S = std::ldexp(1.0, R[k] - 1);
         const int range = rep_dd_range_for(C[k]);  // the slots are the columns
         const int64_t walkers = (int64_t)batch_grid_locked(E, range) * (kBlock / kWave) * rep_dd_walkers(range);
         const int st = plan_task(A[k], R[k], C[k], ld[k], rm.data(), cm.data(), choose_L(S, S, walkers, false),
-                                 plans[(size_t)k], true);
+                                 plans[(size_t)k], nullptr, true);
         if (st) return n > 1 ? fail(st, "matrix " + std::to_string(k) + ": " + t_err) : st;
     }
     std::vector<double> out6;

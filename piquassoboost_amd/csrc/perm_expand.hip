@@ -1,4 +1,4 @@
-// Tables of the expanded plain sweep: perm(A) of a square matrix by expansion
+// Tables of the expanded sweeps: perm(A) of a square matrix by expansion
 // along one row r,
 //
 //     perm(A) = sum_j a_rj perm(A without row r and column j)
@@ -19,6 +19,9 @@
 //  * an entry is not finite or beyond 2^20;
 //  * every entry is a (Gaussian) integer: small integer matrices sum without
 //    rounding, which a division would lose.
+// Repeated-row tasks (batch.hip plans them) are divided here too: a row of multiplicity D
+// contributes the coefficient of x^D, times D!.
+//
 // Quotients are formed in double-double and rounded once, the product of the
 // scales is kept in double-double, so the scaling adds half an ulp per entry.
 //
@@ -69,6 +72,21 @@ __device__ __forceinline__ double dd_quot(dd x, dd y) {
     // x - q y, leading parts cancel
     const double r = ((x.h - qy.h) - qy.l) + x.l - q * y.l;
     return q + r / y.h;
+}
+
+// a / b
+__device__ __forceinline__ double2 cquot(double2 a, double2 b) {
+    const dd den = dd_sum(dd_prod(b.x, b.x), dd_prod(b.y, b.y));
+    return make_double2(dd_quot(dd_sum(dd_prod(a.x, b.x), dd_prod(a.y, b.y)), den),
+                        dd_quot(dd_sum(dd_prod(a.y, b.x), dd_prod(-a.x, b.y)), den));
+}
+
+// The product of n <= 64 complex numbers, on every lane of a wave.
+__device__ __forceinline__ ddc wave_product(const double2* v, int n, int lane) {
+    ddc f = {1.0, 0.0, 0.0, 0.0};
+    if (lane < n) f = ddc_from(v[lane].x, v[lane].y);
+    for (int s = 1; s < kWave; s <<= 1) f = ddc_times(f, ddc_shfl_xor(f, s));
+    return f;
 }
 
 constexpr double kLargest = 0x1p20, kSmallest = 0x1p-20, kSpread = 0x1p-16;
@@ -133,20 +151,52 @@ __global__ __launch_bounds__(256) void plain_expand_kernel(const double2* __rest
     const int m = (n - 1) * n;
     for (int e = threadIdx.x; e < m; e += blockDim.x) {
         const int k = e / n, j = e - k * n;
-        const double2 a = A[(k < r ? k : k + 1) * n + j];
-        const double2 b = A[r * n + j];
-        const dd den = dd_sum(dd_prod(b.x, b.x), dd_prod(b.y, b.y));
-        const double2 q = make_double2(2.0 * dd_quot(dd_sum(dd_prod(a.x, b.x), dd_prod(a.y, b.y)), den),
-                                       2.0 * dd_quot(dd_sum(dd_prod(a.y, b.x), dd_prod(-a.x, b.y)), den));
+        double2 q = cquot(A[(k < r ? k : k + 1) * n + j], A[r * n + j]);
+        q = make_double2(2.0 * q.x, 2.0 * q.y);
         M2[e] = q;
         M2[m + e] = make_double2(-q.x, -q.y);
     }
     if (wid == 0) {  // the product of the scales, after the table
-        ddc f = {1.0, 0.0, 0.0, 0.0};
-        if (lane < n) f = ddc_from(A[r * n + lane].x, A[r * n + lane].y);
-        for (int s = 1; s < kWave; s <<= 1) f = ddc_times(f, ddc_shfl_xor(f, s));
+        const ddc f = wave_product(A + r * n, n, lane);
         if (lane == 0) *reinterpret_cast<ddc*>(M2 + 2 * m) = f;
     }
+}
+
+// Repeated-row tasks: the rows are divided in place, the base (anchor + sum of the walked
+// rows' multiples, the seed of every chunk) formed from the quotients, and the product of
+// the scales, each slot's entry of the expanded row, taken into the task's scale.
+__global__ __launch_bounds__(256) void rep_expand_kernel(RepTask* tasks) {
+    RepTask& T = tasks[blockIdx.x];
+    if (T.degree == 0) return;
+    const int NS = T.NS, lane = threadIdx.x & (kWave - 1);
+    double2* const A = const_cast<double2*>(T.A);
+    if (threadIdx.x >= 3 * kWave) {  // one wave forms the scale beside the others' quotients
+        const ddc f = ddc_times(wave_product(T.xrow, NS, lane), ddc_from(T.scale[0], 0.0));
+        if (lane == 0) {
+            T.scale[0] = f.hr;
+            T.scale[1] = f.lr;
+            T.scale[2] = f.hi;
+            T.scale[3] = f.li;
+        }
+    } else {
+        for (int e = threadIdx.x; e < T.rows * NS; e += 3 * kWave) A[e] = cquot(A[e], T.xrow[e % NS]);
+    }
+    __syncthreads();
+    if (threadIdx.x < NS) {
+        double2 b = A[lane];
+        for (int d = 0; d < T.nlow; ++d) {
+            const double m = (double)(T.lrad[d] - 1);
+            const double2 a = A[(1 + d) * NS + lane];
+            b.x += m * a.x;
+            b.y += m * a.y;
+        }
+        const_cast<double2*>(T.base)[lane] = b;
+    }
+}
+
+hipError_t launch_rep_expand(RepTask* tasks, int64_t ntasks, hipStream_t st) {
+    hipLaunchKernelGGL(rep_expand_kernel, dim3((unsigned)ntasks), dim3(256), 0, st, tasks);
+    return hipGetLastError();
 }
 
 int plain_expand_row(const double* A, int n, int64_t ld) {

@@ -317,34 +317,6 @@ __device__ __forceinline__ void sweep_run(const char* __restrict__ Mb, const int
     }
 }
 
-// (hr + lr) + i (hi + li) times the double-double complex f, for the scale of an
-// expanded sweep: products split exactly, the cross terms in FP64.  The empty asm
-// keeps each rounded product out of contraction, so that its FMA is its error.
-__device__ __forceinline__ void two_prod(double a, double b, double& p, double& e) {
-    p = a * b;
-    asm volatile("" : "+v"(p));
-    e = fma(a, b, -p);
-}
-
-__device__ __forceinline__ void dd_mul(double ah, double al, double bh, double bl, double& h, double& l) {
-    double p, e;
-    two_prod(ah, bh, p, e);
-    e = fma(ah, bl, fma(al, bh, e));
-    fast_two_sum(p, e, h, l);
-}
-
-__device__ __forceinline__ ddc ddc_mul(const ddc& a, const ddc& f) {
-    ddc r;
-    double h, l;
-    dd_mul(a.hr, a.lr, f.hr, f.lr, r.hr, r.lr);
-    dd_mul(a.hi, a.li, f.hi, f.li, h, l);
-    dd_add(r.hr, r.lr, -h, -l);
-    dd_mul(a.hr, a.lr, f.hi, f.li, r.hi, r.li);
-    dd_mul(a.hi, a.li, f.hr, f.lr, h, l);
-    dd_add(r.hi, r.li, h, l);
-    return r;
-}
-
 // EXPANDED: the sweep over the R-1 rows of a square matrix's expanded table, else over
 // all R rows.  Two kernels and not one with both sweeps: registers are allocated for
 // the whole kernel, and the pair did not fit (28 VGPRs spilled at 30 columns; 156 and

@@ -92,6 +92,47 @@ __device__ __forceinline__ void add_wterm(const double (&cr)[NS], const double (
     }
 }
 
+// acc += w * [x^D] prod_s (c_s + x), D >= 1: the coefficients p_0 .. p_D of the running
+// product, one column after another, p_k <- p_k c + p_{k-1} (4 FMAs; p_0 <- p_0 c and the
+// leading ones less).  The coefficients of a column are independent of each other, so one
+// chain of columns keeps the FP64 pipe busy; only those that reach x^D are formed.
+template <int NS, int D>
+__device__ __forceinline__ void add_wcoeff(const double (&cr)[NS], const double (&ci)[NS], double w, double& ar,
+                                           double& ai) {
+    static_assert(NS > D && D >= 1, "a row besides the expanded one");
+    double pr[D + 1], pi[D + 1];
+    pr[0] = cr[0];
+    pi[0] = ci[0];
+#pragma unroll
+    for (int j = 2; j <= NS; ++j) {  // the j-th column: the product so far has degree j - 1, leading one
+        const double xr = cr[j - 1], xi = ci[j - 1];
+#pragma unroll
+        for (int k = D; k >= 0; --k) {
+            if (k >= j || k < D - (NS - j)) continue;
+            if (k == j - 1) {
+                pr[k] = xr + pr[k - 1];
+                pi[k] = xi + pi[k - 1];
+            } else if (k == 0) {
+                cmul(pr[0], pi[0], xr, xi);
+            } else {
+                double tr = fma(pr[k], xr, pr[k - 1]);
+                double ti = fma(pr[k], xi, pi[k - 1]);
+                pr[k] = fma(-pi[k], xi, tr);
+                pi[k] = fma(pi[k], xr, ti);
+            }
+        }
+    }
+    ar = fma(w, pr[D], ar);
+    ai = fma(w, pi[D], ai);
+}
+
+template <int NS, int D>
+__device__ __forceinline__ void add_wsweep_term(const double (&cr)[NS], const double (&ci)[NS], double w, double& ar,
+                                                double& ai) {
+    if constexpr (D == 0) add_wterm<NS>(cr, ci, w, ar, ai);
+    else add_wcoeff<NS, D>(cr, ci, w, ar, ai);
+}
+
 // colsum += f * row, f = +/-2.  The row is an SGPR operand (scalar loads); a
 // VALU instruction reads at most one SGPR here, so the wave-uniform factor is
 // kept in a VGPR (one move per step) rather than branching between two
@@ -110,7 +151,7 @@ __device__ __forceinline__ void rep_add_row(double (&cr)[NS], double (&ci)[NS], 
 }
 
 // Weighted sum over one chunk: sum_t w_t prod_s colsum_s(t), times the chunk weight.
-template <int NS>
+template <int NS, int D>
 __device__ __forceinline__ void rep_chunk(cptr<RepTask> T, const double* __restrict__ binom, uint32_t chunk,
                                           double& outr, double& outi) {
     double cr[NS], ci[NS];
@@ -149,7 +190,7 @@ __device__ __forceinline__ void rep_chunk(cptr<RepTask> T, const double* __restr
         wc *= (k & 1u) ? -b : b;
     }
     double ar = 0.0, ai = 0.0;
-    add_wterm<NS>(cr, ci, 1.0, ar, ai);
+    add_wsweep_term<NS, D>(cr, ci, 1.0, ar, ai);
     const cptr<RepStep> tab = to_const(T->table);
     const int L = T->L;
     if (L > 1) {
@@ -158,7 +199,7 @@ __device__ __forceinline__ void rep_chunk(cptr<RepTask> T, const double* __restr
             const RepStep en = tab[t + 1 < L ? t + 1 : t];  // next entry, loaded ahead
             const cptr<double2> row = A + (size_t)e.row * NS;
             rep_add_row<NS>(cr, ci, row, e.dir ? -2.0 : 2.0);
-            add_wterm<NS>(cr, ci, e.w, ar, ai);
+            add_wsweep_term<NS, D>(cr, ci, e.w, ar, ai);
             e = en;
         }
     }
@@ -166,10 +207,10 @@ __device__ __forceinline__ void rep_chunk(cptr<RepTask> T, const double* __restr
     outi = fma(wc, ai, outi);
 }
 
-template <int NS>
+template <int NS, int D>
 __device__ __forceinline__ void rep_item(cptr<RepTask> T, const double* __restrict__ binom, uint32_t chunk0,
                                          uint32_t count, int lane, double& sr, double& si) {
-    for (uint32_t j = lane; j < count; j += kWave) rep_chunk<NS>(T, binom, chunk0 + j, sr, si);
+    for (uint32_t j = lane; j < count; j += kWave) rep_chunk<NS, D>(T, binom, chunk0 + j, sr, si);
 }
 
 // Dispatch on the slot count over the compile-time range [LO, HI].
@@ -178,7 +219,15 @@ __device__ __forceinline__ void rep_dispatch(int ns, cptr<RepTask> T, const doub
                                              uint32_t chunk0, uint32_t count, int lane, double& sr, double& si) {
     if constexpr (LO <= HI) {
         if (ns == LO) {
-            rep_item<LO>(T, binom, chunk0, count, lane, sr, si);
+            if constexpr (LO >= kExpandedMinSlots) {
+                switch (T->degree) {
+                    case 1: rep_item<LO, 1>(T, binom, chunk0, count, lane, sr, si); return;
+                    case 2: rep_item<LO, 2>(T, binom, chunk0, count, lane, sr, si); return;
+                    case 3: rep_item<LO, 3>(T, binom, chunk0, count, lane, sr, si); return;
+                    default: break;
+                }
+            }
+            rep_item<LO, 0>(T, binom, chunk0, count, lane, sr, si);
         } else {
             rep_dispatch<LO + 1, HI>(ns, T, binom, chunk0, count, lane, sr, si);
         }
@@ -242,7 +291,8 @@ __global__ __launch_bounds__(kReduceThreads) void rep_reduce_kernel(RepBatchPara
         }
         s = block_reduce(s, red);
         if (threadIdx.x == 0) {
-            s = ddc_scale(s, T.scale);
+            if (T.degree == 0) s = ddc_scale(s, T.scale[0]);
+            else s = ddc_mul(s, {T.scale[0], T.scale[1], T.scale[2], T.scale[3]});
             double* o = p.out + 6 * (size_t)T.out_index;
             o[0] = s.hr + s.lr;
             o[1] = s.hi + s.li;

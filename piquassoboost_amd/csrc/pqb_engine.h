@@ -38,6 +38,14 @@ PlainParams plain_params(const PlainPlan& pl, int R, const double2* m2, int64_t 
 int plain_device_launch(const double2* dA, int64_t count, int R, int C, const PlainPlan& pl, const PlainPlan* xp,
                         double2* m2, ddc* partials, unsigned* counters, double* d_out, hipStream_t st);
 
+// Which sweep a repeated-row task takes (batch.hip): orientation and expanded row.
+struct SweepChoice {
+    bool transpose = false;
+    int degree = 0;          // multiplicity of the expanded row, 0: none
+    int64_t row = -1;        // the expanded row: original row (column when transposed)
+    double steps = 0;        // Gray steps
+};
+
 // One planned repeated-row permanent (see batch.hip).
 struct TaskPlan {
     bool trivial = false;      // decided without a sweep: value (tre, tim)
@@ -48,7 +56,9 @@ struct TaskPlan {
     int nlow = 0, nhigh = 0;
     uint64_t L = 1;            // walk length
     uint64_t nchunks = 1;
-    double scale = 1.0;        // 2^-(N-1)
+    int degree = 0;            // RepTask::degree
+    double scale = 1.0;        // 2^-(N-1); expanded: D! 2^-(N-D-1)
+    std::vector<double> xrow;  // expanded: NS complex, the expanded row
     std::vector<double> A;     // R x NS complex (interleaved)
     std::vector<double> base;  // NS complex
     std::vector<int> low_radix;
@@ -56,7 +66,8 @@ struct TaskPlan {
 };
 
 int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int64_t* rmult,
-              const int64_t* cmult, uint64_t target_L, TaskPlan& P, bool plain = false);
+              const int64_t* cmult, uint64_t target_L, TaskPlan& P, const SweepChoice* choice = nullptr,
+              bool plain = false);
 int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, double* out,
                 int64_t L_override);
 struct Engine;

@@ -47,6 +47,11 @@ struct ExactParams {
 };
 
 // ---- repeated-row / batched sweep ----
+// A row of multiplicity D <= kMaxDegree may be expanded (plan_task): the columns are
+// divided by its entries and its digit is replaced by a term of degree D.  Tasks that are
+// expanded have at least kExpandedMinSlots slots.
+constexpr int kMaxDegree = 3;
+constexpr int kExpandedMinSlots = 13;
 constexpr int kMaxDigits = 40;
 constexpr int kMaxSlots = 40;
 constexpr int kBinomStride = 41;  // binomial table: binom[m * 41 + k], 0 <= k <= m <= 40
@@ -70,7 +75,11 @@ struct RepTask {
     uint32_t nitems;
     uint32_t out_index;    // result slot
     uint32_t nchunks;      // prod_high (m_i + 1)
-    double scale;          // 2^-(N-1)
+    int degree;            // 0: term prod_s c_s; D > 0: the coefficient of x^D in prod_s (c_s + x)
+    int rows;              // rows of A
+    const double2* xrow;   // expanded: NS, the expanded row r
+    double scale[4];       // double-double complex: 2^-(N-1); expanded: D! 2^-(N-D-1), times
+                           // prod_s a_rs once rep_expand_kernel has run
     uint32_t hrow[kMaxDigits];  // row (in A) of high digit h
     uint32_t hrad[kMaxDigits];  // radix m_h + 1 of high digit h (digit 0 varies fastest)
     uint32_t lrad[kMaxDigits];  // radix m_d + 1 of low digit d (row 1 + d); read by the
@@ -101,6 +110,8 @@ constexpr int kReduceThreads = 256;  // one block of four waves per task
 
 // Kernel instantiations cover slot ranges; rep_range_for() picks the narrowest
 // one for a batch (-1: the batch needs splitting at 32 slots).
+// Divides the rows and bases of the expanded tasks by their expanded rows, in place.
+hipError_t launch_rep_expand(RepTask* tasks, int64_t ntasks, hipStream_t st);
 int rep_range_for(int min_ns, int max_ns);
 const void* rep_batch_kernel_fn(int range);
 hipError_t launch_rep_batch(int range, const RepBatchParams& p, int grid_blocks, hipStream_t st);

@@ -105,3 +105,55 @@ def test_non_finite_entries_stay_non_finite():
         A[3, 7] = bad
         v = C.permanent(A, C.ALGO_BBFG, C.PREC_FP64)
         assert not (np.isfinite(v.real) and np.isfinite(v.imag))
+
+
+def _spread_over_rows(rng, photons, rows, only=None):
+    """Multiplicities of `rows` rows with `photons` photons; only: every one that value."""
+    if only:
+        return np.full(photons // only, only, dtype=np.int64)
+    return (1 + rng.multinomial(photons - rows, np.full(rows, 1.0 / rows))).astype(np.int64)
+
+
+@pytest.mark.parametrize("photons,rows,only", [(13, 13, 0), (14, 13, 0), (16, 0, 2), (18, 0, 3), (21, 12, 0),
+                                               (26, 16, 0), (20, 0, 4)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_repeated_rows(photons, rows, only, transposed):
+    """Degrees 1, 2, 3 and none (every multiplicity 4), from the smallest expanded slot
+    count on, both orientations, over the forms the rows can have; alone, in a batch with
+    the others, and with no digit walked."""
+    rng = np.random.default_rng(9500 + photons * 2 + transposed)
+    mult = _spread_over_rows(rng, photons, rows, only)
+    R = len(mult)
+    one = np.ones(photons, np.int64)
+    base = random_complex(rng, R, photons)
+    mats = {"dense": base, "zeros in the single rows": np.where((mult == 1)[:, None] & (rng.random(base.shape) < 0.2),
+                                                                0, base),
+            "zeros in all rows": np.where(rng.random(base.shape) < 0.15, 0, base),
+            "small": base * 1e-5, "integers": rng.integers(1, 4, base.shape) + 1j}
+    tasks, want = [], []
+    for name, m in mats.items():
+        A, r, c = (np.ascontiguousarray(m.T), one, mult) if transposed else (m, mult, one)
+        tasks.append((A, r, c))
+        want.append(oracle.bbfg_repeated(np.ascontiguousarray(A, dtype=np.complex128), c, r, "dd"))
+        print(f"expand: repeated {photons}/{R} {name} transposed={transposed}", flush=True)
+        assert rel_err(C.permanent_repeated(A, r, c), want[-1]) < TOL, name
+    for walk in (0, 1, 16):
+        got = C.permanent_batch(tasks, walk_length=walk)
+        for v, w in zip(got, want):
+            assert rel_err(v, w) < TOL, walk
+
+
+def test_repeated_rows_and_columns():
+    """Multiplicities on both sides, up to the largest slot count (past 32 slots the batch
+    is split), against the double-double sweep."""
+    rng = np.random.default_rng(9600)
+    tasks = []
+    for photons, rows, cols in ((24, 14, 20), (31, 12, 26), (33, 13, 13), (36, 14, 12), (40, 14, 11)):
+        tasks.append((random_complex(rng, rows, cols), _spread_over_rows(rng, photons, rows),
+                      _spread_over_rows(rng, photons, cols)))
+    print("expand: repeated rows and columns", flush=True)
+    got = C.permanent_batch(tasks)
+    want = C.permanent_batch(tasks, precision=C.PREC_INF)
+    for v, w, (A, r, c) in zip(got, want, tasks):
+        assert rel_err(v, w) < 1e-10, int(r.sum())
+        assert rel_err(C.permanent_repeated(A, r, c), w) < 1e-10
