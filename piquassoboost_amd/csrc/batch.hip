@@ -53,8 +53,7 @@ static uint64_t binom_u64(int n, int k) {
 }
 
 // Gray steps of the repeated sweep for multiplicities v (nonzero entries; at most 2^40,
-// exact in a double.  Not long double: an x87 operation takes ~70 ns on the GPU hosts, and
-// planning 4096 tasks in it cost milliseconds).
+// exact in a double).
 static double sweep_steps(const std::vector<int64_t>& v) {
     if (v.empty()) return 0.0;
     size_t mi = 0;
