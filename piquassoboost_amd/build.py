@@ -44,7 +44,7 @@ CFLAGS = [
 # transformations, which stay error-free only if no product is fused into a
 # later sum: no contraction anywhere in that translation unit (a pragma does
 # not cover the negations and the math-header wrappers that get inlined).
-EXTRA_FLAGS = {"perm_dd.hip": ["-ffp-contract=off"], "perm_expand.hip": ["-ffp-contract=off"]}
+EXTRA_FLAGS = {name: ["-ffp-contract=off"] for name in ("perm_dd.hip", "perm_exact.hip", "perm_expand.hip")}
 
 
 def _compile(src: Path, verbose: bool) -> Path:

@@ -384,52 +384,90 @@ typedef __int128 i128;
 
 static double i128_to_double(i128 v) { return (double)v; }
 
+// Steps between flushes of the exact sweep on the FP64 pipe, 0: its group products may
+// exceed 46 bits (perm_exact.hip).
+static int exact_fp64_flush(int64_t cmax, int C) {
+    const int g = (C + 2) / 3;
+    int64_t q = 1;
+    for (int k = 0; k < g; ++k) {
+        q *= std::max<int64_t>(cmax, 1);
+        if (q > ((int64_t)1 << 46)) return 0;
+    }
+    return 1 << std::min(8, 140 - 3 * ceil_log2(q));
+}
+
 // Exact route: sum_delta (prod delta) prod_j c_j  (mod 2^128) on the GPU,
 // then divide by 2^(R-1).  The caller holds the lease of E.
 static int run_exact_locked(Engine& E, const std::vector<int>& ai, int R, int C, i128* result) {
     const int T = R - 1;
-    int64_t lr = E.resident_waves_locked(C) * kWave;
-    const int lg = floor_log2(std::max<int64_t>(lr, kWave));
-    const int H = std::min(T, std::max(0, lg));
-    const int K = T - H;
-    if (K > 30) return fail(PQB_ERR_SIZE, "exact sweep too large");
-    const int64_t nlanes = (int64_t)1 << H;
-    const int block = (int)std::min<int64_t>(kBlock, ((nlanes + kWave - 1) / kWave) * kWave);
-    const int64_t blocks = (nlanes + block - 1) / block;
-
-    const size_t a_bytes = ai.size() * sizeof(int);
-    const size_t part_off = kCounterBytes;
-    const size_t part_bytes = (size_t)blocks * 2 * sizeof(unsigned long long);
-    const size_t out_off = part_off + ((part_bytes + 255) / 256) * 256;
-    const size_t a_off = out_off + 256;
-    int st = E.ensure_buffers_locked(a_off + a_bytes, a_bytes + 256);
-    if (st) return st;
-    char* d = static_cast<char*>(E.dbuf);
-    std::memcpy(E.hbuf, ai.data(), a_bytes);
-    hipError_t e = hipMemcpyAsync(d + a_off, E.hbuf, a_bytes, hipMemcpyHostToDevice, E.stream);
-    if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync");
-    // every running column sum is bounded by its column's abs sum: 28^13, 1400^6 and
-    // (2^30)^2 are below 2^63 (integer_matrix admits column abs sums below 2^30)
+    // every running column sum is bounded by its column's abs sum
     int64_t cmax = 0;
     for (int j = 0; j < C; ++j) {
         int64_t s = 0;
         for (int i = 0; i < R; ++i) s += std::llabs((long long)ai[(size_t)i * C + j]);
         cmax = std::max(cmax, s);
     }
-    ExactParams p;
-    p.A = reinterpret_cast<const int*>(d + a_off);
-    p.R = R;
-    p.K = K;
-    p.H = H;
-    p.group = cmax <= 28 ? 13 : (cmax <= 1400 ? 6 : 2);
-    p.nlanes = nlanes;
-    p.partials = reinterpret_cast<unsigned long long*>(d + part_off);
-    p.counter = reinterpret_cast<unsigned*>(d);
-    p.out = reinterpret_cast<unsigned long long*>(d + out_off);
-    e = launch_plain_exact(C, p, (int)blocks, block, E.stream);
+    const int flush = exact_fp64_flush(cmax, C);
+    int K, B = 0, H, block;
+    int64_t blocks;
+    if (flush) {
+        // four waves per SIMD, walks of at least 8 steps
+        K = std::max(T - (floor_log2((int64_t)16 * E.cus) + 6), std::min(T, 3));
+        B = std::min(6, T - K);
+        H = T - K - B;
+        const int64_t waves = (int64_t)1 << H;
+        block = (int)std::min<int64_t>(kExactBlock, waves * kWave);
+        blocks = waves * kWave / block;
+    } else {
+        const int64_t lr = E.resident_waves_locked(C) * kWave;
+        H = std::min(T, std::max(0, floor_log2(std::max<int64_t>(lr, kWave))));
+        K = T - H;
+        const int64_t nlanes = (int64_t)1 << H;
+        block = (int)std::min<int64_t>(kBlock, ((nlanes + kWave - 1) / kWave) * kWave);
+        blocks = (nlanes + block - 1) / block;
+    }
+    if (K > 30) return fail(PQB_ERR_SIZE, "exact sweep too large");
+
+    const size_t a_bytes = ai.size() * sizeof(double);  // doubles, or ints in half of it
+    const size_t part_off = kCounterBytes;
+    const size_t part_bytes = (size_t)blocks * 2 * sizeof(unsigned long long);
+    const size_t out_off = part_off + round256(part_bytes);
+    const size_t a_off = out_off + 256;
+    int st = E.ensure_buffers_locked(a_off + a_bytes, a_bytes + 256);
+    if (st) return st;
+    char* d = static_cast<char*>(E.dbuf);
+    if (flush) {
+        double* h = static_cast<double*>(E.hbuf);
+        for (size_t k = 0; k < ai.size(); ++k) h[k] = 2.0 * ai[k];
+    } else {
+        std::memcpy(E.hbuf, ai.data(), ai.size() * sizeof(int));
+    }
+    hipError_t e = hipMemcpyAsync(d + a_off, E.hbuf, ai.size() * (flush ? sizeof(double) : sizeof(int)),
+                                  hipMemcpyHostToDevice, E.stream);
+    if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync");
+    auto* partials = reinterpret_cast<unsigned long long*>(d + part_off);
+    auto* counter = reinterpret_cast<unsigned*>(d);
+    auto* dout = reinterpret_cast<unsigned long long*>(d + out_off);
+    if (flush) {
+        const ExactF64Params p{reinterpret_cast<const double*>(d + a_off), R, K, B, H, flush, partials, counter, dout};
+        e = launch_plain_exact_fp64(C, p, (int)blocks, block, E.stream);
+    } else {
+        // 28^13, 1400^6 and (2^30)^2 are below 2^63 (integer_matrix admits column abs sums below 2^30)
+        ExactParams p;
+        p.A = reinterpret_cast<const int*>(d + a_off);
+        p.R = R;
+        p.K = K;
+        p.H = H;
+        p.group = cmax <= 28 ? 13 : (cmax <= 1400 ? 6 : 2);
+        p.nlanes = (int64_t)1 << H;
+        p.partials = partials;
+        p.counter = counter;
+        p.out = dout;
+        e = launch_plain_exact(C, p, (int)blocks, block, E.stream);
+    }
     if (e != hipSuccess) return drain_fail(E, e, "exact sweep launch");
     unsigned long long* hout = reinterpret_cast<unsigned long long*>(static_cast<char*>(E.hbuf) + a_bytes);
-    e = hipMemcpyAsync(hout, d + out_off, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, E.stream);
+    e = hipMemcpyAsync(hout, dout, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, E.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(E.stream);
     if (e != hipSuccess) return hip_fail(e, "exact sweep");
     const unsigned __int128 u = ((unsigned __int128)hout[1] << 64) | hout[0];

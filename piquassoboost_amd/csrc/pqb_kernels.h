@@ -29,6 +29,17 @@ struct PlainParams {
     double scale;        // 2^-(R-1)
 };
 
+// The same sum with products in exact doubles (perm_exact.hip).
+constexpr int kExactBlock = 1024;  // threads per block at most
+struct ExactF64Params {
+    const double* A2;    // R x NC, packed: 2 a_ij
+    int R, K, B, H;      // walk, lane (<= 6) and group bits, K + B + H = R - 1; a wave per group
+    int flush;           // steps between flushes, even
+    unsigned long long* partials;  // two words per block
+    unsigned* counter;
+    unsigned long long* out;
+};
+
 // Square matrices from this size on may be swept in expanded form (perm_expand.hip);
 // plain_expand_kernel decides per matrix and sets this bit of the matrix's counter.
 constexpr int kExpandedMinCols = 14;
@@ -164,6 +175,7 @@ hipError_t launch_plain(int nc, bool expanded, const PlainParams& p, int nblocks
 hipError_t launch_plain_expand(const double2* A, double2* M2, int n, int64_t count, unsigned* counters,
                                hipStream_t st);
 hipError_t launch_plain_prep(const double2* A, double2* M2, int n, int64_t count, hipStream_t st);
+hipError_t launch_plain_exact_fp64(int nc, const ExactF64Params& p, int nblocks, int bdim, hipStream_t st);
 hipError_t launch_plain_exact(int nc, const ExactParams& p, int nblocks, int bdim, hipStream_t st);
 const void* plain_kernel_fn(int nc, bool expanded);
 // The row an n x n host matrix (row stride ld) is expanded along, -1 for none: the
