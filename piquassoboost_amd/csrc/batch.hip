@@ -483,9 +483,11 @@ struct BatchBuffers {
            total = 0;
     hipGraphExec_t graph[kRanges] = {};  // FP64 slot ranges, then the double-double ones
     int grid[kRanges] = {};
-    // last prepared batch (for replays)
+    // last prepared batch (for replays): its graph's range, or the one-block launch
     int last_range = -1;
     int last_ntasks = 0;
+    int last_tiny_ns = 0;  // > 0: last_tiny
+    TinyParams last_tiny = {};
 
     void layout(size_t nt, size_t ni, size_t nd) {
         cap_tasks = nt;
@@ -497,8 +499,8 @@ struct BatchBuffers {
         off_order = align256(off_items + ni * sizeof(RepItem));
         off_data = align256(off_order + ni * sizeof(unsigned));
         off_part = align256(off_data + nd);
-        off_out = align256(off_part + ni * sizeof(ddc));
-        total = align256(off_out + nt * 6 * sizeof(double));
+        total = align256(off_part + ni * sizeof(ddc));
+        off_out = align256(off_data + nd);  // in the staging buffer: the kernels write there
     }
     void drop_graphs() {
         for (auto& g : graph)
@@ -528,6 +530,7 @@ void release_batch_locked(Engine& E) {
     for (int& g : B.grid) g = 0;
     B.last_range = -1;
     B.last_ntasks = 0;
+    B.last_tiny_ns = 0;
 }
 
 // The context whose batch ran last: pqb_batch_replay replays it.
@@ -558,7 +561,7 @@ static int ensure_batch_buffers_locked(Engine& E, size_t nt, size_t ni, size_t n
         release();
         return hip_fail(e, "hipMalloc(batch)");
     }
-    e = hipHostMalloc(&B.hbuf, B.off_data + B.cap_data, hipHostMallocDefault);
+    e = hipHostMalloc(&B.hbuf, B.off_out + (B.cap_tasks * 6 + 1) * sizeof(double), hipHostMallocCoherent);
     if (e != hipSuccess) {
         B.hbuf = nullptr;
         release();
@@ -587,7 +590,7 @@ static RepBatchParams batch_params(Engine& E) {
     p.order = reinterpret_cast<const unsigned*>(d + B.off_order);
     p.binom = reinterpret_cast<const double*>(d + B.off_binom);
     p.partials = reinterpret_cast<ddc*>(d + B.off_part);
-    p.out = reinterpret_cast<double*>(d + B.off_out);
+    p.out = reinterpret_cast<double*>(static_cast<char*>(B.hbuf) + B.off_out);
     p.head = reinterpret_cast<unsigned*>(d);
     p.counts = reinterpret_cast<const unsigned*>(d + 64);
     return p;
@@ -877,15 +880,46 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     }
     e = hipGraphLaunch(gx, E.stream);
     if (e != hipSuccess) return drain_fail(E, e, "hipGraphLaunch");
-    std::vector<double> res(live.size() * 6);
-    e = hipMemcpyAsync(res.data(), d + B.off_out, res.size() * sizeof(double), hipMemcpyDeviceToHost,
-                       E.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(E.stream);
+    e = hipStreamSynchronize(E.stream);
     if (e != hipSuccess) return hip_fail(e, "batch sweep");
+    const double* res = reinterpret_cast<const double*>(h + B.off_out);
     for (size_t k = 0; k < live.size(); ++k) std::copy(&res[6 * k], &res[6 * k] + 6, &out6[6 * live[k]]);
     B.last_range = range;
+    B.last_tiny_ns = 0;
     B.last_ntasks = (int)live.size();
     g_last_batch.store(&E);
+    return PQB_OK;
+}
+
+// One task of few steps in one block (perm_tiny.hip); *done false when it does not fit.
+static int run_tiny_locked(Engine& E, const pqb_task& t, const SweepChoice& choice, double* out, bool* done) {
+    TaskPlan P;
+    int st = plan_task(t.A, t.rows, t.cols, t.ld, t.row_mult, t.col_mult, 1, P, &choice);
+    if (st || P.nhigh > kTinyDigits) return st;
+    TinyParams p = {};
+    for (int d = 0; d < P.nhigh; ++d) p.radix[d] = (unsigned char)P.hrad[(size_t)d];
+    if (P.nlow != 0 || P.degree != 0 || !tiny_split(p, P.NS, P.R)) return PQB_OK;
+    st = ensure_batch_buffers_locked(E, 1, 1, P.A.size() * sizeof(double));
+    if (st) return st;
+    BatchBuffers& B = batch_of(E);
+    char* h = static_cast<char*>(B.hbuf);
+    std::memcpy(h + B.off_data, P.A.data(), P.A.size() * sizeof(double));
+    p.A = reinterpret_cast<const double2*>(h + B.off_data);
+    p.out = reinterpret_cast<double*>(h + B.off_out);
+    p.scale = P.scale;
+    p.done = reinterpret_cast<unsigned*>(p.out + 6);
+    *p.done = 0u;
+    hipError_t e = launch_tiny(P.NS, p, 1, E.stream);
+    if (e == hipSuccess) e = wait_result(E, p.done);
+    if (e != hipSuccess) return drain_fail(E, e, "batch sweep");
+    out[0] = p.out[0];
+    out[1] = p.out[1];
+    B.last_range = -1;
+    B.last_ntasks = 1;
+    B.last_tiny_ns = P.NS;
+    B.last_tiny = p;
+    g_last_batch.store(&E);
+    *done = true;
     return PQB_OK;
 }
 
@@ -996,6 +1030,11 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
     int st = L.status();
     if (st) return st;
     Engine& E = *L;
+    if (ntasks == 1 && !dd && L_override <= 0 && choices[0].steps <= (double)kTinySteps && photons[0] <= kTinySlots) {
+        bool done = false;
+        st = run_tiny_locked(E, tasks[0], choices[0], out, &done);
+        if (st || done) return st;
+    }
     // chunks in flight: a lane each (FP64), a group of lanes each (double-double)
     const int dd_range = rep_dd_range_for(max_photons);
     const int64_t lanes = dd ? (int64_t)batch_grid_locked(E, dd_range) * (kBlock / kWave) * rep_dd_walkers(dd_range)
@@ -1076,12 +1115,16 @@ int batch_replay(int iters, double* ms) {
     if (L.status()) return L.status();
     Engine& E = *L;
     BatchBuffers& B = batch_of(E);
-    if (B.last_range < 0 || !B.graph[B.last_range]) return fail(PQB_ERR_ARG, "no batch has been run yet");
+    const bool tiny = B.last_tiny_ns > 0;
+    if (!tiny && (B.last_range < 0 || !B.graph[B.last_range]))
+        return fail(PQB_ERR_ARG, "no batch has been run yet");
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hipError_t e = hipEventCreate(&e0);
     if (e == hipSuccess) e = hipEventCreate(&e1);
     if (e == hipSuccess) e = hipEventRecord(e0, E.stream);
-    for (int i = 0; e == hipSuccess && i < iters; ++i) e = hipGraphLaunch(B.graph[B.last_range], E.stream);
+    for (int i = 0; e == hipSuccess && i < iters; ++i)
+        e = tiny ? launch_tiny(B.last_tiny_ns, B.last_tiny, 1, E.stream)
+                 : hipGraphLaunch(B.graph[B.last_range], E.stream);
     if (e == hipSuccess) e = hipEventRecord(e1, E.stream);
     if (e == hipSuccess) e = hipEventSynchronize(e1);
     float f = 0.f;

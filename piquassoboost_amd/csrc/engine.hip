@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdlib>
 #include <cmath>
 #include <cstdio>
@@ -43,6 +44,21 @@ int fail(int code, const std::string& msg) {
 
 int hip_fail(hipError_t e, const char* what) {
     return fail(PQB_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// A few microseconds of a small call are the runtime's: hipStreamSynchronize queues a
+// marker behind the kernel and waits for its signal.  The kernel's own word in host memory
+// is polled instead for about as long as a small call takes; a longer one, or one that
+// failed, is waited for as usual.  The stream stays in order, so the next call needs no more.
+hipError_t wait_result(Engine& E, const unsigned* done) {
+    const auto began = std::chrono::steady_clock::now();
+    do {
+        for (int k = 0; k < 64; ++k) {
+            if (__atomic_load_n(done, __ATOMIC_ACQUIRE)) return hipSuccess;
+            __builtin_ia32_pause();
+        }
+    } while (std::chrono::steady_clock::now() - began < std::chrono::microseconds(200));
+    return hipStreamSynchronize(E.stream);
 }
 
 int drain_fail(Engine& E, hipError_t e, const char* what) {
@@ -184,7 +200,7 @@ int Engine::ensure_buffers_locked(size_t dneed, size_t hneed) {
             hbytes = 0;
         }
         const size_t sz = std::max<size_t>(std::max<size_t>(hneed, 2 * old_h), (size_t)1 << 20);
-        hipError_t e = hipHostMalloc(&hbuf, sz, hipHostMallocDefault);
+        hipError_t e = hipHostMalloc(&hbuf, sz, hipHostMallocCoherent);
         if (e != hipSuccess) {
             hbuf = nullptr;
             return hip_fail(e, "hipHostMalloc(staging)");
@@ -278,6 +294,18 @@ PlainPlan make_plain_plan(int R, int NC, int64_t waves_resident) {
     return pl;
 }
 
+// From 12 rows on the block's LDS traffic costs more than the sweep's copy and second
+// launch (device entry, tiny / sweep: n = 11 8.0 / 9.1 us, n = 12 10.4 / 9.2), and so it
+// does for more matrices than CUs (8192 x 10: 69 / 31 us).
+bool plain_tiny(int R, int C, int64_t count, TinyParams& p) {
+    if (R > kTinyRows || count > 256) return false;
+    p = TinyParams{};
+    std::fill(p.radix, p.radix + (R - 1), (unsigned char)2);
+    p.stride = (int64_t)R * C;
+    p.scale = std::ldexp(1.0, -(R - 1));
+    return tiny_split(p, C, R);
+}
+
 // The expanded sweep does 10 n instead of 12 n FP64 instructions per pair of sign
 // vectors; its table costs a launch, and device matrices a second sweep launch for the
 // ones that keep all rows.  From 2^24 sign vectors on that pays (all rows / expanded,
@@ -318,6 +346,7 @@ PlainParams plain_params(const PlainPlan& pl, int R, const double2* m2, int64_t 
     p.counter = counter;
     p.out = out;
     p.scale = std::ldexp(1.0, -(R - 1));
+    p.done = nullptr;
     return p;
 }
 
@@ -431,8 +460,7 @@ static int run_exact_locked(Engine& E, const std::vector<int>& ai, int R, int C,
     const size_t a_bytes = ai.size() * sizeof(double);  // doubles, or ints in half of it
     const size_t part_off = kCounterBytes;
     const size_t part_bytes = (size_t)blocks * 2 * sizeof(unsigned long long);
-    const size_t out_off = part_off + round256(part_bytes);
-    const size_t a_off = out_off + 256;
+    const size_t a_off = part_off + round256(part_bytes);
     int st = E.ensure_buffers_locked(a_off + a_bytes, a_bytes + 256);
     if (st) return st;
     char* d = static_cast<char*>(E.dbuf);
@@ -447,9 +475,13 @@ static int run_exact_locked(Engine& E, const std::vector<int>& ai, int R, int C,
     if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync");
     auto* partials = reinterpret_cast<unsigned long long*>(d + part_off);
     auto* counter = reinterpret_cast<unsigned*>(d);
-    auto* dout = reinterpret_cast<unsigned long long*>(d + out_off);
+    // the kernel writes the result to the staging buffer itself
+    auto* hout = reinterpret_cast<unsigned long long*>(static_cast<char*>(E.hbuf) + a_bytes);
+    auto* done = reinterpret_cast<unsigned*>(hout + 2);
+    *done = 0u;
     if (flush) {
-        const ExactF64Params p{reinterpret_cast<const double*>(d + a_off), R, K, B, H, flush, partials, counter, dout};
+        const ExactF64Params p{reinterpret_cast<const double*>(d + a_off), R, K, B, H, flush, partials, counter, hout,
+                               done};
         e = launch_plain_exact_fp64(C, p, (int)blocks, block, E.stream);
     } else {
         // 28^13, 1400^6 and (2^30)^2 are below 2^63 (integer_matrix admits column abs sums below 2^30)
@@ -462,13 +494,11 @@ static int run_exact_locked(Engine& E, const std::vector<int>& ai, int R, int C,
         p.nlanes = (int64_t)1 << H;
         p.partials = partials;
         p.counter = counter;
-        p.out = dout;
+        p.out = hout;
         e = launch_plain_exact(C, p, (int)blocks, block, E.stream);
     }
     if (e != hipSuccess) return drain_fail(E, e, "exact sweep launch");
-    unsigned long long* hout = reinterpret_cast<unsigned long long*>(static_cast<char*>(E.hbuf) + a_bytes);
-    e = hipMemcpyAsync(hout, dout, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, E.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(E.stream);
+    e = flush ? wait_result(E, done) : hipStreamSynchronize(E.stream);
     if (e != hipSuccess) return hip_fail(e, "exact sweep");
     const unsigned __int128 u = ((unsigned __int128)hout[1] << 64) | hout[0];
     const i128 sum = (i128)u;
@@ -480,14 +510,31 @@ static int run_exact_locked(Engine& E, const std::vector<int>& ai, int R, int C,
 
 // FP64 route.  The caller holds the lease of E.
 static int run_plain_locked(Engine& E, const double* A, int R, int C, int64_t ld, double* out) {
+    TinyParams t;
+    if (plain_tiny(R, C, 1, t)) {
+        const size_t a_bytes = (size_t)R * C * sizeof(double2);
+        int st = E.ensure_buffers_locked(0, a_bytes + 7 * sizeof(double));
+        if (st) return st;
+        double* h = static_cast<double*>(E.hbuf);
+        pack_rows(A, R, C, ld, h);
+        t.A = reinterpret_cast<const double2*>(h);
+        t.out = h + a_bytes / sizeof(double);
+        t.done = reinterpret_cast<unsigned*>(t.out + 6);
+        *t.done = 0u;
+        hipError_t e = launch_tiny(C, t, 1, E.stream);
+        if (e == hipSuccess) e = wait_result(E, t.done);
+        if (e != hipSuccess) return drain_fail(E, e, "plain sweep");
+        out[0] = t.out[0];
+        out[1] = t.out[1];
+        return PQB_OK;
+    }
     const bool expanded = plain_expandable(R, C, 1) && plain_expand_row(A, C, ld) >= 0;
     const int rows = expanded ? R - 1 : R;
     const PlainPlan pl = make_plain_plan(rows, C, E.resident_waves_locked(C, expanded));
     const size_t a_bytes = (size_t)R * C * sizeof(double2), m2_bytes = 2 * a_bytes;
     const size_t part_off = kCounterBytes;
     const size_t part_bytes = (size_t)pl.blocks * sizeof(ddc);
-    const size_t out_off = part_off + round256(part_bytes);
-    const size_t m2_off = out_off + 256;
+    const size_t m2_off = part_off + round256(part_bytes);
     const size_t a_off = m2_off + round256(m2_bytes);
     // the upload: the +-2A table, or the matrix whose expanded table a kernel builds
     const size_t up_bytes = expanded ? a_bytes : m2_bytes;
@@ -496,22 +543,19 @@ static int run_plain_locked(Engine& E, const double* A, int R, int C, int64_t ld
     double* h = static_cast<double*>(E.hbuf);
     if (expanded) pack_rows(A, R, C, ld, h);
     else fill_m2(A, R, C, ld, h);
+    double* hout = h + up_bytes / sizeof(double);  // the kernel writes the result here itself
     char* d = static_cast<char*>(E.dbuf);
     unsigned* counter = reinterpret_cast<unsigned*>(d);
     double2* m2 = reinterpret_cast<double2*>(d + m2_off);
     hipError_t e = hipMemcpyAsync(d + (expanded ? a_off : m2_off), h, up_bytes, hipMemcpyHostToDevice, E.stream);
     if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync");
     if (expanded) e = launch_plain_expand(reinterpret_cast<const double2*>(d + a_off), m2, C, 1, counter, E.stream);
-    if (e == hipSuccess)
-        e = launch_plain(C, expanded,
-                         plain_params(pl, R, m2, 2 * R * C, reinterpret_cast<ddc*>(d + part_off), counter,
-                                      reinterpret_cast<double*>(d + out_off)),
-                         pl.blocks, pl.block, 1, E.stream);
-    if (e != hipSuccess) return drain_fail(E, e, "plain sweep launch");
-    double* hout = h + up_bytes / sizeof(double);
-    e = hipMemcpyAsync(hout, d + out_off, 6 * sizeof(double), hipMemcpyDeviceToHost, E.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(E.stream);
-    if (e != hipSuccess) return hip_fail(e, "plain sweep");
+    PlainParams p = plain_params(pl, R, m2, 2 * R * C, reinterpret_cast<ddc*>(d + part_off), counter, hout);
+    p.done = reinterpret_cast<unsigned*>(hout + 6);
+    *p.done = 0u;
+    if (e == hipSuccess) e = launch_plain(C, expanded, p, pl.blocks, pl.block, 1, E.stream);
+    if (e == hipSuccess) e = wait_result(E, p.done);
+    if (e != hipSuccess) return drain_fail(E, e, "plain sweep");
     out[0] = hout[0];
     out[1] = hout[1];
     return PQB_OK;
@@ -613,8 +657,9 @@ static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld
     struct Group {
         size_t first, count;
         int R, C;
-        bool expanded;
+        bool expanded, tiny;
         PlainPlan pl;
+        TinyParams t;
         size_t up_off;            // byte offset in the upload: +-2A tables, or (expanded) the matrices
         size_t part_off, m2_off;  // device byte offsets of the group's partials and tables
     };
@@ -629,27 +674,32 @@ static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld
         g.R = f.R;
         g.C = f.C;
         g.expanded = f.expanded;
-        g.pl = make_plain_plan(f.expanded ? f.R - 1 : f.R, f.C, E.resident_waves_locked(f.C, f.expanded));
+        g.tiny = plain_tiny(f.R, f.C, 1, g.t);
+        if (!g.tiny)
+            g.pl = make_plain_plan(f.expanded ? f.R - 1 : f.R, f.C, E.resident_waves_locked(f.C, f.expanded));
         groups.push_back(g);
         k = e;
     }
     const size_t n = items.size();
     const size_t cnt_off = kCounterBytes;  // offset 0 stays the single-call counter
     size_t off = cnt_off + round256(n * sizeof(unsigned));
-    const size_t out_off = off;
-    off += round256(n * 6 * sizeof(double));
     for (Group& g : groups) {
         g.part_off = off;
-        off += round256(g.count * (size_t)g.pl.blocks * sizeof(ddc));
+        if (!g.tiny) off += round256(g.count * (size_t)g.pl.blocks * sizeof(ddc));
     }
     // the upload holds the +-2A tables of the all-rows groups, used in place, and the
-    // matrices of the expanded ones, whose tables a kernel builds behind it
+    // matrices of the expanded ones, whose tables a kernel builds behind it; the matrices of
+    // the tiny groups stay in the staging buffer, past the upload
     const size_t up_base = off;
-    size_t up_total = 0;
-    for (Group& g : groups) {
-        g.up_off = up_total;
-        g.m2_off = up_base + up_total;
-        up_total += round256(g.count * (size_t)g.R * g.C * sizeof(double2) * (g.expanded ? 1 : 2));
+    size_t up_total = 0, staged = 0;
+    for (int tiny = 0; tiny < 2; ++tiny) {
+        for (Group& g : groups)
+            if (g.tiny == (tiny != 0)) {
+                g.up_off = staged;
+                g.m2_off = up_base + staged;
+                staged += round256(g.count * (size_t)g.R * g.C * sizeof(double2) * (g.expanded || g.tiny ? 1 : 2));
+            }
+        if (!tiny) up_total = staged;
     }
     off += up_total;
     for (Group& g : groups)
@@ -657,7 +707,7 @@ static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld
             g.m2_off = off;
             off += round256(g.count * (size_t)2 * g.R * g.C * sizeof(double2));
         }
-    int st = E.ensure_buffers_locked(off, up_total + n * 6 * sizeof(double));
+    int st = E.ensure_buffers_locked(off, staged + n * 6 * sizeof(double));
     if (st) return st;
     double* h = static_cast<double*>(E.hbuf);
     for (const Group& g : groups) {
@@ -665,17 +715,28 @@ static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld
         double* hg = h + g.up_off / sizeof(double);
         for (size_t k = 0; k < g.count; ++k) {
             const int64_t i = items[g.first + k].idx;
-            if (g.expanded) pack_rows(A[i], g.R, g.C, ld[i], hg + 2 * rc * k);
+            if (g.expanded || g.tiny) pack_rows(A[i], g.R, g.C, ld[i], hg + 2 * rc * k);
             else fill_m2(A[i], g.R, g.C, ld[i], hg + 4 * rc * k);
         }
     }
     char* d = static_cast<char*>(E.dbuf);
     unsigned* counters = reinterpret_cast<unsigned*>(d + cnt_off);
-    hipError_t e = hipMemsetAsync(counters, 0, n * sizeof(unsigned), E.stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(d + up_base, h, up_total, hipMemcpyHostToDevice, E.stream);
+    double* const hout = h + staged / sizeof(double);  // the kernels write the results here themselves
+    hipError_t e = hipSuccess;
+    if (up_total > 0) {
+        e = hipMemsetAsync(counters, 0, n * sizeof(unsigned), E.stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(d + up_base, h, up_total, hipMemcpyHostToDevice, E.stream);
+    }
     if (e != hipSuccess) return drain_fail(E, e, "list upload");
     constexpr size_t kMaxGridY = 65535;
-    for (const Group& g : groups) {
+    for (Group& g : groups) {
+        if (g.tiny) {
+            g.t.A = reinterpret_cast<const double2*>(h + g.up_off / sizeof(double));
+            g.t.out = hout + 6 * g.first;
+            e = launch_tiny(g.C, g.t, (int64_t)g.count, E.stream);
+            if (e != hipSuccess) return drain_fail(E, e, "list sweep launch");
+            continue;
+        }
         double2* const m2 = reinterpret_cast<double2*>(d + g.m2_off);
         const int64_t m2n = (int64_t)2 * g.R * g.C;
         if (g.expanded) {
@@ -688,14 +749,12 @@ static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld
             const PlainParams p = plain_params(
                 g.pl, g.R, m2 + o * (size_t)m2n, m2n,
                 reinterpret_cast<ddc*>(d + g.part_off) + o * (size_t)g.pl.blocks, counters + g.first + o,
-                reinterpret_cast<double*>(d + out_off) + 6 * (g.first + o));
+                hout + 6 * (g.first + o));
             e = launch_plain(g.C, g.expanded, p, g.pl.blocks, g.pl.block, (int)nt, E.stream);
             if (e != hipSuccess) return drain_fail(E, e, "list sweep launch");
         }
     }
-    double* hout = h + up_total / sizeof(double);
-    e = hipMemcpyAsync(hout, d + out_off, n * 6 * sizeof(double), hipMemcpyDeviceToHost, E.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(E.stream);
+    e = hipStreamSynchronize(E.stream);
     if (e != hipSuccess) return drain_fail(E, e, "list sweep");
     for (size_t k = 0; k < n; ++k) {
         out[2 * items[k].idx] = hout[6 * k];
@@ -816,6 +875,13 @@ static int plain_device_plan(int64_t count, int R, int C, PlainPlan* pl, PlainPl
 // rows, then (plan xp given) the expanded one; counters zero before, zero after.
 int plain_device_launch(const double2* dA, int64_t count, int R, int C, const PlainPlan& pl, const PlainPlan* xp,
                         double2* m2, ddc* partials, unsigned* counters, double* d_out, hipStream_t st) {
+    TinyParams t;
+    if (plain_tiny(R, C, count, t)) {
+        t.A = dA;
+        t.out = d_out;
+        const hipError_t e = launch_tiny(C, t, count, st);
+        return e == hipSuccess ? PQB_OK : hip_fail(e, "plain sweep launch");
+    }
     const int64_t m2n = (int64_t)2 * R * C;
     hipError_t e = xp ? launch_plain_expand(dA, m2, C, count, counters, st)
                       : launch_plain_prep(dA, m2, R * C, count, st);

@@ -115,6 +115,10 @@ static int noalloc_entry(const double* dA, int64_t rows, int64_t cols, double* d
                                       " columns: the static scratch buffer holds at most 41 x " +
                                       std::to_string(PQB_MAX_COLS));
     const int R = (int)rows, C = (int)cols;
+    TinyParams t;
+    if (plain_tiny(R, C, 1, t))  // one kernel without scratch
+        return plain_device_launch(reinterpret_cast<const double2*>(dA), 1, R, C, PlainPlan(), nullptr, nullptr,
+                                   nullptr, nullptr, d_out, st);
     ScratchDevice* s = nullptr;
     const bool expandable = plain_expandable(R, C, 1);
     int64_t wr[2] = {1, 1};

@@ -206,6 +206,7 @@ __global__ __launch_bounds__(kExactBlock) void plain_exact_fp64_kernel(ExactF64P
                 p.out[0] = lo;
                 p.out[1] = hi;
                 *p.counter = 0u;
+                announce(p.done);
             }
         }
     }

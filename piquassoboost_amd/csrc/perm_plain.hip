@@ -392,6 +392,7 @@ void plain_sweep_kernel(PlainParams p) {
             out[4] = s.hi;
             out[5] = s.li;
             *counter = 0u;  // leave the counter ready for the next launch
+            announce(p.done);
         }
     }
 }

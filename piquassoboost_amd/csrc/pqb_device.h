@@ -134,6 +134,12 @@ __device__ __forceinline__ T load_through(const T* p) {
 
 __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// A synchronous host call's result is in host memory: says so there, where the host polls
+// (wait_result in engine.hip), without waiting for the kernel's end to be noticed.
+__device__ __forceinline__ void announce(unsigned* done) {
+    if (done) __hip_atomic_store(done, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __device__ __forceinline__ void ddc_store_through(ddc* p, const ddc& v) {
     store_through(&p->hr, v.hr);
     store_through(&p->lr, v.lr);

@@ -26,6 +26,11 @@ struct PlainPlan {
 
 PlainPlan make_plain_plan(int R, int NC, int64_t waves_resident);
 
+struct TinyParams;
+// `count` R x C plain permanents that one block each evaluates (perm_tiny.hip): p set but
+// for A and out.
+bool plain_tiny(int R, int C, int64_t count, TinyParams& p);
+
 // Whether `count` R x C matrices are worth expanding (perm_expand.hip) where their
 // entries allow it.
 bool plain_expandable(int R, int C, int64_t count);
@@ -146,6 +151,9 @@ extern thread_local std::string t_err;
 
 int fail(int code, const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
+// Waits until the kernel queued on the context's stream last has set *done (host memory,
+// zeroed before its launch).
+hipError_t wait_result(Engine& E, const unsigned* done);
 // hip_fail after waiting for the context's stream: for failures after an upload
 // from the staging buffer was queued, so that no copy still reads it when the
 // context is released.

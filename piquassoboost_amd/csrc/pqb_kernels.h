@@ -27,6 +27,7 @@ struct PlainParams {
                          // the last block restores it to zero
     double* out;         // 6 per matrix: [re, im, hi_re, lo_re, hi_im, lo_im]
     double scale;        // 2^-(R-1)
+    unsigned* done;      // host memory, set to 1 after `out` (NULL: not wanted)
 };
 
 // The same sum with products in exact doubles (perm_exact.hip).
@@ -38,6 +39,7 @@ struct ExactF64Params {
     unsigned long long* partials;  // two words per block
     unsigned* counter;
     unsigned long long* out;
+    unsigned* done;      // as in PlainParams
 };
 
 // Square matrices from this size on may be swept in expanded form (perm_expand.hip);
@@ -56,6 +58,25 @@ struct ExactParams {
     unsigned* counter;
     unsigned long long* out;       // [lo, hi] of sum_delta (...) mod 2^128
 };
+
+// ---- one block per matrix (perm_tiny.hip) ----
+constexpr int kTinyDigits = 12;    // rows besides the anchor
+constexpr int kTinySteps = 2048;   // signed terms (repeated-row tasks)
+constexpr int kTinyRows = 11;      // rows of a plain permanent
+constexpr int kTinySlots = 24;     // columns (column slots)
+struct TinyParams {
+    const double2* A;      // per matrix R x NS, packed: row 0 the anchor, row 1 + d digit d's
+    int64_t stride;        // elements between consecutive matrices
+    double* out;           // 6 per matrix (RepBatchParams::out)
+    double scale;          // 2^-(N-1)
+    unsigned* done;        // as in PlainParams; one matrix only
+    int R, S, P, nlow;     // S = product of the radices, P = that of the first nlow
+    unsigned lds_bytes;
+    unsigned char radix[kTinyDigits];  // multiplicity + 1
+};
+// Fills the split of the digits whose radices are set; false: not for this kernel.
+bool tiny_split(TinyParams& p, int NS, int R);
+hipError_t launch_tiny(int ns, const TinyParams& p, int64_t count, hipStream_t st);
 
 // ---- repeated-row / batched sweep ----
 // A row of multiplicity D <= kMaxDegree may be expanded (plan_task): the columns are
