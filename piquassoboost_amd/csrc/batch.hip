@@ -475,12 +475,35 @@ static void host_parallel(int64_t n, int64_t grain, F&& fn) {
     for (std::thread& th : spawned) th.join();
 }
 
+// Byte offsets in a batch's device buffer; the staging buffer mirrors all but the partials.
+// The binomials stay, everything from the head on is uploaded for each batch.
+struct BatchLayout {
+    static constexpr size_t binom = 0, head = 13568;  // 41 x 41 doubles, then 256 bytes
+    size_t tasks = 0, items = 0, order = 0, data = 0, part = 0, end = 0;
+
+    void set(size_t nt, size_t ni, size_t nd) {
+        tasks = head + 256;
+        items = align256(tasks + nt * sizeof(RepTask));
+        order = align256(items + ni * sizeof(RepItem));
+        data = align256(order + ni * sizeof(unsigned));
+        part = align256(data + nd);
+        end = align256(part + ni * sizeof(ddc));
+    }
+};
+static_assert(BatchLayout::head % 256 == 0 && BatchLayout::head >= sizeof(double) * kBinomStride * kBinomStride, "");
+
+// Batches of up to this many tasks are laid out as tightly as they come and launched
+// directly: the layout for the capacities, which the captured graph needs, is 120 KB longer
+// to upload, and a graph's launch costs more than two kernels' (one task of
+// 14 photons and 2304 steps: 64.7 -> 33.5 us a call, of 30 photons 160 -> 144 us).
+constexpr size_t kDirectTasks = 64;
+
 struct BatchBuffers {
     void* dbuf = nullptr;
     void* hbuf = nullptr;
     size_t cap_tasks = 0, cap_items = 0, cap_data = 0;
-    size_t off_binom = 0, off_tasks = 0, off_items = 0, off_order = 0, off_data = 0, off_part = 0, off_out = 0,
-           total = 0;
+    BatchLayout at;  // for the capacities
+    size_t off_out = 0, total = 0;
     hipGraphExec_t graph[kRanges] = {};  // FP64 slot ranges, then the double-double ones
     int grid[kRanges] = {};
     // last prepared batch (for replays): its graph's range, or the one-block launch
@@ -488,19 +511,16 @@ struct BatchBuffers {
     int last_ntasks = 0;
     int last_tiny_ns = 0;  // > 0: last_tiny
     TinyParams last_tiny = {};
+    bool last_is_direct = false;      // last_direct, of last_ntasks tasks
+    RepBatchParams last_direct = {};
 
     void layout(size_t nt, size_t ni, size_t nd) {
         cap_tasks = nt;
         cap_items = ni;
         cap_data = nd;
-        off_binom = 256;
-        off_tasks = align256(off_binom + sizeof(double) * kBinomStride * kBinomStride);
-        off_items = align256(off_tasks + nt * sizeof(RepTask));
-        off_order = align256(off_items + ni * sizeof(RepItem));
-        off_data = align256(off_order + ni * sizeof(unsigned));
-        off_part = align256(off_data + nd);
-        total = align256(off_part + ni * sizeof(ddc));
-        off_out = align256(off_data + nd);  // in the staging buffer: the kernels write there
+        at.set(nt, ni, nd);
+        total = at.end;
+        off_out = at.part;  // in the staging buffer: the kernels write there
     }
     void drop_graphs() {
         for (auto& g : graph)
@@ -541,6 +561,8 @@ static int ensure_batch_buffers_locked(Engine& E, size_t nt, size_t ni, size_t n
     if (B.dbuf && nt <= B.cap_tasks && ni <= B.cap_items && nd <= B.cap_data) return PQB_OK;
     (void)hipStreamSynchronize(E.stream);
     B.drop_graphs();
+    B.last_range = -1;  // nothing to replay in the buffers that follow
+    B.last_tiny_ns = 0;
     if (B.dbuf) (void)hipFree(B.dbuf);
     if (B.hbuf) (void)hipHostFree(B.hbuf);
     B.dbuf = B.hbuf = nullptr;
@@ -567,12 +589,12 @@ static int ensure_batch_buffers_locked(Engine& E, size_t nt, size_t ni, size_t n
         release();
         return hip_fail(e, "hipHostMalloc(batch)");
     }
-    std::memset(B.hbuf, 0, B.off_data);
-    double* bt = reinterpret_cast<double*>(static_cast<char*>(B.hbuf) + B.off_binom);
+    std::memset(B.hbuf, 0, B.at.data);
+    double* bt = reinterpret_cast<double*>(static_cast<char*>(B.hbuf) + BatchLayout::binom);
     for (int m = 0; m < kBinomStride; ++m)
         for (int k = 0; k < kBinomStride; ++k) bt[m * kBinomStride + k] = (double)binom_u64(m, k);
     // counter + header start at zero on the device
-    e = hipMemcpyAsync(B.dbuf, B.hbuf, B.off_tasks, hipMemcpyHostToDevice, E.stream);
+    e = hipMemcpyAsync(B.dbuf, B.hbuf, B.at.tasks, hipMemcpyHostToDevice, E.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(E.stream);
     if (e != hipSuccess) {
         release();
@@ -581,19 +603,25 @@ static int ensure_batch_buffers_locked(Engine& E, size_t nt, size_t ni, size_t n
     return PQB_OK;
 }
 
-static RepBatchParams batch_params(Engine& E) {
+static RepBatchParams batch_params(Engine& E, const BatchLayout& at) {
     BatchBuffers& B = batch_of(E);
     char* d = static_cast<char*>(B.dbuf);
     RepBatchParams p;
-    p.tasks = reinterpret_cast<const RepTask*>(d + B.off_tasks);
-    p.items = reinterpret_cast<const RepItem*>(d + B.off_items);
-    p.order = reinterpret_cast<const unsigned*>(d + B.off_order);
-    p.binom = reinterpret_cast<const double*>(d + B.off_binom);
-    p.partials = reinterpret_cast<ddc*>(d + B.off_part);
+    p.tasks = reinterpret_cast<const RepTask*>(d + at.tasks);
+    p.items = reinterpret_cast<const RepItem*>(d + at.items);
+    p.order = reinterpret_cast<const unsigned*>(d + at.order);
+    p.binom = reinterpret_cast<const double*>(d + BatchLayout::binom);
+    p.partials = reinterpret_cast<ddc*>(d + at.part);
     p.out = reinterpret_cast<double*>(static_cast<char*>(B.hbuf) + B.off_out);
-    p.head = reinterpret_cast<unsigned*>(d);
-    p.counts = reinterpret_cast<const unsigned*>(d + 64);
+    p.head = reinterpret_cast<unsigned*>(d + BatchLayout::head);
+    p.counts = reinterpret_cast<const unsigned*>(d + BatchLayout::head + 64);
+    p.done = nullptr;
     return p;
+}
+
+static hipError_t launch_batch(int range, const RepBatchParams& p, int grid, int reduce_blocks, hipStream_t st) {
+    return range >= kDDRange0 ? launch_rep_dd(range, p, grid, reduce_blocks, st)
+                              : launch_rep_batch(range, p, grid, reduce_blocks, st);
 }
 
 static int batch_grid_locked(Engine& E, int range) {
@@ -608,24 +636,28 @@ static int batch_grid_locked(Engine& E, int range) {
     return B.grid[range];
 }
 
+static int capture_batch(Engine& E, int range, const RepBatchParams& p, int reduce_blocks, hipGraphExec_t* out) {
+    const int grid = batch_grid_locked(E, range);
+    hipGraph_t g = nullptr;
+    hipError_t e = hipStreamBeginCapture(E.stream, hipStreamCaptureModeThreadLocal);
+    if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
+    hipError_t le = launch_batch(range, p, grid, reduce_blocks, E.stream);
+    e = hipStreamEndCapture(E.stream, &g);
+    if (le != hipSuccess) return hip_fail(le, "batch launch (capture)");
+    if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
+    hipGraphExec_t ex = nullptr;
+    e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    if (e != hipSuccess) return hip_fail(e, "hipGraphInstantiate");
+    *out = ex;
+    return PQB_OK;
+}
+
 static int batch_graph_locked(Engine& E, int range, hipGraphExec_t* out) {
     BatchBuffers& B = batch_of(E);
     if (!B.graph[range]) {
-        const int grid = batch_grid_locked(E, range);
-        const RepBatchParams p = batch_params(E);
-        hipGraph_t g = nullptr;
-        hipError_t e = hipStreamBeginCapture(E.stream, hipStreamCaptureModeThreadLocal);
-        if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
-        hipError_t le = range >= kDDRange0 ? launch_rep_dd(range, p, grid, E.stream)
-                                           : launch_rep_batch(range, p, grid, E.stream);
-        e = hipStreamEndCapture(E.stream, &g);
-        if (le != hipSuccess) return hip_fail(le, "batch launch (capture)");
-        if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
-        hipGraphExec_t ex = nullptr;
-        e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (e != hipSuccess) return hip_fail(e, "hipGraphInstantiate");
-        B.graph[range] = ex;
+        const int st = capture_batch(E, range, batch_params(E, B.at), kReduceBlocks, &B.graph[range]);
+        if (st) return st;
     }
     *out = B.graph[range];
     return PQB_OK;
@@ -813,14 +845,17 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     }
     int st = ensure_batch_buffers_locked(E, live.size(), items.size(), nd);
     if (st) return st;
+    const bool direct = live.size() <= kDirectTasks;
+    BatchLayout at = B.at;
+    if (direct) at.set(live.size(), items.size(), nd);
     char* h = static_cast<char*>(B.hbuf);
     char* d = static_cast<char*>(B.dbuf);
     // header: head counter (0), counts
-    std::memset(h, 0, 256);
-    unsigned* counts = reinterpret_cast<unsigned*>(h + 64);
+    std::memset(h + BatchLayout::head, 0, 256);
+    unsigned* counts = reinterpret_cast<unsigned*>(h + BatchLayout::head + 64);
     counts[0] = (unsigned)items.size();
     counts[1] = (unsigned)live.size();
-    RepTask* T = reinterpret_cast<RepTask*>(h + B.off_tasks);
+    RepTask* T = reinterpret_cast<RepTask*>(h + at.tasks);
     // descriptors and per-task data into the pinned staging buffer (disjoint
     // regions per task; ~20 MB for 4096 tasks of up to 26 photons)
     host_parallel((int64_t)live.size(), 256, [&](int64_t lo, int64_t hi) {
@@ -828,9 +863,9 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         const TaskPlan& P = plans[live[(size_t)k]];
         RepTask t;
         std::memset(&t, 0, sizeof(t));
-        t.A = reinterpret_cast<const double2*>(d + B.off_data + a_off[k]);
-        t.base = reinterpret_cast<const double2*>(d + B.off_data + b_off[k]);
-        t.table = reinterpret_cast<const RepStep*>(d + B.off_data + t_off[k]);
+        t.A = reinterpret_cast<const double2*>(d + at.data + a_off[k]);
+        t.base = reinterpret_cast<const double2*>(d + at.data + b_off[k]);
+        t.table = reinterpret_cast<const RepStep*>(d + at.data + t_off[k]);
         t.NS = P.NS;
         t.L = (int)P.L;
         t.nhigh = P.nhigh;
@@ -842,49 +877,64 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         t.nchunks = (uint32_t)P.nchunks;
         t.degree = P.degree;
         t.rows = P.R;
-        t.xrow = reinterpret_cast<const double2*>(d + B.off_data + x_off[k]);
+        t.xrow = reinterpret_cast<const double2*>(d + at.data + x_off[k]);
         t.scale[0] = P.scale;
         for (int hd = 0; hd < P.nhigh; ++hd) {
             t.hrow[hd] = (uint32_t)(1 + P.nlow + hd);
             t.hrad[hd] = P.hrad[(size_t)hd];
         }
         T[k] = t;
-        std::memcpy(h + B.off_data + a_off[(size_t)k], P.A.data(), P.A.size() * sizeof(double));
-        std::memcpy(h + B.off_data + b_off[(size_t)k], P.base.data(), P.base.size() * sizeof(double));
+        std::memcpy(h + at.data + a_off[(size_t)k], P.A.data(), P.A.size() * sizeof(double));
+        std::memcpy(h + at.data + b_off[(size_t)k], P.base.data(), P.base.size() * sizeof(double));
         if (P.degree > 0)
-            std::memcpy(h + B.off_data + x_off[(size_t)k], P.xrow.data(), P.xrow.size() * sizeof(double));
+            std::memcpy(h + at.data + x_off[(size_t)k], P.xrow.data(), P.xrow.size() * sizeof(double));
     }
     });
     host_parallel((int64_t)tables.size(), 4, [&](int64_t lo, int64_t hi) {
         for (int64_t i = lo; i < hi; ++i) {
             const std::vector<int>& rad = plans[live[tables[(size_t)i].second]].low_radix;
-            build_table(rad.data(), rad.size(), reinterpret_cast<RepStep*>(h + B.off_data + tables[(size_t)i].first));
+            build_table(rad.data(), rad.size(), reinterpret_cast<RepStep*>(h + at.data + tables[(size_t)i].first));
         }
     });
-    RepItem* I = reinterpret_cast<RepItem*>(h + B.off_items);
+    RepItem* I = reinterpret_cast<RepItem*>(h + at.items);
     std::memcpy(I, items.data(), items.size() * sizeof(RepItem));
-    unsigned* O = reinterpret_cast<unsigned*>(h + B.off_order);
+    unsigned* O = reinterpret_cast<unsigned*>(h + at.order);
     std::memcpy(O, order.data(), order.size() * sizeof(unsigned));
 
-    hipError_t e = hipMemcpyAsync(d, h, B.off_data + nd, hipMemcpyHostToDevice, E.stream);
+    hipError_t e = hipMemcpyAsync(d + BatchLayout::head, h + BatchLayout::head, at.data + nd - BatchLayout::head,
+                                  hipMemcpyHostToDevice, E.stream);
     if (e != hipSuccess) return hip_fail(e, "batch upload");
     if (any_expanded) {  // outside the graph: it divides the uploaded rows in place, once
-        e = launch_rep_expand(reinterpret_cast<RepTask*>(d + B.off_tasks), (int64_t)live.size(), E.stream);
+        e = launch_rep_expand(reinterpret_cast<RepTask*>(d + at.tasks), (int64_t)live.size(), E.stream);
         if (e != hipSuccess) return drain_fail(E, e, "prep launch");
     }
-    hipGraphExec_t gx = nullptr;
-    st = batch_graph_locked(E, range, &gx);
-    if (st) {
-        (void)hipStreamSynchronize(E.stream);  // the upload may still read the staging buffer
-        return st;
+    if (direct) {
+        RepBatchParams p = batch_params(E, at);
+        if (live.size() == 1) {
+            p.done = reinterpret_cast<unsigned*>(h + B.off_out + 6 * sizeof(double));
+            *p.done = 0u;
+        }
+        e = launch_batch(range, p, batch_grid_locked(E, range), (int)live.size(), E.stream);
+        if (e == hipSuccess) e = p.done ? wait_result(E, p.done) : hipStreamSynchronize(E.stream);
+        if (e != hipSuccess) return drain_fail(E, e, "batch sweep");
+        p.done = nullptr;
+        B.last_direct = p;
+    } else {
+        hipGraphExec_t gx = nullptr;
+        st = batch_graph_locked(E, range, &gx);
+        if (st) {
+            (void)hipStreamSynchronize(E.stream);  // the upload may still read the staging buffer
+            return st;
+        }
+        e = hipGraphLaunch(gx, E.stream);
+        if (e != hipSuccess) return drain_fail(E, e, "hipGraphLaunch");
+        e = hipStreamSynchronize(E.stream);
+        if (e != hipSuccess) return hip_fail(e, "batch sweep");
     }
-    e = hipGraphLaunch(gx, E.stream);
-    if (e != hipSuccess) return drain_fail(E, e, "hipGraphLaunch");
-    e = hipStreamSynchronize(E.stream);
-    if (e != hipSuccess) return hip_fail(e, "batch sweep");
     const double* res = reinterpret_cast<const double*>(h + B.off_out);
     for (size_t k = 0; k < live.size(); ++k) std::copy(&res[6 * k], &res[6 * k] + 6, &out6[6 * live[k]]);
     B.last_range = range;
+    B.last_is_direct = direct;
     B.last_tiny_ns = 0;
     B.last_ntasks = (int)live.size();
     g_last_batch.store(&E);
@@ -903,8 +953,8 @@ static int run_tiny_locked(Engine& E, const pqb_task& t, const SweepChoice& choi
     if (st) return st;
     BatchBuffers& B = batch_of(E);
     char* h = static_cast<char*>(B.hbuf);
-    std::memcpy(h + B.off_data, P.A.data(), P.A.size() * sizeof(double));
-    p.A = reinterpret_cast<const double2*>(h + B.off_data);
+    std::memcpy(h + B.at.data, P.A.data(), P.A.size() * sizeof(double));
+    p.A = reinterpret_cast<const double2*>(h + B.at.data);
     p.out = reinterpret_cast<double*>(h + B.off_out);
     p.scale = P.scale;
     p.done = reinterpret_cast<unsigned*>(p.out + 6);
@@ -1115,20 +1165,27 @@ int batch_replay(int iters, double* ms) {
     if (L.status()) return L.status();
     Engine& E = *L;
     BatchBuffers& B = batch_of(E);
-    const bool tiny = B.last_tiny_ns > 0;
-    if (!tiny && (B.last_range < 0 || !B.graph[B.last_range]))
+    const bool tiny = B.last_tiny_ns > 0, direct = !tiny && B.last_range >= 0 && B.last_is_direct;
+    if (!tiny && !direct && (B.last_range < 0 || !B.graph[B.last_range]))
         return fail(PQB_ERR_ARG, "no batch has been run yet");
+    // the launches of a small batch, captured here
+    hipGraphExec_t gx = tiny ? nullptr : B.graph[B.last_range];
+    if (direct) {
+        const int st = capture_batch(E, B.last_range, B.last_direct, B.last_ntasks, &gx);
+        if (st) return st;
+    }
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hipError_t e = hipEventCreate(&e0);
     if (e == hipSuccess) e = hipEventCreate(&e1);
     if (e == hipSuccess) e = hipEventRecord(e0, E.stream);
     for (int i = 0; e == hipSuccess && i < iters; ++i)
         e = tiny ? launch_tiny(B.last_tiny_ns, B.last_tiny, 1, E.stream)
-                 : hipGraphLaunch(B.graph[B.last_range], E.stream);
+                 : hipGraphLaunch(gx, E.stream);
     if (e == hipSuccess) e = hipEventRecord(e1, E.stream);
     if (e == hipSuccess) e = hipEventSynchronize(e1);
     float f = 0.f;
     if (e == hipSuccess) e = hipEventElapsedTime(&f, e0, e1);
+    if (direct) (void)hipGraphExecDestroy(gx);
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     if (e != hipSuccess) return hip_fail(e, "batch replay");

@@ -346,7 +346,7 @@ const void* rep_dd_kernel_fn(int range) {
     }
 }
 
-hipError_t launch_rep_dd(int range, const RepBatchParams& p, int grid_blocks, hipStream_t st) {
+hipError_t launch_rep_dd(int range, const RepBatchParams& p, int grid_blocks, int reduce_blocks, hipStream_t st) {
     switch (range - kDDRange0) {
         case 0: hipLaunchKernelGGL((rep_dd_kernel<1, 8>), dim3(grid_blocks), dim3(256), 0, st, p); break;
         case 1: hipLaunchKernelGGL((rep_dd_kernel<2, 8>), dim3(grid_blocks), dim3(256), 0, st, p); break;
@@ -356,7 +356,7 @@ hipError_t launch_rep_dd(int range, const RepBatchParams& p, int grid_blocks, hi
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_rep_reduce(p, st);
+    return launch_rep_reduce(p, reduce_blocks, st);
 }
 
 }  // namespace pqb

@@ -231,6 +231,7 @@ void rep_batch_kernel(RepBatchParams p) {
 __global__ __launch_bounds__(kReduceThreads) void rep_reduce_kernel(RepBatchParams p) {
     __shared__ ddc red[kReduceThreads / kWave];
     const unsigned ntasks = to_const(p.counts)[1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *p.head = 0u;
     for (unsigned task = blockIdx.x; task < ntasks; task += gridDim.x) {
         const RepTask& T = p.tasks[task];
         ddc s = {0.0, 0.0, 0.0, 0.0};
@@ -251,10 +252,10 @@ __global__ __launch_bounds__(kReduceThreads) void rep_reduce_kernel(RepBatchPara
             o[3] = s.lr;
             o[4] = s.hi;
             o[5] = s.li;
+            announce(p.done);
         }
         __syncthreads();  // `red` is reused by the next task
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) *p.head = 0u;
 }
 
 // Slot ranges of the batch kernel instantiations.
@@ -278,7 +279,7 @@ int rep_range_for(int min_ns, int max_ns) {
 
 const void* rep_batch_kernel_fn(int range) { return rep_fn(range); }
 
-hipError_t launch_rep_batch(int range, const RepBatchParams& p, int grid_blocks, hipStream_t st) {
+hipError_t launch_rep_batch(int range, const RepBatchParams& p, int grid_blocks, int reduce_blocks, hipStream_t st) {
     switch (range) {
         case 0: hipLaunchKernelGGL((rep_batch_kernel<1, 12>), dim3(grid_blocks), dim3(256), 0, st, p); break;
         case 1: hipLaunchKernelGGL((rep_batch_kernel<1, 20>), dim3(grid_blocks), dim3(256), 0, st, p); break;
@@ -289,11 +290,11 @@ hipError_t launch_rep_batch(int range, const RepBatchParams& p, int grid_blocks,
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_rep_reduce(p, st);
+    return launch_rep_reduce(p, reduce_blocks, st);
 }
 
-hipError_t launch_rep_reduce(const RepBatchParams& p, hipStream_t st) {
-    hipLaunchKernelGGL(rep_reduce_kernel, dim3(kReduceBlocks), dim3(kReduceThreads), 0, st, p);
+hipError_t launch_rep_reduce(const RepBatchParams& p, int blocks, hipStream_t st) {
+    hipLaunchKernelGGL(rep_reduce_kernel, dim3(blocks), dim3(kReduceThreads), 0, st, p);
     return hipGetLastError();
 }
 

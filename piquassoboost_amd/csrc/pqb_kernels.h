@@ -133,11 +133,12 @@ struct RepBatchParams {
     ddc* partials;          // one per item
     double* out;            // 6 doubles per task result
     unsigned* head;         // item counter, zero on entry; the reduce kernel resets it
+    unsigned* done;         // as in PlainParams; one task only
     const unsigned* counts; // device: counts[0] = items, counts[1] = tasks (read by the
                             // kernels, so a captured graph serves every batch that fits)
 };
 
-constexpr int kReduceBlocks = 512;    // fixed grid of the per-task reduction
+constexpr int kReduceBlocks = 512;   // grid of the per-task reduction in a captured graph
 constexpr int kReduceThreads = 256;  // one block of four waves per task
 
 // Kernel instantiations cover slot ranges; rep_range_for() picks the narrowest
@@ -146,9 +147,9 @@ constexpr int kReduceThreads = 256;  // one block of four waves per task
 hipError_t launch_rep_expand(RepTask* tasks, int64_t ntasks, hipStream_t st);
 int rep_range_for(int min_ns, int max_ns);
 const void* rep_batch_kernel_fn(int range);
-hipError_t launch_rep_batch(int range, const RepBatchParams& p, int grid_blocks, hipStream_t st);
+hipError_t launch_rep_batch(int range, const RepBatchParams& p, int grid_blocks, int reduce_blocks, hipStream_t st);
 // per-task sum of the item partials (shared by the FP64 and double-double sweeps)
-hipError_t launch_rep_reduce(const RepBatchParams& p, hipStream_t st);
+hipError_t launch_rep_reduce(const RepBatchParams& p, int blocks, hipStream_t st);
 
 // Double-double sweep over the same tasks and items (precision PQB_PREC_INF).
 // Ranges kDDRange0 .. kDDRange0 + 3 cover up to 8, 16, 32 and 40 slots with a
@@ -158,7 +159,7 @@ constexpr int kRanges = kDDRange0 + 4;
 int rep_dd_range_for(int max_ns);
 int rep_dd_walkers(int range);
 const void* rep_dd_kernel_fn(int range);
-hipError_t launch_rep_dd(int range, const RepBatchParams& p, int grid_blocks, hipStream_t st);
+hipError_t launch_rep_dd(int range, const RepBatchParams& p, int grid_blocks, int reduce_blocks, hipStream_t st);
 
 // ---- adjoint sweep (permanent + all first derivatives of square matrices) ----
 // Adjoint mode: square n x n matrices.  Minors mode: n x (n+1) matrices, the
