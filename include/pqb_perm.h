@@ -304,6 +304,17 @@ int pqb_perm_minors(const double* A, int64_t rows, int64_t cols, int64_t ld, dou
 int pqb_perm_minors_batch(const double* A, int64_t count, int64_t rows, int64_t cols, int64_t ld,
                           int64_t stride, double* out);
 
+/* The photon loop of the generalized-Clifford sampler for `count` samples at once
+ * (fill_r_sample, CGeneralizedCliffordsBSimulationStrategy.cpp:281-305): U is the
+ * modes x modes interferometer, element (i, j) at U[2 * (i * ld + j)]; sample s takes
+ * photons[s] <= max_photons photons (at most PQB_MAX_COLS), photon t entering in input
+ * mode entering[s * max_photons + t] and its output mode drawn from compute_pmf's
+ * distribution (samplingHelperFunctions.cpp:78-342) with the uniform number
+ * draws[s * max_photons + t] (:350-367).  samples: count x modes occupation numbers.
+ * Host pointers, synchronous. */
+int pqb_sample_photons(const double* U, int64_t modes, int64_t ld, int64_t count, int64_t max_photons,
+                       const int64_t* photons, const int64_t* entering, const double* draws, int64_t* samples);
+
 /* Launch plan of the adjoint sweep: plan[0] = M (columns per lane), [1] = K
  * (register bits), [2] = L (lane bits), [3] = H (high bits), [4] = waves per
  * matrix, [5] = blocks, [6] = LDS bytes per block.  waves_resident > 0: plan

@@ -76,6 +76,8 @@ SIGNATURES = {
     "pqb_perm_minors": (ctypes.c_int, [_dp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, _dp]),
     "pqb_perm_minors_batch": (ctypes.c_int, [_dp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
                                              ctypes.c_int64, _dp]),
+    "pqb_sample_photons": (ctypes.c_int, [_dp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
+                                          _i64p, _i64p, _dp, _i64p]),
     "pqb_perm_batch_device_workspace": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
                                                        ctypes.POINTER(ctypes.c_size_t)]),
     "pqb_probe_fp64_fma": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, _dp, _dp]),
@@ -504,6 +506,27 @@ def permanent_minors_batch(A) -> np.ndarray:
         return out
     _check(lib().pqb_perm_minors_batch(M.ctypes.data_as(_dp), count, rows, cols, ld, stride,
                                        out.ctypes.data_as(_dp)))
+    return out
+
+
+def sample_photons(U, photons, entering, draws) -> np.ndarray:
+    """Occupation numbers (count, modes) of `count` samples whose photons enter the modes
+    entering[s, t] and whose output modes are drawn with draws[s, t], t < photons[s]
+    (see pqb_sample_photons)."""
+    M, ld = as_rows(U)
+    modes = M.shape[0]
+    if M.shape[1] != modes:
+        raise Exception("sample_photons: a square interferometer matrix is needed")
+    photons = np.ascontiguousarray(photons, dtype=np.int64)
+    entering = np.ascontiguousarray(entering, dtype=np.int64)
+    draws = np.ascontiguousarray(draws, dtype=np.float64)
+    count = photons.shape[0]
+    if entering.ndim != 2 or entering.shape[0] != count or draws.shape != entering.shape:
+        raise Exception("sample_photons: one row of entering modes and draws per sample is needed")
+    out = np.empty((count, modes), dtype=np.int64)
+    _check(lib().pqb_sample_photons(M.ctypes.data_as(_dp), modes, ld, count, entering.shape[1],
+                                    photons.ctypes.data_as(_i64p), entering.ctypes.data_as(_i64p),
+                                    draws.ctypes.data_as(_dp), out.ctypes.data_as(_i64p)))
     return out
 
 

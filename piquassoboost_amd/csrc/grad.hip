@@ -135,11 +135,9 @@ static int grad_check(int64_t count, int64_t n) {
     return PQB_OK;
 }
 
-// Launch on `st`: dA packed count x n x cols, outputs packed.  `work` holds the
-// partials (grad_partials_bytes).  Adjoint: d_grad count x n x n and d_perm
-// count; minors: d_grad count x (n+1), d_perm unused.
-static int grad_launch(const GradPlan& g, const double2* dA, int n, int64_t count, double2* d_perm,
-                       double2* d_grad, void* work, hipStream_t st) {
+// The sweep's launch on `st`: dA packed count x n x cols, partials at `work`
+// (grad_partials_bytes).
+static int grad_sweep_launch(const GradPlan& g, const double2* dA, int n, void* work, hipStream_t st) {
     if (g.blocks > 0x7fffffff) return fail(PQB_ERR_SIZE, "adjoint launch too large");
     GradParams p;
     p.A = dA;
@@ -149,23 +147,51 @@ static int grad_launch(const GradPlan& g, const double2* dA, int n, int64_t coun
     p.L = g.L;
     p.H = g.H;
     p.wpt = (int)g.wpt;
-    hipError_t e = launch_grad(g.M, g.K, g.minors, p, (int)g.blocks, g.lds, st);
-    if (e != hipSuccess) return hip_fail(e, "adjoint sweep launch");
+    const hipError_t e = launch_grad(g.M, g.K, g.minors, p, (int)g.blocks, g.lds, st);
+    return e == hipSuccess ? PQB_OK : hip_fail(e, "adjoint sweep launch");
+}
+
+// Launch on `st`: dA packed count x n x cols, outputs packed.  `work` holds the
+// partials (grad_partials_bytes).  Adjoint: d_grad count x n x n and d_perm
+// count; minors: d_grad count x (n+1), d_perm unused.
+static int grad_launch(const GradPlan& g, const double2* dA, int n, int64_t count, double2* d_perm,
+                       double2* d_grad, void* work, hipStream_t st) {
+    const int rc = grad_sweep_launch(g, dA, n, work, st);
+    if (rc) return rc;
     GradReduceParams r;
-    r.partials = p.partials;
+    r.partials = static_cast<double2*>(work);
     r.out = d_grad;
     r.tail = nullptr;
     r.main = g.minors ? n + 1 : n * n;
     r.nblk = (int)(g.wpt / 4);
     r.count = (int)count;
     r.scale = std::ldexp(1.0, -(n - 1));
-    e = launch_grad_reduce(r, st);
+    hipError_t e = launch_grad_reduce(r, st);
     if (e != hipSuccess) return hip_fail(e, "adjoint reduction launch");
     if (!g.minors) {  // the permanent from row 0 of the gradient (Laplace expansion)
         e = launch_grad_perm(dA, d_grad, d_perm, n, (int)count, st);
         if (e != hipSuccess) return hip_fail(e, "permanent (Laplace row 0) launch");
     }
     return PQB_OK;
+}
+
+int minors_sweep_plan(int rows, int64_t count, MinorsSweep* out) {
+    GradPlan g;
+    const int st = grad_plan(rows, count, &g, true);
+    if (st) return st;
+    out->rows = rows;
+    out->wpt = g.wpt;
+    out->blocks = g.blocks;
+    out->nblk = (int)(g.wpt / 4);
+    out->partial_bytes = grad_partials_bytes(rows, count, g.wpt, true);
+    return PQB_OK;
+}
+
+int minors_sweep_launch(const MinorsSweep& s, const double2* dA, void* partials, hipStream_t st) {
+    GradPlan g = grad_shape(s.rows, true);
+    g.wpt = s.wpt;
+    g.blocks = s.blocks;
+    return grad_sweep_launch(g, dA, s.rows, partials, st);
 }
 
 static int grad_host_entry(const double* A, int64_t count, int64_t n, int64_t ld, int64_t stride,

@@ -102,6 +102,16 @@ int bind_device(int dev, int* device, int* cus);
 // Resident waves of the plain sweep for `nc` columns on the bound device.
 int64_t resident_waves(int nc, bool expanded);
 
+// A column-minors sweep of `count` packed rows x (rows+1) device matrices without the sum
+// over its partials, nblk x (rows+1) per matrix (grad.hip).
+struct MinorsSweep {
+    int rows = 0, nblk = 0;
+    int64_t wpt = 0, blocks = 0;
+    size_t partial_bytes = 0;
+};
+int minors_sweep_plan(int rows, int64_t count, MinorsSweep* out);
+int minors_sweep_launch(const MinorsSweep& s, const double2* dA, void* partials, hipStream_t st);
+
 struct BatchBuffers;  // persistent-batch buffers and captured graphs (batch.hip)
 
 // One execution context: a stream, a device workspace, a pinned staging

@@ -17,7 +17,8 @@ compute_pmf needs, for every occupied input mode, the permanent of the effective
 with one photon removed from that mode (the reference calls
 BBFGPermanentCalculatorRepeated once per mode).  These are the column minors of the
 expanded (k-1) x k matrix, and one column-minors sweep on the GPU (pqb_perm_minors) gives
-all of them; the per-mode batched form is kept as method="batch".  The random numbers
+all of them; the per-mode batched form is kept as method="batch".  simulate() hands the whole
+photon loop to the GPU (pqb_sample_photons).  The random numbers
 come from the shared std::mt19937 restated in
 ``piquassoboost_amd.sampling.mt19937`` (seeded as the reference does), so seeded runs give
 the reference's samples.
@@ -30,6 +31,7 @@ import time
 import numpy as np
 
 from ... import _capi as C
+from ..mt19937 import MAX as RNG_MAX
 from ..mt19937 import MT19937
 
 # one generator shared by every strategy, as pic::rng_gen (samplingHelperFunctions.cpp:56-60)
@@ -182,46 +184,59 @@ class GeneralizedCliffordsBSimulationStrategy:
         input_state = np.asarray(input_state, dtype=np.int64)
         particles = modes_state_to_particle_state(input_state)
         n_samples = max(0, int(samples_number))
-        if self._pmf_method == "minors" and self._perm is None and n_samples > 1:
-            return self._simulate_lockstep(input_state, particles, n_samples)
+        if self._pmf_method == "minors" and self._perm is None and n_samples > 0:
+            return self._simulate_together(input_state, particles, n_samples)
         samples = []
-        for _ in range(max(0, int(samples_number))):
+        for _ in range(n_samples):
             sample = np.zeros(input_state.shape[0], dtype=np.int64)
             current_input = np.zeros(input_state.shape[0], dtype=np.int64)
             self._fill_r_sample(sample, current_input, particles.copy(), self._photons(input_state))
             samples.append(sample)
         return tuple(samples)
 
-    def _simulate_lockstep(self, input_state, particles, n_samples: int):
-        """The samples advanced together: one column-minors launch per photon step covers
-        every sample still filling.  The random numbers depend on the seed alone (the
+    def _simulate_together(self, input_state, particles, n_samples: int):
+        """The samples advanced together.  The random numbers depend on the seed alone (the
         photon count, which particle enters at each step, the uniform draw of each step),
         never on the permanents, so they are taken first in the order of the sequential
         loop; the samples are those of the sequential loop."""
-        U = self.interferometer_matrix
-        m = input_state.shape[0]
-        inputs, draws = [], []  # per sample: input state after each step, uniform draw of each step
+        entering, draws = [], []  # per sample: mode of the photon entering at each step, uniform draw
         for _ in range(n_samples):
             photons = self._photons(input_state)
-            working = particles.copy()
-            current = np.zeros(m, dtype=np.int64)
-            ins, ds = [], []
-            for _k in range(photons):
-                working = update_input_by_single_photon(current, working)
-                ins.append(current.copy())
-                ds.append(rng_gen.random_double_0_1())
-            inputs.append(ins)
-            draws.append(ds)
-        samples = [np.zeros(m, dtype=np.int64) for _ in range(n_samples)]
-        for k in range(max((len(d) for d in draws), default=0)):
-            active = [s for s in range(n_samples) if len(draws[s]) > k]
-            expanded = [_expanded(U, samples[s], inputs[s][k]) for s in active]
+            working = particles.tolist()
+            raw = rng_gen.take(2 * min(photons, len(working)))  # random_index, random_double_0_1 in turn
+            entering.append([working.pop(v % len(working)) for v in raw[::2]])
+            draws.append([v / float(RNG_MAX) for v in raw[1::2]])
+            if photons > len(particles):
+                update_input_by_single_photon(None, particles[:0])  # raises
+        m = input_state.shape[0]
+        most = max(map(len, draws))
+        # the whole photon loop on the GPU; matrices of another shape and photon counts the
+        # engine does not take go step by step, and fail there as they always did
+        if self.interferometer_matrix.shape == (m, m) and 0 < most <= C.MAX_COLS and C.device_count() > 0:
+            ent = np.zeros((n_samples, most), dtype=np.int64)
+            uni = np.zeros((n_samples, most))
+            for s in range(n_samples):
+                ent[s, : len(draws[s])] = entering[s]
+                uni[s, : len(draws[s])] = draws[s]
+            return tuple(C.sample_photons(self.interferometer_matrix, [len(d) for d in draws], ent, uni))
+        return self._simulate_lockstep(m, entering, draws)
+
+    def _simulate_lockstep(self, m: int, entering, draws):
+        """The photon loop on the host, one column-minors launch per step for every sample
+        still filling."""
+        U = self.interferometer_matrix
+        samples = [np.zeros(m, dtype=np.int64) for _ in draws]
+        inputs = [np.zeros(m, dtype=np.int64) for _ in draws]
+        for k in range(max(map(len, draws))):
+            active = [s for s in range(len(draws)) if len(draws[s]) > k]
+            for s in active:
+                inputs[s][entering[s][k]] += 1
+            expanded = [_expanded(U, samples[s], inputs[s]) for s in active]
             minors = C.permanent_minors_batch(np.stack([E for E, _ in expanded]))
             for a, s in enumerate(active):
-                current = inputs[s][k]
-                col_idx = np.flatnonzero(current > 0)
+                col_idx = np.flatnonzero(inputs[s] > 0)
                 addends = _addends_from_minors(minors[a], expanded[a][1], col_idx)
-                pmf = _pmf_from_addends(U, samples[s], current, col_idx, addends)
+                pmf = _pmf_from_addends(U, samples[s], inputs[s], col_idx, addends)
                 _sample_with_draw(samples[s], pmf, draws[s][k])
         return tuple(samples)
 
