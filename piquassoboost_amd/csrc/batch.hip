@@ -74,8 +74,8 @@ struct Digit {
 // of tasks on host threads, and fresh vectors per task made the allocator the
 // bottleneck.
 struct PlanScratch {
-    std::vector<int64_t> ri, rm, ci, cm, slot_col;
-    std::vector<Digit> digits, low, high, order_rows;
+    std::vector<int64_t> ri, rm, ci, cm;
+    std::vector<Digit> digits, low, high;
     std::vector<size_t> ord;
 };
 }  // namespace
@@ -228,24 +228,18 @@ int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int
         choice = &own;
     }
     const bool transpose = choice->transpose;
-    // element (r, c) of the oriented compact matrix
-    auto elem = [&](int64_t r, int64_t c, double* re, double* im) {
-        // oriented row r / column c -> original row i, column j
-        const int64_t i = transpose ? ri[(size_t)c] : ri[(size_t)r];
-        const int64_t j = transpose ? ci[(size_t)r] : ci[(size_t)c];
-        *re = A[2 * (i * ld + j)];
-        *im = A[2 * (i * ld + j) + 1];
-    };
+    P.src = A;
+    P.ld = ld;
+    P.transpose = transpose;
     const std::vector<int64_t>& row_m = transpose ? cm : rm;
     const std::vector<int64_t>& col_m = transpose ? rm : cm;
     const std::vector<int64_t>& row_i = transpose ? ci : ri;
+    const std::vector<int64_t>& col_i = transpose ? ri : ci;
 
     // column slots
-    std::vector<int64_t>& slot_col = sc.slot_col;
-    slot_col.clear();
+    int NS = 0;
     for (size_t c = 0; c < col_m.size(); ++c)
-        for (int64_t k = 0; k < col_m[c]; ++k) slot_col.push_back((int64_t)c);
-    const int NS = (int)slot_col.size();
+        for (int64_t k = 0; k < col_m[c]; ++k) P.slot[NS++] = (uint32_t)col_i[c];
 
     // the expanded row, and the anchor: of the others the smallest multiplicity, first occurrence
     size_t expanded = row_m.size();
@@ -264,12 +258,10 @@ int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int
     }
     P.degree = choice->degree;
     P.scale = std::ldexp(1.0, -(int)(N - 1));
-    if (P.degree > 0) {  // the columns' scales follow on the GPU (rep_expand_kernel)
+    if (P.degree > 0) {  // the columns' scales follow on the GPU (rep_layout_kernel)
         P.scale = std::ldexp(1.0, -(int)(N - P.degree - 1));
         for (int d = 2; d <= P.degree; ++d) P.scale *= d;
-        P.xrow.assign((size_t)NS * 2, 0.0);
-        for (int s = 0; s < NS; ++s)
-            elem((int64_t)expanded, slot_col[(size_t)s], &P.xrow[2 * (size_t)s], &P.xrow[2 * (size_t)s + 1]);
+        P.xrow = (uint32_t)row_i[expanded];
     }
     // low / high split: largest radices first into the walk while it fits
     std::vector<size_t>& ord = sc.ord;
@@ -302,46 +294,55 @@ int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int
         for (const Digit& d : high) nch *= (double)(d.m + 1);
         if (nch < 4.0e9) {
             P.nchunks = (uint64_t)nch;
-            // rows of A: anchor, low digits in walk order, high digits
-            std::vector<Digit>& order_rows = sc.order_rows;
-            order_rows.clear();
-            order_rows.push_back({(int64_t)anchor, 1});
-            for (const Digit& d : low) order_rows.push_back(d);
-            for (const Digit& d : high) order_rows.push_back(d);
-            P.R = (int)order_rows.size();
+            // rows: anchor, low digits in walk order, high digits
+            P.R = 0;
+            P.row[P.R++] = (uint32_t)row_i[anchor];
+            for (const Digit& d : low) P.row[P.R++] = (uint32_t)row_i[(size_t)d.src];
+            for (const Digit& d : high) P.row[P.R++] = (uint32_t)row_i[(size_t)d.src];
             P.NS = NS;
             P.N = (int)N;
             P.nlow = (int)low.size();
             P.nhigh = (int)high.size();
             P.L = L;
-            P.A.assign((size_t)P.R * NS * 2, 0.0);
-            for (int r = 0; r < P.R; ++r)
-                for (int s = 0; s < NS; ++s) {
-                    double re, im;
-                    elem(order_rows[(size_t)r].src, slot_col[(size_t)s], &re, &im);
-                    P.A[2 * ((size_t)r * NS + s)] = re;
-                    P.A[2 * ((size_t)r * NS + s) + 1] = im;
-                }
-            P.base.assign((size_t)NS * 2, 0.0);
-            for (int s = 0; s < NS; ++s) {
-                // anchor + sum_low m a: in the order of the reference seed
-                // (BBFGPermanentCalculatorRepeated.hpp:202-226)
-                double br = P.A[2 * (size_t)s], bi = P.A[2 * (size_t)s + 1];
-                for (int d = 0; d < P.nlow; ++d) {
-                    const double m = (double)low[(size_t)d].m;
-                    br += P.A[2 * ((size_t)(1 + d) * NS + s)] * m;
-                    bi += P.A[2 * ((size_t)(1 + d) * NS + s) + 1] * m;
-                }
-                P.base[2 * (size_t)s] = br;
-                P.base[2 * (size_t)s + 1] = bi;
-            }
-            P.low_radix.clear();
-            for (const Digit& d : low) P.low_radix.push_back(d.m + 1);
-            P.hrad.clear();
-            for (const Digit& d : high) P.hrad.push_back((uint32_t)(d.m + 1));
+            for (size_t d = 0; d < low.size(); ++d) P.low_radix[d] = (unsigned char)(low[d].m + 1);
+            for (size_t d = 0; d < high.size(); ++d) P.high_radix[d] = (unsigned char)(high[d].m + 1);
             return PQB_OK;
         }
         target_L *= 4;  // too many chunks for 32-bit chunk indices: walk more per chunk
+    }
+}
+
+// A plan's rows (R x NS), base (NS) and expanded row (NS) from its matrix.
+static void fill_rows(const TaskPlan& P, double* A) {
+    for (int r = 0; r < P.R; ++r)
+        for (int s = 0; s < P.NS; ++s, A += 2) {
+            const double* a = P.entry(r, s);
+            A[0] = a[0];
+            A[1] = a[1];
+        }
+}
+
+static void fill_base(const TaskPlan& P, double* base) {
+    for (int s = 0; s < P.NS; ++s) {
+        // anchor + sum_low m a: in the order of the reference seed
+        // (BBFGPermanentCalculatorRepeated.hpp:202-226)
+        double br = P.entry(0, s)[0], bi = P.entry(0, s)[1];
+        for (int d = 0; d < P.nlow; ++d) {
+            const double m = (double)(P.low_radix[d] - 1);
+            br += P.entry(1 + d, s)[0] * m;
+            bi += P.entry(1 + d, s)[1] * m;
+        }
+        base[2 * s] = br;
+        base[2 * s + 1] = bi;
+    }
+}
+
+static void fill_xrow(const TaskPlan& P, double* x) {
+    for (int s = 0; s < P.NS; ++s, x += 2) {
+        const double* a =
+            P.src + 2 * (P.transpose ? (int64_t)P.slot[s] * P.ld + P.xrow : (int64_t)P.xrow * P.ld + P.slot[s]);
+        x[0] = a[0];
+        x[1] = a[1];
     }
 }
 
@@ -350,9 +351,9 @@ int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int
 // has prod(radix) entries.  A step moves one digit by one, so the weight
 // prod C(m, k) changes by one exact ratio of binomials (an int64: the digits of a
 // walk hold at most 40 photons, prod C <= 2^40) and its sign alternates.
-static void build_table(const int* radix, size_t n, RepStep* tab) {
+static void build_table(const unsigned char* radix, size_t n, RepStep* tab) {
     uint64_t L = 1;
-    for (size_t k = 0; k < n; ++k) L *= (uint64_t)radix[k];
+    for (size_t k = 0; k < n; ++k) L *= radix[k];
     int g[kMaxDigits], o[kMaxDigits];
     int64_t bw[kMaxDigits][kMaxSlots + 1];
     for (size_t k = 0; k < n; ++k) {
@@ -695,9 +696,17 @@ static uint64_t choose_L(double S, double total, int64_t lanes, bool fp64, doubl
     return (uint64_t)L;
 }
 
+// The matrix of every task of a batch, where they share one.
+struct SharedMatrix {
+    const double* A = nullptr;
+    int64_t rows = 0, cols = 0, ld = 0;
+    size_t bytes() const { return (size_t)rows * (size_t)cols * sizeof(double2); }
+};
+
 // Run a list of planned tasks; results (6 doubles each) into out6.  dd: the
 // double-double sweep (a chunk per quad of lanes) instead of the FP64 one.
-static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector<double>& out6, bool dd) {
+static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector<double>& out6, bool dd,
+                            const SharedMatrix& shared = SharedMatrix()) {
     BatchBuffers& B = batch_of(E);
     const size_t nt = plans.size();
     out6.assign(nt * 6, 0.0);
@@ -726,17 +735,17 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         std::vector<size_t> ilo, ihi;
         for (size_t i : live) {
             if (plans[i].NS <= 32) {
-                lo.push_back(std::move(plans[i]));
+                lo.push_back(plans[i]);
                 ilo.push_back(i);
             } else {
-                hi.push_back(std::move(plans[i]));
+                hi.push_back(plans[i]);
                 ihi.push_back(i);
             }
         }
         std::vector<double> olo, ohi;
-        int st = run_tasks_locked(E, lo, olo, dd);
+        int st = run_tasks_locked(E, lo, olo, dd, shared);
         if (st) return st;
-        st = run_tasks_locked(E, hi, ohi, dd);
+        st = run_tasks_locked(E, hi, ohi, dd, shared);
         if (st) return st;
         for (size_t k = 0; k < ilo.size(); ++k) std::copy(&olo[6 * k], &olo[6 * k] + 6, &out6[6 * ilo[k]]);
         for (size_t k = 0; k < ihi.size(); ++k) std::copy(&ohi[6 * k], &ohi[6 * k] + 6, &out6[6 * ihi[k]]);
@@ -823,29 +832,37 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     std::string key;
     std::vector<std::pair<size_t, size_t>> tables;  // (offset, task whose radices it walks)
     std::vector<size_t> a_off(live.size()), b_off(live.size()), x_off(live.size()), t_off(live.size());
-    size_t nd = 0;
+    auto area = [](size_t complexes) { return align256(complexes * sizeof(double2)); };
+    size_t own = 0;  // the tasks' own rows, bases and expanded rows
+    for (size_t k : live) {
+        const TaskPlan& P = plans[k];
+        own += area((size_t)P.R * P.NS) + area((size_t)P.NS) + (P.degree > 0 ? area((size_t)P.NS) : 0);
+    }
+    // a shared matrix is uploaded instead and the tasks' rows formed on the GPU (rep_layout_kernel)
+    const bool direct = live.size() <= kDirectTasks;
+    const bool gather = !direct && shared.A && shared.bytes() <= own;
+    size_t nd = gather ? align256(shared.bytes()) : 0;
+    for (size_t k = 0; k < live.size(); ++k) {
+        const TaskPlan& P = plans[live[k]];
+        key.assign(reinterpret_cast<const char*>(P.low_radix), (size_t)P.nlow);
+        const auto it = table_off.emplace(key, nd);
+        t_off[k] = it.first->second;
+        if (it.second) {
+            tables.emplace_back(nd, k);
+            nd = align256(nd + (size_t)P.L * sizeof(RepStep));
+        }
+    }
+    size_t uploaded = nd;
     for (size_t k = 0; k < live.size(); ++k) {
         const TaskPlan& P = plans[live[k]];
         a_off[k] = nd;
-        nd = align256(nd + P.A.size() * sizeof(double));
-        b_off[k] = nd;
-        nd = align256(nd + P.base.size() * sizeof(double));
-        x_off[k] = nd;
-        nd = align256(nd + P.xrow.size() * sizeof(double));
-        key.assign(P.low_radix.begin(), P.low_radix.end());
-        auto it = table_off.find(key);
-        if (it == table_off.end()) {
-            tables.emplace_back(nd, k);
-            table_off.emplace(key, nd);
-            t_off[k] = nd;
-            nd = align256(nd + (size_t)P.L * sizeof(RepStep));
-        } else {
-            t_off[k] = it->second;
-        }
+        b_off[k] = nd += area((size_t)P.R * P.NS);
+        x_off[k] = nd += area((size_t)P.NS);
+        if (P.degree > 0 && !gather) nd += area((size_t)P.NS);
     }
+    if (!gather) uploaded = nd;
     int st = ensure_batch_buffers_locked(E, live.size(), items.size(), nd);
     if (st) return st;
-    const bool direct = live.size() <= kDirectTasks;
     BatchLayout at = B.at;
     if (direct) at.set(live.size(), items.size(), nd);
     char* h = static_cast<char*>(B.hbuf);
@@ -856,8 +873,12 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     counts[0] = (unsigned)items.size();
     counts[1] = (unsigned)live.size();
     RepTask* T = reinterpret_cast<RepTask*>(h + at.tasks);
+    if (gather)
+        for (int64_t r = 0; r < shared.rows; ++r)
+            std::memcpy(h + at.data + (size_t)r * shared.cols * sizeof(double2), shared.A + 2 * r * shared.ld,
+                        (size_t)shared.cols * sizeof(double2));
     // descriptors and per-task data into the pinned staging buffer (disjoint
-    // regions per task; ~20 MB for 4096 tasks of up to 26 photons)
+    // regions per task)
     host_parallel((int64_t)live.size(), 256, [&](int64_t lo, int64_t hi) {
     for (int64_t k = lo; k < hi; ++k) {
         const TaskPlan& P = plans[live[(size_t)k]];
@@ -870,7 +891,7 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         t.L = (int)P.L;
         t.nhigh = P.nhigh;
         t.nlow = P.nlow;
-        for (int ld = 0; ld < P.nlow; ++ld) t.lrad[ld] = (uint32_t)P.low_radix[(size_t)ld];
+        for (int ld = 0; ld < P.nlow; ++ld) t.lrad[ld] = P.low_radix[ld];
         t.item0 = task_items[k].first;
         t.nitems = task_items[k].second;
         t.out_index = (uint32_t)k;
@@ -881,19 +902,27 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         t.scale[0] = P.scale;
         for (int hd = 0; hd < P.nhigh; ++hd) {
             t.hrow[hd] = (uint32_t)(1 + P.nlow + hd);
-            t.hrad[hd] = P.hrad[(size_t)hd];
+            t.hrad[hd] = P.high_radix[hd];
+        }
+        if (gather) {
+            t.src = reinterpret_cast<const double2*>(d + at.data);
+            t.src_ld = shared.cols;
+            t.transpose = P.transpose;
+            t.src_xrow = P.xrow;
+            std::copy(P.row, P.row + P.R, t.src_row);
+            std::copy(P.slot, P.slot + P.NS, t.src_slot);
+        } else {
+            fill_rows(P, reinterpret_cast<double*>(h + at.data + a_off[(size_t)k]));
+            fill_base(P, reinterpret_cast<double*>(h + at.data + b_off[(size_t)k]));
+            if (P.degree > 0) fill_xrow(P, reinterpret_cast<double*>(h + at.data + x_off[(size_t)k]));
         }
         T[k] = t;
-        std::memcpy(h + at.data + a_off[(size_t)k], P.A.data(), P.A.size() * sizeof(double));
-        std::memcpy(h + at.data + b_off[(size_t)k], P.base.data(), P.base.size() * sizeof(double));
-        if (P.degree > 0)
-            std::memcpy(h + at.data + x_off[(size_t)k], P.xrow.data(), P.xrow.size() * sizeof(double));
     }
     });
     host_parallel((int64_t)tables.size(), 4, [&](int64_t lo, int64_t hi) {
         for (int64_t i = lo; i < hi; ++i) {
-            const std::vector<int>& rad = plans[live[tables[(size_t)i].second]].low_radix;
-            build_table(rad.data(), rad.size(), reinterpret_cast<RepStep*>(h + at.data + tables[(size_t)i].first));
+            const TaskPlan& P = plans[live[tables[(size_t)i].second]];
+            build_table(P.low_radix, (size_t)P.nlow, reinterpret_cast<RepStep*>(h + at.data + tables[(size_t)i].first));
         }
     });
     RepItem* I = reinterpret_cast<RepItem*>(h + at.items);
@@ -901,11 +930,11 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     unsigned* O = reinterpret_cast<unsigned*>(h + at.order);
     std::memcpy(O, order.data(), order.size() * sizeof(unsigned));
 
-    hipError_t e = hipMemcpyAsync(d + BatchLayout::head, h + BatchLayout::head, at.data + nd - BatchLayout::head,
+    hipError_t e = hipMemcpyAsync(d + BatchLayout::head, h + BatchLayout::head, at.data + uploaded - BatchLayout::head,
                                   hipMemcpyHostToDevice, E.stream);
     if (e != hipSuccess) return hip_fail(e, "batch upload");
-    if (any_expanded) {  // outside the graph: it divides the uploaded rows in place, once
-        e = launch_rep_expand(reinterpret_cast<RepTask*>(d + at.tasks), (int64_t)live.size(), E.stream);
+    if (any_expanded || gather) {  // outside the graph: it divides uploaded rows in place, once
+        e = launch_rep_layout(reinterpret_cast<RepTask*>(d + at.tasks), (int64_t)live.size(), E.stream);
         if (e != hipSuccess) return drain_fail(E, e, "prep launch");
     }
     if (direct) {
@@ -947,13 +976,13 @@ static int run_tiny_locked(Engine& E, const pqb_task& t, const SweepChoice& choi
     int st = plan_task(t.A, t.rows, t.cols, t.ld, t.row_mult, t.col_mult, 1, P, &choice);
     if (st || P.nhigh > kTinyDigits) return st;
     TinyParams p = {};
-    for (int d = 0; d < P.nhigh; ++d) p.radix[d] = (unsigned char)P.hrad[(size_t)d];
+    for (int d = 0; d < P.nhigh; ++d) p.radix[d] = P.high_radix[d];
     if (P.nlow != 0 || P.degree != 0 || !tiny_split(p, P.NS, P.R)) return PQB_OK;
-    st = ensure_batch_buffers_locked(E, 1, 1, P.A.size() * sizeof(double));
+    st = ensure_batch_buffers_locked(E, 1, 1, (size_t)P.R * P.NS * sizeof(double2));
     if (st) return st;
     BatchBuffers& B = batch_of(E);
     char* h = static_cast<char*>(B.hbuf);
-    std::memcpy(h + B.at.data, P.A.data(), P.A.size() * sizeof(double));
+    fill_rows(P, reinterpret_cast<double*>(h + B.at.data));
     p.A = reinterpret_cast<const double2*>(h + B.at.data);
     p.out = reinterpret_cast<double*>(h + B.off_out);
     p.scale = P.scale;
@@ -1122,8 +1151,13 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
             t_err = (ntasks > 1 ? "task " + std::to_string(i) + ": " : std::string()) + perr[(size_t)i];
             return pst[(size_t)i];
         }
+    SharedMatrix shared{tasks[0].A, tasks[0].rows, tasks[0].cols, tasks[0].ld};
+    for (int64_t i = 1; i < ntasks && shared.A; ++i)
+        if (tasks[i].A != shared.A || tasks[i].rows != shared.rows || tasks[i].cols != shared.cols ||
+            tasks[i].ld != shared.ld)
+            shared = SharedMatrix();
     std::vector<double> out6;
-    st = run_tasks_locked(E, plans, out6, dd);
+    st = run_tasks_locked(E, plans, out6, dd, shared);
     if (st) return st;
     for (int64_t i = 0; i < ntasks; ++i) {
         out[2 * i] = out6[(size_t)(6 * i)];

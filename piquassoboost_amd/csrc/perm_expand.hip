@@ -162,24 +162,42 @@ __global__ __launch_bounds__(256) void plain_expand_kernel(const double2* __rest
     }
 }
 
-// Repeated-row tasks: the rows are divided in place, the base (anchor + sum of the walked
-// rows' multiples, the seed of every chunk) formed from the quotients, and the product of
-// the scales, each slot's entry of the expanded row, taken into the task's scale.
-__global__ __launch_bounds__(256) void rep_expand_kernel(RepTask* tasks) {
+// Repeated-row tasks.  Of a large batch on one matrix (thousands of transitions of one
+// interferometer) only the tasks' row and slot numbers are uploaded: each task's rows, with
+// a column per slot, and its base (anchor + sum of the walked rows' multiples, the seed of
+// every chunk) are formed here.  4096 transitions of 8..26 photons are 18 MB of them, which
+// cost the host 2.9 ms of a call to lay out, copy, upload and free.  Expanded tasks: the
+// rows are divided by the expanded one, and the product of the scales, each slot's entry of
+// that row, taken into the task's scale.  A block per task; bound by the host's planning,
+// which it follows.
+__global__ __launch_bounds__(256) void rep_layout_kernel(RepTask* tasks) {
+    __shared__ double2 x[kMaxSlots];
     RepTask& T = tasks[blockIdx.x];
-    if (T.degree == 0) return;
+    const bool gather = T.src != nullptr, expand = T.degree > 0;
+    if (!gather && !expand) return;
     const int NS = T.NS, lane = threadIdx.x & (kWave - 1);
     double2* const A = const_cast<double2*>(T.A);
+    auto entry = [&](uint32_t row, int s) {
+        return T.src[T.transpose ? (int64_t)T.src_slot[s] * T.src_ld + row : (int64_t)row * T.src_ld + T.src_slot[s]];
+    };
+    if (expand && threadIdx.x < NS) x[lane] = gather ? entry(T.src_xrow, lane) : T.xrow[lane];
+    __syncthreads();
     if (threadIdx.x >= 3 * kWave) {  // one wave forms the scale beside the others' quotients
-        const ddc f = ddc_times(wave_product(T.xrow, NS, lane), ddc_from(T.scale[0], 0.0));
-        if (lane == 0) {
-            T.scale[0] = f.hr;
-            T.scale[1] = f.lr;
-            T.scale[2] = f.hi;
-            T.scale[3] = f.li;
+        if (expand) {
+            const ddc f = ddc_times(wave_product(x, NS, lane), ddc_from(T.scale[0], 0.0));
+            if (lane == 0) {
+                T.scale[0] = f.hr;
+                T.scale[1] = f.lr;
+                T.scale[2] = f.hi;
+                T.scale[3] = f.li;
+            }
         }
     } else {
-        for (int e = threadIdx.x; e < T.rows * NS; e += 3 * kWave) A[e] = cquot(A[e], T.xrow[e % NS]);
+        for (int e = threadIdx.x; e < T.rows * NS; e += 3 * kWave) {
+            const int r = e / NS, s = e - r * NS;
+            const double2 a = gather ? entry(T.src_row[r], s) : A[e];
+            A[e] = expand ? cquot(a, x[s]) : a;
+        }
     }
     __syncthreads();
     if (threadIdx.x < NS) {
@@ -187,15 +205,22 @@ __global__ __launch_bounds__(256) void rep_expand_kernel(RepTask* tasks) {
         for (int d = 0; d < T.nlow; ++d) {
             const double m = (double)(T.lrad[d] - 1);
             const double2 a = A[(1 + d) * NS + lane];
-            b.x += m * a.x;
-            b.y += m * a.y;
+            if (expand) {
+                b.x += m * a.x;
+                b.y += m * a.y;
+            } else {  // rounded as on the host (fill_base in batch.hip)
+                double px = m * a.x, py = m * a.y;
+                asm volatile("" : "+v"(px), "+v"(py));
+                b.x += px;
+                b.y += py;
+            }
         }
         const_cast<double2*>(T.base)[lane] = b;
     }
 }
 
-hipError_t launch_rep_expand(RepTask* tasks, int64_t ntasks, hipStream_t st) {
-    hipLaunchKernelGGL(rep_expand_kernel, dim3((unsigned)ntasks), dim3(256), 0, st, tasks);
+hipError_t launch_rep_layout(RepTask* tasks, int64_t ntasks, hipStream_t st) {
+    hipLaunchKernelGGL(rep_layout_kernel, dim3((unsigned)ntasks), dim3(256), 0, st, tasks);
     return hipGetLastError();
 }
 

@@ -7,6 +7,7 @@
 #include <string>
 #include <vector>
 
+#include "pqb_kernels.h"
 #include "pqb_perm.h"
 
 namespace pqb {
@@ -26,7 +27,6 @@ struct PlainPlan {
 
 PlainPlan make_plain_plan(int R, int NC, int64_t waves_resident);
 
-struct TinyParams;
 // `count` R x C plain permanents that one block each evaluates (perm_tiny.hip): p set but
 // for A and out.
 bool plain_tiny(int R, int C, int64_t count, TinyParams& p);
@@ -51,23 +51,32 @@ struct SweepChoice {
     double steps = 0;        // Gray steps
 };
 
-// One planned repeated-row permanent (see batch.hip).
+// One planned repeated-row permanent (see batch.hip).  Its rows are not copied: they are
+// taken from the task's matrix where they are laid out for the sweep.  No allocations of
+// its own, so that thousands of plans cost nothing to make and to drop.
 struct TaskPlan {
     bool trivial = false;      // decided without a sweep: value (tre, tim)
+    bool transpose = false;    // rows of the sweep are columns of the matrix
     double tre = 1.0, tim = 0.0;
+    const double* src = nullptr;  // the matrix, row stride ld
+    int64_t ld = 0;
     int NS = 0;                // column slots
-    int R = 0;                 // rows of A: anchor, low digits, high digits
+    int R = 0;                 // rows: anchor, low digits, high digits
     int N = 0;                 // photons
     int nlow = 0, nhigh = 0;
     uint64_t L = 1;            // walk length
     uint64_t nchunks = 1;
     int degree = 0;            // RepTask::degree
+    uint32_t xrow = 0;         // expanded: the expanded row (column when transposed)
     double scale = 1.0;        // 2^-(N-1); expanded: D! 2^-(N-D-1)
-    std::vector<double> xrow;  // expanded: NS complex, the expanded row
-    std::vector<double> A;     // R x NS complex (interleaved)
-    std::vector<double> base;  // NS complex
-    std::vector<int> low_radix;
-    std::vector<uint32_t> hrad;
+    uint32_t row[kMaxRepRows];    // R rows of the matrix (columns when transposed)
+    uint32_t slot[kMaxSlots];     // NS columns of it (rows when transposed)
+    unsigned char low_radix[kMaxDigits], high_radix[kMaxDigits];  // multiplicity + 1
+
+    TaskPlan() {}              // the arrays stay as they are
+    const double* entry(int r, int s) const {
+        return src + 2 * (transpose ? (int64_t)slot[s] * ld + row[r] : (int64_t)row[r] * ld + slot[s]);
+    }
 };
 
 int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int64_t* rmult,

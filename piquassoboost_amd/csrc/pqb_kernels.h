@@ -86,6 +86,7 @@ constexpr int kMaxDegree = 3;
 constexpr int kExpandedMinSlots = 13;
 constexpr int kMaxDigits = 40;
 constexpr int kMaxSlots = 40;
+constexpr int kMaxRepRows = kMaxDigits + 1;  // anchor and digits
 constexpr int kBinomStride = 41;  // binomial table: binom[m * 41 + k], 0 <= k <= m <= 40
 
 struct RepStep {          // one step of the low-digit Gray walk
@@ -111,11 +112,17 @@ struct RepTask {
     int rows;              // rows of A
     const double2* xrow;   // expanded: NS, the expanded row r
     double scale[4];       // double-double complex: 2^-(N-1); expanded: D! 2^-(N-D-1), times
-                           // prod_s a_rs once rep_expand_kernel has run
+                           // prod_s a_rs once rep_layout_kernel has run
     uint32_t hrow[kMaxDigits];  // row (in A) of high digit h
     uint32_t hrad[kMaxDigits];  // radix m_h + 1 of high digit h (digit 0 varies fastest)
     uint32_t lrad[kMaxDigits];  // radix m_d + 1 of low digit d (row 1 + d); read by the
                                 // double-double sweep, which seeds chunks from A exactly
+    const double2* src;    // A and base are taken from this matrix by rep_layout_kernel
+                           // (row stride src_ld); NULL: they are in place
+    int64_t src_ld;
+    uint32_t transpose;    // rows are the matrix's columns
+    uint32_t src_xrow;     // the expanded row
+    uint32_t src_row[kMaxRepRows], src_slot[kMaxSlots];
 };
 
 struct RepItem {
@@ -143,8 +150,9 @@ constexpr int kReduceThreads = 256;  // one block of four waves per task
 
 // Kernel instantiations cover slot ranges; rep_range_for() picks the narrowest
 // one for a batch (-1: the batch needs splitting at 32 slots).
-// Divides the rows and bases of the expanded tasks by their expanded rows, in place.
-hipError_t launch_rep_expand(RepTask* tasks, int64_t ntasks, hipStream_t st);
+// Rows and bases of the tasks whose matrix is elsewhere; the expanded tasks' are divided by
+// their expanded rows.
+hipError_t launch_rep_layout(RepTask* tasks, int64_t ntasks, hipStream_t st);
 int rep_range_for(int min_ns, int max_ns);
 const void* rep_batch_kernel_fn(int range);
 hipError_t launch_rep_batch(int range, const RepBatchParams& p, int grid_blocks, int reduce_blocks, hipStream_t st);
