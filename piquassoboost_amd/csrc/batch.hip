@@ -346,6 +346,53 @@ static void fill_xrow(const TaskPlan& P, double* x) {
     }
 }
 
+// Whether the double-double sweep may take a plan's rows in two parts (RepTask::split), and
+// E with entries below 2^E.  A column sum of at most 40 rows is then below 2^(E+6), so parts
+// on the grid of 2^(E-47) add up exactly in a double; those below it add up to less than
+// 2^(E-42), and are multiples of 2^(E-92) when no entry but zeros is below 2^(E-40), so they
+// do too.
+static bool split_exact(const TaskPlan& P, int* E) {
+    double most = 0.0, least = HUGE_VAL;
+    for (int r = 0; r < P.R; ++r)
+        for (int s = 0; s < P.NS; ++s)
+            for (int c = 0; c < 2; ++c) {
+                const double v = std::fabs(P.entry(r, s)[c]);
+                if (!(v <= 0x1p900)) return false;
+                most = std::max(most, v);
+                if (v > 0.0) least = std::min(least, v);
+            }
+    if (!(most >= 0x1p-900)) return false;
+    *E = std::ilogb(most) + 1;
+    return least >= std::ldexp(1.0, *E - 40);
+}
+
+// The parts of the rows and of the base.  A chunk's `group` lanes have `own` slots each, lane
+// q from q * own on; a row holds the lanes' k-th slots side by side, (re_hi, re_lo) of each,
+// then (im_hi, im_lo), so that a load of the wave is one line.
+static void fill_split(const TaskPlan& P, int group, double* out) {
+    const int own = (P.NS + group - 1) / group, slots = own * group;
+    auto at = [&](int r, int s, int c) {
+        return out + 2 * ((((size_t)r * own + s % own) * 2 + c) * group + s / own);
+    };
+    int E = 0;
+    (void)split_exact(P, &E);
+    const double shift = std::ldexp(1.5, E + 5);  // ulp 2^(E-47)
+    std::fill(out, out + (size_t)4 * (P.R + 1) * slots, 0.0);
+    for (int s = P.NS; s < slots; ++s) at(P.R, s, 0)[0] = 1.0;  // a padding slot's factor
+    for (int r = 0; r < P.R; ++r) {
+        const double m = r == 0 ? 1.0 : r <= P.nlow ? (double)(P.low_radix[r - 1] - 1) : 0.0;
+        for (int s = 0; s < P.NS; ++s)
+            for (int c = 0; c < 2; ++c) {
+                const double v = P.entry(r, s)[c], hi = (v + shift) - shift, lo = v - hi;
+                double *const o = at(r, s, c), *const b = at(P.R, s, c);
+                o[0] = hi;
+                o[1] = lo;
+                b[0] += m * hi;
+                b[1] += m * lo;
+            }
+    }
+}
+
 // Reflected mixed-radix Gray walk from k = 0 over digits with the given radices
 // (digit 0 moves fastest).  Entry t describes the move into index t; the table
 // has prod(radix) entries.  A step moves one digit by one, so the weight
@@ -728,7 +775,14 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         max_ns = std::max(max_ns, plans[i].NS);
     }
     if (live.empty()) return PQB_OK;
-    const int range = dd ? rep_dd_range_for(max_ns) : rep_range_for(min_ns, max_ns);
+    std::atomic<bool> split{dd};
+    if (dd)
+        host_parallel((int64_t)live.size(), 256, [&](int64_t lo, int64_t hi) {
+            int E = 0;
+            for (int64_t k = lo; k < hi && split; ++k)
+                if (!split_exact(plans[live[(size_t)k]], &E)) split = false;
+        });
+    const int range = dd ? rep_dd_range_for(max_ns, split) : rep_range_for(min_ns, max_ns);
     if (range < 0) {
         // split at 32 slots and run the two halves
         std::vector<TaskPlan> lo, hi;
@@ -832,6 +886,8 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     std::string key;
     std::vector<std::pair<size_t, size_t>> tables;  // (offset, task whose radices it walks)
     std::vector<size_t> a_off(live.size()), b_off(live.size()), x_off(live.size()), t_off(live.size());
+    const int group = (int)(64 / walkers);  // lanes of a chunk
+    auto slots_of = [&](const TaskPlan& P) { return (P.NS + group - 1) / group * group; };
     auto area = [](size_t complexes) { return align256(complexes * sizeof(double2)); };
     size_t own = 0;  // the tasks' own rows, bases and expanded rows
     for (size_t k : live) {
@@ -840,7 +896,7 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     }
     // a shared matrix is uploaded instead and the tasks' rows formed on the GPU (rep_layout_kernel)
     const bool direct = live.size() <= kDirectTasks;
-    const bool gather = !direct && shared.A && shared.bytes() <= own;
+    const bool gather = !direct && !dd && shared.A && shared.bytes() <= own;
     size_t nd = gather ? align256(shared.bytes()) : 0;
     for (size_t k = 0; k < live.size(); ++k) {
         const TaskPlan& P = plans[live[k]];
@@ -857,8 +913,9 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         const TaskPlan& P = plans[live[k]];
         a_off[k] = nd;
         b_off[k] = nd += area((size_t)P.R * P.NS);
-        x_off[k] = nd += area((size_t)P.NS);
+        x_off[k] = nd += area((size_t)P.NS);  // expanded row, or the split rows
         if (P.degree > 0 && !gather) nd += area((size_t)P.NS);
+        if (split) nd += area((size_t)2 * (P.R + 1) * slots_of(P));
     }
     if (!gather) uploaded = nd;
     int st = ensure_batch_buffers_locked(E, live.size(), items.size(), nd);
@@ -914,6 +971,10 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         } else {
             fill_rows(P, reinterpret_cast<double*>(h + at.data + a_off[(size_t)k]));
             fill_base(P, reinterpret_cast<double*>(h + at.data + b_off[(size_t)k]));
+            if (split) {
+                fill_split(P, group, reinterpret_cast<double*>(h + at.data + x_off[(size_t)k]));
+                t.split = reinterpret_cast<const double2*>(d + at.data + x_off[k]);
+            }
             if (P.degree > 0) fill_xrow(P, reinterpret_cast<double*>(h + at.data + x_off[(size_t)k]));
         }
         T[k] = t;
@@ -1115,7 +1176,7 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
         if (st || done) return st;
     }
     // chunks in flight: a lane each (FP64), a group of lanes each (double-double)
-    const int dd_range = rep_dd_range_for(max_photons);
+    const int dd_range = rep_dd_range_for(max_photons, true);
     const int64_t lanes = dd ? (int64_t)batch_grid_locked(E, dd_range) * (kBlock / kWave) * rep_dd_walkers(dd_range)
                              : (int64_t)batch_grid_locked(E, 2) * kBlock;
     const bool large_batch = total >= 1024.0 * (double)lanes;  // steps per lane
@@ -1172,7 +1233,7 @@ int run_plain_dd_list_locked(Engine& E, const double* const* A, const int* R, co
     for (int64_t k = 0; k < n; ++k) {
         const std::vector<int64_t> rm((size_t)R[k], 1), cm((size_t)C[k], 1);
         const double S = std::ldexp(1.0, R[k] - 1);
-        const int range = rep_dd_range_for(C[k]);  // the slots are the columns
+        const int range = rep_dd_range_for(C[k], true);  // the slots are the columns
         const int64_t walkers = (int64_t)batch_grid_locked(E, range) * (kBlock / kWave) * rep_dd_walkers(range);
         const int st = plan_task(A[k], R[k], C[k], ld[k], rm.data(), cm.data(), choose_L(S, S, walkers, false),
                                  plans[(size_t)k], nullptr, true);

@@ -28,11 +28,22 @@
 // q*M .. q*M+M-1 (M = ceil(NS/G), four doubles per slot), multiplies them in
 // two independent chains, and the group combines its partial products with
 // DPP quad permutations (one for a pair, two for a quad).  A wave works on
-// 64/G chunks at a time.  G grows with the slot count so that a lane holds at
-// most 8 slots, which fits the 168 VGPRs of three waves per SIMD: G = 1 up to
-// 8 slots, 2 up to 16, 4 up to 32 (each exchange repeats a product on every
-// lane of the group, so smaller groups do less work); 33..40 slots take 10 per
-// lane at two waves per SIMD.
+// 64/G chunks at a time.  Each exchange repeats a product on every lane of the
+// group, so smaller groups do less work, as far as their registers go.
+//
+// Bound by its FP64 instructions: 38 for a product of two columns.  Two forms:
+//
+// * Rows split on a grid (RepTask::split) for matrices whose entries lie within
+//   2^40 of each other: the column sums are exact, at 5 instructions instead of
+//   11 per component, and short enough that up to 32 slots a pair of lanes holds
+//   them at two waves per SIMD.  The next row is loaded during the product, a
+//   chunk's lanes' parts side by side: lanes 256 bytes apart (32 slots in quads)
+//   took twice the time.  Calls of n = 24 / 26 / 28 / 30: 547 / 2009 / 7740 /
+//   34800 us before, 400 / 1530 / 6140 / 26800 us now (quads up to 32 slots, rows
+//   split: 456 / 1702 / 6594 / 29273).
+// * Any other: normalised double-double sums, at most 8 slots per lane (three
+//   waves per SIMD), G = 1 up to 8 slots, 2 up to 16, 4 up to 32; 33..40 slots
+//   take 10 per lane at two waves per SIMD.
 //
 // The file also holds grad_perm_kernel (the permanent from the finished
 // gradient by a double-double Laplace sum).
@@ -142,24 +153,22 @@ __device__ __forceinline__ void ddc_acc_w(ddc& acc, double w, const ddc& x) {
     }
 }
 
-// Product of all column sums of the chunk: the lane's M slots as two
-// independent chains (same number of products, twice the ILP), then across
-// the group of G lanes.
-template <int G, int M>
-__device__ __forceinline__ ddc group_product(const double (&hr)[M], const double (&lr)[M], const double (&hi)[M],
-                                             const double (&li)[M]) {
+// Product of all column sums of the chunk, column(k) being the lane's k-th: its M slots as
+// two independent chains (same number of products, twice the ILP), then across the group
+// of G lanes.
+template <int G, int M, class Column>
+__device__ __forceinline__ ddc group_product(Column&& column) {
     constexpr int H = M / 2;  // second chain starts at slot H (M >= 2)
-    ddc p = {hr[0], lr[0], hi[0], li[0]};
+    ddc p = column(0);
     if constexpr (M >= 2) {
-        ddc u = {hr[H], lr[H], hi[H], li[H]};
+        ddc u = column(H);
 #pragma unroll
         for (int k = 1; k < M; ++k) {
             if (k == H) continue;
-            const ddc c = {hr[k], lr[k], hi[k], li[k]};
             if (k < H)
-                ddc_mul(p, c);
+                ddc_mul(p, column(k));
             else
-                ddc_mul(u, c);
+                ddc_mul(u, column(k));
         }
         ddc_mul(p, u);
     }
@@ -172,6 +181,93 @@ __device__ __forceinline__ ddc group_product(const double (&hr)[M], const double
         ddc_mul(p, x);  // product of the quad
     }
     return p;
+}
+
+// Weighted double-double sum over one chunk, column sums from the split rows (RepTask::
+// split): each is h + l with h a multiple of the task's grid and l the rest, and neither
+// rounds, so a row's flip is one FMA for each and the pair is normalised when it is
+// multiplied: 5 instructions per component and step against 11 for an error-free sum
+// that keeps it normalised.
+template <int G, int M>
+__device__ __forceinline__ void dd_chunk_split(cptr<RepTask> T, const double* __restrict__ binom, uint32_t chunk,
+                                               int q, ddc& acc) {
+    constexpr int kPitch = 2 * G * M;  // double2 per row, padding slots included
+    const double2* __restrict__ S = T->split + q;  // slot k's parts at 2 k G and (2 k + 1) G
+    double hr[M], lr[M], hi[M], li[M];
+    const double2* base = S + (size_t)T->rows * kPitch;  // anchor and low digits at k = 0
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+        const double2 x = base[2 * k * G], y = base[(2 * k + 1) * G];
+        hr[k] = x.x;
+        lr[k] = x.y;
+        hi[k] = y.x;
+        li[k] = y.y;
+    }
+    auto add = [&](int k, double f, double2 x, double2 y) __attribute__((always_inline)) {
+        hr[k] = fma(f, x.x, hr[k]);
+        lr[k] = fma(f, x.y, lr[k]);
+        hi[k] = fma(f, y.x, hi[k]);
+        li[k] = fma(f, y.y, li[k]);
+    };
+    // slots [k0, M) of a row, at most four (32 VGPRs) in flight
+    auto add_row = [&](uint32_t r, double f, int k0) __attribute__((always_inline)) {
+        const double2* row = S + (size_t)r * kPitch;
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+            if (k < k0) continue;
+            add(k, f, row[2 * k * G], row[(2 * k + 1) * G]);
+            if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto product = [&]() __attribute__((always_inline)) {
+        return group_product<G, M>([&](int k) __attribute__((always_inline)) {
+            ddc c;
+            fast_two_sum(hr[k], lr[k], c.hr, c.lr);
+            fast_two_sum(hi[k], li[k], c.hi, c.li);
+            return c;
+        });
+    };
+    // high digits from the chunk index: coefficient m - 2k, chunk weight (-1)^k C(m, k)
+    double wc = 1.0;
+    uint32_t c = chunk;
+    const int nhigh = T->nhigh;
+    for (int h = 0; h < nhigh; ++h) {
+        const uint32_t r = T->hrad[h];
+        const uint32_t qq = c / r;
+        const uint32_t kd = c - qq * r;
+        c = qq;
+        const int m = (int)r - 1;
+        add_row(T->hrow[h], (double)(m - 2 * (int)kd), 0);
+        const double b = binom[m * kBinomStride + kd];
+        wc *= (kd & 1u) ? -b : b;
+    }
+    const cptr<RepStep> tab = to_const(T->table);
+    const int L = T->L;
+    // the next step's row, or the slots of it that there are registers for, is loaded while
+    // this one's product is formed
+    constexpr int kAhead = M < 4 ? M : M > 12 ? 4 : M > 8 ? 8 : 2;
+    double2 x[kAhead], y[kAhead];
+    RepStep e = tab[0];
+    auto load_ahead = [&](int t) __attribute__((always_inline)) {
+        e = tab[t < L ? t : 0];
+        const double2* row = S + (size_t)e.row * kPitch;
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            x[k] = row[2 * k * G];
+            y[k] = row[(2 * k + 1) * G];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load_ahead(1);
+    ddc_acc_w(acc, wc, product());
+    for (int t = 1; t < L; ++t) {
+        const double f = e.dir ? -2.0 : 2.0, w = wc * e.w;
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) add(k, f, x[k], y[k]);
+        add_row(e.row, f, kAhead);
+        load_ahead(t + 1);
+        ddc_acc_w(acc, w, product());
+    }
 }
 
 // Weighted double-double sum over one chunk (every lane of the group ends
@@ -194,6 +290,7 @@ __device__ __forceinline__ void dd_chunk(cptr<RepTask> T, const double* __restri
         hi[k] = a.y;
         li[k] = 0.0;
     }
+    auto column = [&](int k) __attribute__((always_inline)) { return ddc{hr[k], lr[k], hi[k], li[k]}; };
     // low digits at k = 0: coefficient m
     const int nlow = T->nlow;
     for (int dg = 0; dg < nlow; ++dg) {
@@ -227,7 +324,7 @@ __device__ __forceinline__ void dd_chunk(cptr<RepTask> T, const double* __restri
         const double b = binom[m * kBinomStride + kd];
         wc *= (kd & 1u) ? -b : b;
     }
-    ddc_acc_w(acc, wc, group_product<G, M>(hr, lr, hi, li));
+    ddc_acc_w(acc, wc, group_product<G, M>(column));
     const cptr<RepStep> tab = to_const(T->table);
     const int L = T->L;
     for (int t = 1; t < L; ++t) {
@@ -240,27 +337,29 @@ __device__ __forceinline__ void dd_chunk(cptr<RepTask> T, const double* __restri
             dd_add_d(hr[k], lr[k], f * a.x);
             dd_add_d(hi[k], li[k], f * a.y);
         }
-        ddc_acc_w(acc, wc * e.w, group_product<G, M>(hr, lr, hi, li));
+        ddc_acc_w(acc, wc * e.w, group_product<G, M>(column));
     }
 }
 
-template <int G, int MLO, int MHI>
+template <int G, int MLO, int MHI, bool SPLIT>
 __device__ __forceinline__ void dd_dispatch(int m, cptr<RepTask> T, const double* __restrict__ binom, uint32_t chunk0,
                                             uint32_t count, int q, int walker, ddc& acc) {
     if constexpr (MLO <= MHI) {
         if (m == MLO) {
-            for (uint32_t j = (uint32_t)walker; j < count; j += kWave / G)
-                dd_chunk<G, MLO>(T, binom, chunk0 + j, q, acc);
+            for (uint32_t j = (uint32_t)walker; j < count; j += kWave / G) {
+                if constexpr (SPLIT) dd_chunk_split<G, MLO>(T, binom, chunk0 + j, q, acc);
+                else dd_chunk<G, MLO>(T, binom, chunk0 + j, q, acc);
+            }
         } else {
-            dd_dispatch<G, MLO + 1, MHI>(m, T, binom, chunk0, count, q, walker, acc);
+            dd_dispatch<G, MLO + 1, MHI, SPLIT>(m, T, binom, chunk0, count, q, walker, acc);
         }
     }
 }
 
 // Persistent grid over the work items (same item protocol as rep_batch_kernel);
 // a chunk per group of G lanes, slot counts up to G * MHI.
-template <int G, int MHI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MHI <= 8 ? 3 : 1))) void rep_dd_kernel(
+template <int G, int MHI, bool SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MHI <= 8 ? 3 : SPLIT ? 2 : 1))) void rep_dd_kernel(
     RepBatchParams p) {
     const int lane = threadIdx.x & (kWave - 1);
     const int q = lane & (G - 1);
@@ -277,7 +376,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MHI <= 8 ? 
         const RepItem it = items[idx];
         const cptr<RepTask> T = tasks + it.task;
         ddc acc = {0.0, 0.0, 0.0, 0.0};
-        dd_dispatch<G, 1, MHI>((T->NS + G - 1) / G, T, p.binom, it.chunk0, it.count, q, walker, acc);
+        dd_dispatch<G, 1, MHI, SPLIT>((T->NS + G - 1) / G, T, p.binom, it.chunk0, it.count, q, walker, acc);
         if (q != 0) acc = ddc{0.0, 0.0, 0.0, 0.0};
         const ddc v = wave_reduce(acc);
         if (lane == 0) p.partials[idx] = v;
@@ -320,38 +419,42 @@ hipError_t launch_grad_perm(const double2* A, const double2* G, double2* perm, i
     return hipGetLastError();
 }
 
-// Ranges: lanes per chunk G and slots per lane, by the batch's largest slot count.
-int rep_dd_range_for(int max_ns) {
-    if (max_ns <= 8) return kDDRange0;       // G = 1, up to 8 slots
-    if (max_ns <= 16) return kDDRange0 + 1;  // G = 2, up to 8 per lane
-    if (max_ns <= 32) return kDDRange0 + 2;  // G = 4, up to 8 per lane
-    return kDDRange0 + 3;                    // G = 4, up to 10 per lane
+// Ranges: rows as they are or split, lanes per chunk G and slots per lane, by the batch's
+// largest slot count.
+#define PQB_DD_RANGES(X) \
+    X(0, 1, 8, false) X(1, 2, 8, false) X(2, 4, 8, false) X(3, 4, 10, false) \
+    X(4, 1, 8, true) X(5, 2, 8, true) X(6, 2, 12, true) X(7, 2, 16, true) X(8, 4, 10, true)
+
+int rep_dd_range_for(int max_ns, bool split) {
+#define PQB_CASE(N, G, M, S) \
+    if (S == split && max_ns <= G * M) return kDDRange0 + N;
+    PQB_DD_RANGES(PQB_CASE)
+#undef PQB_CASE
+    return -1;
 }
 
 int rep_dd_walkers(int range) {
-    switch (range - kDDRange0) {
-        case 0: return kWave;
-        case 1: return kWave / 2;
-        default: return kWave / 4;
-    }
+#define PQB_CASE(N, G, M, S) \
+    if (range == kDDRange0 + N) return kWave / G;
+    PQB_DD_RANGES(PQB_CASE)
+#undef PQB_CASE
+    return kWave;
 }
 
 const void* rep_dd_kernel_fn(int range) {
-    switch (range - kDDRange0) {
-        case 0: return reinterpret_cast<const void*>(&rep_dd_kernel<1, 8>);
-        case 1: return reinterpret_cast<const void*>(&rep_dd_kernel<2, 8>);
-        case 2: return reinterpret_cast<const void*>(&rep_dd_kernel<4, 8>);
-        case 3: return reinterpret_cast<const void*>(&rep_dd_kernel<4, 10>);
-        default: return nullptr;
-    }
+#define PQB_CASE(N, G, M, S) \
+    if (range == kDDRange0 + N) return reinterpret_cast<const void*>(&rep_dd_kernel<G, M, S>);
+    PQB_DD_RANGES(PQB_CASE)
+#undef PQB_CASE
+    return nullptr;
 }
 
 hipError_t launch_rep_dd(int range, const RepBatchParams& p, int grid_blocks, int reduce_blocks, hipStream_t st) {
     switch (range - kDDRange0) {
-        case 0: hipLaunchKernelGGL((rep_dd_kernel<1, 8>), dim3(grid_blocks), dim3(256), 0, st, p); break;
-        case 1: hipLaunchKernelGGL((rep_dd_kernel<2, 8>), dim3(grid_blocks), dim3(256), 0, st, p); break;
-        case 2: hipLaunchKernelGGL((rep_dd_kernel<4, 8>), dim3(grid_blocks), dim3(256), 0, st, p); break;
-        case 3: hipLaunchKernelGGL((rep_dd_kernel<4, 10>), dim3(grid_blocks), dim3(256), 0, st, p); break;
+#define PQB_CASE(N, G, M, S) \
+    case N: hipLaunchKernelGGL((rep_dd_kernel<G, M, S>), dim3(grid_blocks), dim3(256), 0, st, p); break;
+        PQB_DD_RANGES(PQB_CASE)
+#undef PQB_CASE
         default: return hipErrorInvalidValue;
     }
     hipError_t e = hipGetLastError();

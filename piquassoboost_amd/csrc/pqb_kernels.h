@@ -117,6 +117,10 @@ struct RepTask {
     uint32_t hrad[kMaxDigits];  // radix m_h + 1 of high digit h (digit 0 varies fastest)
     uint32_t lrad[kMaxDigits];  // radix m_d + 1 of low digit d (row 1 + d); read by the
                                 // double-double sweep, which seeds chunks from A exactly
+    // double-double sweep: rows + 1 rows of the entries' parts (hi, lo) on and below a grid on
+    // which no column sum rounds, the last row being the base, laid out for the lanes of a
+    // chunk (fill_split in batch.hip); NULL: not in such a range
+    const double2* split;
     const double2* src;    // A and base are taken from this matrix by rep_layout_kernel
                            // (row stride src_ld); NULL: they are in place
     int64_t src_ld;
@@ -160,11 +164,12 @@ hipError_t launch_rep_batch(int range, const RepBatchParams& p, int grid_blocks,
 hipError_t launch_rep_reduce(const RepBatchParams& p, int blocks, hipStream_t st);
 
 // Double-double sweep over the same tasks and items (precision PQB_PREC_INF).
-// Ranges kDDRange0 .. kDDRange0 + 3 cover up to 8, 16, 32 and 40 slots with a
-// chunk per 1, 2, 4 and 4 lanes; rep_dd_walkers() = chunks per wave.
+// Ranges from kDDRange0 on cover up to 8, 16, 32 and 40 slots with a chunk per 1, 2, 4 and
+// 4 lanes, then, rows split (RepTask::split), up to 8, 16, 24, 32 and 40 with one per 1, 2,
+// 2, 4 and 4; rep_dd_walkers() = chunks per wave.
 constexpr int kDDRange0 = 5;
-constexpr int kRanges = kDDRange0 + 4;
-int rep_dd_range_for(int max_ns);
+constexpr int kRanges = kDDRange0 + 9;
+int rep_dd_range_for(int max_ns, bool split);
 int rep_dd_walkers(int range);
 const void* rep_dd_kernel_fn(int range);
 hipError_t launch_rep_dd(int range, const RepBatchParams& p, int grid_blocks, int reduce_blocks, hipStream_t st);
