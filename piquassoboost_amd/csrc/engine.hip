@@ -635,16 +635,20 @@ int plain_entry(const double* A, int64_t rows, int64_t cols, int64_t ld, int alg
 //  * exact-route integer matrices: one exact sweep each (as per call);
 //  * double-double route: every matrix planned as a single call would plan it,
 //    all of them in one batched launch;
-//  * FP64 route: one launch per distinct shape, one grid row (blockIdx.y) per
-//    matrix, each row with the single-call launch plan -- so every value is
-//    bit-identical to its pqb_perm call -- with one upload of all +-2A tables,
-//    one download of all results and one synchronisation.
+//  * FP64 route: one launch for all the shapes that are small, else one per
+//    distinct shape with one grid row (blockIdx.y) per matrix, each matrix
+//    with the single-call launch plan -- so every value is bit-identical to
+//    its pqb_perm call -- with one upload of all +-2A tables and one
+//    synchronisation.
 
 struct ListItem {
     int64_t idx;
     int R, C;
     bool expanded;
 };
+
+// Matrices of one tiny shape, and blocks of one larger shape, up to which it shares a launch.
+constexpr size_t kMixedTiny = 256, kMixedBlocks = 2048;
 
 static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld, std::vector<ListItem>& items,
                             double* out) {
@@ -657,7 +661,7 @@ static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld
     struct Group {
         size_t first, count;
         int R, C;
-        bool expanded, tiny;
+        bool expanded, tiny, mixed;
         PlainPlan pl;
         TinyParams t;
         size_t up_off;            // byte offset in the upload: +-2A tables, or (expanded) the matrices
@@ -677,21 +681,26 @@ static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld
         g.tiny = plain_tiny(f.R, f.C, 1, g.t);
         if (!g.tiny)
             g.pl = make_plain_plan(f.expanded ? f.R - 1 : f.R, f.C, E.resident_waves_locked(f.C, f.expanded));
+        // shapes of one launch: those whose matrices are few, as the others fill the chip by
+        // themselves, at their own size of block and registers
+        g.mixed = g.tiny ? g.count <= kMixedTiny
+                         : !g.expanded && g.C >= kMixedMinCols && g.C <= kMixedMaxCols && g.pl.block == kBlock &&
+                               g.count * (size_t)g.pl.blocks <= kMixedBlocks;
         groups.push_back(g);
         k = e;
     }
     const size_t n = items.size();
-    const size_t cnt_off = kCounterBytes;  // offset 0 stays the single-call counter
-    size_t off = cnt_off + round256(n * sizeof(unsigned));
+    size_t off = kCounterBytes;  // offset 0 stays the single-call counter
     for (Group& g : groups) {
         g.part_off = off;
         if (!g.tiny) off += round256(g.count * (size_t)g.pl.blocks * sizeof(ddc));
     }
-    // the upload holds the +-2A tables of the all-rows groups, used in place, and the
+    // the upload holds the counters, zero, the +-2A tables of the all-rows groups, used in place, and the
     // matrices of the expanded ones, whose tables a kernel builds behind it; the matrices of
     // the tiny groups stay in the staging buffer, past the upload
     const size_t up_base = off;
-    size_t up_total = 0, staged = 0;
+    const size_t cnt_off = up_base, no_tables = round256(n * sizeof(unsigned));
+    size_t up_total = 0, staged = no_tables;
     for (int tiny = 0; tiny < 2; ++tiny) {
         for (Group& g : groups)
             if (g.tiny == (tiny != 0)) {
@@ -723,37 +732,65 @@ static int list_fp64_locked(Engine& E, const double* const* A, const int64_t* ld
     unsigned* counters = reinterpret_cast<unsigned*>(d + cnt_off);
     double* const hout = h + staged / sizeof(double);  // the kernels write the results here themselves
     hipError_t e = hipSuccess;
-    if (up_total > 0) {
-        e = hipMemsetAsync(counters, 0, n * sizeof(unsigned), E.stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(d + up_base, h, up_total, hipMemcpyHostToDevice, E.stream);
-    }
+    std::memset(h, 0, n * sizeof(unsigned));
+    auto params_of = [&](const Group& g, size_t o) {
+        const int64_t m2n = (int64_t)2 * g.R * g.C;
+        return plain_params(g.pl, g.R, reinterpret_cast<double2*>(d + g.m2_off) + o * (size_t)m2n, m2n,
+                            reinterpret_cast<ddc*>(d + g.part_off) + o * (size_t)g.pl.blocks,
+                            counters + g.first + o, hout + 6 * (g.first + o));
+    };
+    if (up_total > no_tables) e = hipMemcpyAsync(d + up_base, h, up_total, hipMemcpyHostToDevice, E.stream);
     if (e != hipSuccess) return drain_fail(E, e, "list upload");
     constexpr size_t kMaxGridY = 65535;
+    TinyMixed tiny;
+    PlainMixed small;
+    tiny.shapes = small.shapes = 0;
+    tiny.first[0] = small.first[0] = 0;
+    auto flush_tiny = [&]() {
+        const hipError_t le = tiny.shapes > 0 ? launch_tiny_mixed(tiny, E.stream) : hipSuccess;
+        tiny.shapes = 0;
+        return le;
+    };
+    auto flush_small = [&]() {
+        const hipError_t le = small.shapes > 0 ? launch_plain_mixed(small, E.stream) : hipSuccess;
+        small.shapes = 0;
+        return le;
+    };
     for (Group& g : groups) {
         if (g.tiny) {
             g.t.A = reinterpret_cast<const double2*>(h + g.up_off / sizeof(double));
             g.t.out = hout + 6 * g.first;
-            e = launch_tiny(g.C, g.t, (int64_t)g.count, E.stream);
-            if (e != hipSuccess) return drain_fail(E, e, "list sweep launch");
-            continue;
+            if (g.mixed) {
+                const int k = tiny.shapes++;
+                tiny.p[k] = g.t;
+                tiny.ns[k] = (unsigned char)g.C;
+                tiny.first[k + 1] = tiny.first[k] + (unsigned)g.count;
+                if (tiny.shapes == kTinyShapes) e = flush_tiny();
+            } else {
+                e = launch_tiny(g.C, g.t, (int64_t)g.count, E.stream);
+            }
+        } else if (g.mixed) {
+            const int k = small.shapes++;
+            small.p[k] = params_of(g, 0);
+            small.nc[k] = g.C;
+            small.blocks[k] = (unsigned)g.pl.blocks;
+            small.first[k + 1] = small.first[k] + (unsigned)(g.count * (size_t)g.pl.blocks);
+            if (small.shapes == kMixedShapes) e = flush_small();
+        } else {
+            if (g.expanded)
+                e = launch_plain_expand(reinterpret_cast<const double2*>(d + up_base + g.up_off),
+                                        reinterpret_cast<double2*>(d + g.m2_off), g.C, (int64_t)g.count,
+                                        counters + g.first, E.stream);
+            for (size_t o = 0; e == hipSuccess && o < g.count; o += kMaxGridY) {
+                const size_t nt = std::min(kMaxGridY, g.count - o);
+                e = launch_plain(g.C, g.expanded, params_of(g, o), g.pl.blocks, g.pl.block, (int)nt, E.stream);
+            }
         }
-        double2* const m2 = reinterpret_cast<double2*>(d + g.m2_off);
-        const int64_t m2n = (int64_t)2 * g.R * g.C;
-        if (g.expanded) {
-            e = launch_plain_expand(reinterpret_cast<const double2*>(d + up_base + g.up_off), m2, g.C,
-                                    (int64_t)g.count, counters + g.first, E.stream);
-            if (e != hipSuccess) return drain_fail(E, e, "prep launch");
-        }
-        for (size_t o = 0; o < g.count; o += kMaxGridY) {
-            const size_t nt = std::min(kMaxGridY, g.count - o);
-            const PlainParams p = plain_params(
-                g.pl, g.R, m2 + o * (size_t)m2n, m2n,
-                reinterpret_cast<ddc*>(d + g.part_off) + o * (size_t)g.pl.blocks, counters + g.first + o,
-                hout + 6 * (g.first + o));
-            e = launch_plain(g.C, g.expanded, p, g.pl.blocks, g.pl.block, (int)nt, E.stream);
-            if (e != hipSuccess) return drain_fail(E, e, "list sweep launch");
-        }
+        if (e != hipSuccess) return drain_fail(E, e, "list sweep launch");
     }
+    e = flush_tiny();
+    if (e == hipSuccess) e = flush_small();
+    if (e != hipSuccess) return drain_fail(E, e, "list sweep launch");
     e = hipStreamSynchronize(E.stream);
     if (e != hipSuccess) return drain_fail(E, e, "list sweep");
     for (size_t k = 0; k < n; ++k) {

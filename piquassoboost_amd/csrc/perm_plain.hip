@@ -317,8 +317,78 @@ __device__ __forceinline__ void sweep_run(const char* __restrict__ Mb, const int
     }
 }
 
-// EXPANDED: the sweep over the R-1 rows of a square matrix's expanded table, else over
-// all R rows.  Two kernels and not one with both sweeps: registers are allocated for
+// Block `block` of the `blocks` that sweep matrix `task` of *p.  EXPANDED: over the R-1 rows
+// of a square matrix's expanded table, else over all R rows.
+template <int NC, bool EXPANDED, class Params>
+__device__ __forceinline__ void sweep_block(const Params p, const unsigned block, const unsigned blocks,
+                                            const unsigned task, SeedLds<NC>& seeds, ddc* red, bool& is_last) {
+    ddc* const partials = p->partials + (size_t)task * blocks;
+    unsigned* const counter = p->counter + task;
+    double* const out = p->out + 6 * (size_t)task;
+
+    const int lane = threadIdx.x & (kWave - 1);
+    // the wave index as a scalar: the run bounds, walk positions and row offsets
+    // derived from it are then uniform for the compiler too (scalar loads, SGPR
+    // operands), not only in fact
+    const int64_t wave = (int64_t)block * (blockDim.x / kWave) +
+                         __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int64_t nwaves = ((int64_t)blocks * blockDim.x) / kWave;
+    const char* __restrict__ Mb = reinterpret_cast<const char*>(p->M2 + (size_t)task * p->m2_stride);
+
+    // Where the tables were built on the GPU the launcher does not know their form and
+    // launches this kernel, then the expanded one; each leaves the other's matrices alone.
+    // (Blocks of this launch only change the counter's low bits until the last of them
+    // resets the word.)
+    if (p->by_flag) {
+        const unsigned c = (unsigned)__builtin_amdgcn_readfirstlane((int)*counter);
+        if (((c & kExpandedFlag) != 0) != EXPANDED) return;
+    }
+    double tr, ti;
+    sweep_run<NC, EXPANDED>(Mb, EXPANDED ? p->R - 1 : p->R, p->K, p->B, p->H, wave, nwaves, lane, seeds, tr, ti);
+    const bool lane_on = lane < (1 << p->B);
+    const double ls = (__popc((unsigned)lane) & 1) ? -1.0 : 1.0;
+    tr = lane_on ? ls * tr : 0.0;
+    ti = lane_on ? ls * ti : 0.0;
+
+    ddc v = block_reduce(ddc_from(tr, ti), red);
+
+    // ---- grid reduction: last block sums the per-block partials ----
+    if (threadIdx.x == 0) {
+        ddc_store_through(&partials[block], v);
+        wait_stores();
+        const unsigned done = atomicAdd(counter, 1u) & ~kExpandedFlag;
+        is_last = (done == blocks - 1);
+    }
+    __syncthreads();
+    if (is_last) {
+        ddc s = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (unsigned b = threadIdx.x; b < blocks; b += blockDim.x) {
+            const ddc q = ddc_load_through(&partials[b]);
+            ddc_add(s, q);
+        }
+        s = block_reduce(s, red);
+        if (threadIdx.x == 0) {
+            if constexpr (EXPANDED) {
+                // one row fewer was summed over (2^-(R-2)); the columns' scales follow the table
+                const ddc f = *reinterpret_cast<const ddc*>(Mb + (size_t)2 * (p->R - 1) * NC * sizeof(double2));
+                s = ddc_mul(ddc_scale(s, 2.0 * p->scale), f);
+            } else {
+                s = ddc_scale(s, p->scale);
+            }
+            out[0] = s.hr + s.lr;
+            out[1] = s.hi + s.li;
+            out[2] = s.hr;
+            out[3] = s.lr;
+            out[4] = s.hi;
+            out[5] = s.li;
+            *counter = 0u;  // leave the counter ready for the next launch
+            announce(p->done);
+        }
+    }
+}
+
+// Two kernels and not one with both sweeps: registers are allocated for
 // the whole kernel, and the pair did not fit (28 VGPRs spilled at 30 columns; 156 and
 // 162 VGPRs without a spill apart).
 template <int NC, bool EXPANDED>
@@ -328,73 +398,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NC <= 32 ? 
 void plain_sweep_kernel(PlainParams p) {
     __shared__ ddc red[256 / kWave];
     __shared__ SeedLds<NC> seeds;
-    // batch of equal-size matrices: blockIdx.y is the matrix, gridDim.x blocks each
-    const unsigned task = blockIdx.y;
-    ddc* const partials = p.partials + (size_t)task * gridDim.x;
-    unsigned* const counter = p.counter + task;
-    double* const out = p.out + 6 * (size_t)task;
-
-    const int lane = threadIdx.x & (kWave - 1);
-    // the wave index as a scalar: the run bounds, walk positions and row offsets
-    // derived from it are then uniform for the compiler too (scalar loads, SGPR
-    // operands), not only in fact
-    const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / kWave) +
-                         __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) / kWave;
-    const char* __restrict__ Mb = reinterpret_cast<const char*>(p.M2 + (size_t)task * p.m2_stride);
-
-    // Where the tables were built on the GPU the launcher does not know their form and
-    // launches this kernel, then the expanded one; each leaves the other's matrices alone.
-    // (Blocks of this launch only change the counter's low bits until the last of them
-    // resets the word.)
-    if (p.by_flag) {
-        const unsigned c = (unsigned)__builtin_amdgcn_readfirstlane((int)*counter);
-        if (((c & kExpandedFlag) != 0) != EXPANDED) return;
-    }
-    double tr, ti;
-    sweep_run<NC, EXPANDED>(Mb, EXPANDED ? p.R - 1 : p.R, p.K, p.B, p.H, wave, nwaves, lane, seeds, tr, ti);
-    const bool lane_on = lane < (1 << p.B);
-    const double ls = (__popc((unsigned)lane) & 1) ? -1.0 : 1.0;
-    tr = lane_on ? ls * tr : 0.0;
-    ti = lane_on ? ls * ti : 0.0;
-
-    ddc v = block_reduce(ddc_from(tr, ti), red);
-
-    // ---- grid reduction: last block sums the per-block partials ----
     __shared__ bool is_last;
-    if (threadIdx.x == 0) {
-        ddc_store_through(&partials[blockIdx.x], v);
-        wait_stores();
-        const unsigned done = atomicAdd(counter, 1u) & ~kExpandedFlag;
-        is_last = (done == gridDim.x - 1);
+    // batch of equal-size matrices: blockIdx.y is the matrix, gridDim.x blocks each
+    sweep_block<NC, EXPANDED>(&p, blockIdx.x, gridDim.x, blockIdx.y, seeds, red, is_last);
+}
+
+// The sweeps over all rows of several small shapes in one launch: a list of uneven matrices
+// is otherwise a launch per shape, one after another, each 8 to 25 us that are mostly a block's
+// start and the grid's end.  A block works as in its own shape's launch, so the values are the
+// same.  64 matrices of n = 5..23, a call: 485 us with a launch per shape (the tiny ones'
+// among them, see perm_tiny.hip), 409 / 379 / 365 / 363 us with shapes up to 17 / 19 / 21 / 22
+// columns here (from 20 on a few registers spill outside the walk); with six of n = 23, which
+// fill the chip by themselves, in it as well, 526 us.
+template <int NC>
+__device__ __forceinline__ void mixed_dispatch(int nc, const PlainParams* p, unsigned block, unsigned blocks,
+                                               unsigned task, char* lds, ddc* red, bool& is_last) {
+    if constexpr (NC >= kMixedMinCols) {
+        if (nc == NC)
+            sweep_block<NC, false>(p, block, blocks, task, *reinterpret_cast<SeedLds<NC>*>(lds), red, is_last);
+        else
+            mixed_dispatch<NC - 1>(nc, p, block, blocks, task, lds, red, is_last);
     }
-    __syncthreads();
-    if (is_last) {
-        ddc s = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-        for (unsigned b = threadIdx.x; b < gridDim.x; b += blockDim.x) {
-            const ddc q = ddc_load_through(&partials[b]);
-            ddc_add(s, q);
-        }
-        s = block_reduce(s, red);
-        if (threadIdx.x == 0) {
-            if constexpr (EXPANDED) {
-                // one row fewer was summed over (2^-(R-2)); the columns' scales follow the table
-                const ddc f = *reinterpret_cast<const ddc*>(Mb + (size_t)2 * (p.R - 1) * NC * sizeof(double2));
-                s = ddc_mul(ddc_scale(s, 2.0 * p.scale), f);
-            } else {
-                s = ddc_scale(s, p.scale);
-            }
-            out[0] = s.hr + s.lr;
-            out[1] = s.hi + s.li;
-            out[2] = s.hr;
-            out[3] = s.lr;
-            out[4] = s.hi;
-            out[5] = s.li;
-            *counter = 0u;  // leave the counter ready for the next launch
-            announce(p.done);
-        }
-    }
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void plain_mixed_kernel(PlainMixed m) {
+    __shared__ ddc red[256 / kWave];
+    __shared__ __attribute__((aligned(16))) char lds[sizeof(SeedLds<kMixedMaxCols>)];
+    __shared__ bool is_last;
+    int at = 0;
+#pragma unroll
+    for (int k = 1; k < kMixedShapes; ++k) at += k < m.shapes && blockIdx.x >= m.first[k] ? 1 : 0;
+    const unsigned blocks = m.blocks[at], local = blockIdx.x - m.first[at], task = local / blocks;
+    mixed_dispatch<kMixedMaxCols>(m.nc[at], &m.p[at], local - task * blocks, blocks, task, lds, red, is_last);
+}
+
+hipError_t launch_plain_mixed(const PlainMixed& m, hipStream_t st) {
+    if (m.shapes < 1 || m.shapes > kMixedShapes) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(plain_mixed_kernel, dim3(m.first[m.shapes]), dim3(256), 0, st, m);
+    return hipGetLastError();
 }
 
 // M2 = [+2A ; -2A] for each of `count` packed matrices of n elements.

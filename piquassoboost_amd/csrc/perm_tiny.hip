@@ -17,22 +17,23 @@
 // with the copies, the general sweep and a stream synchronisation; a transition of 10
 // photons to 7 modes, 192 steps: 20.1 us against 71.6 us through the batched launch).
 
+#include <algorithm>
+
 #include "pqb_device.h"
 #include "pqb_kernels.h"
 #include "pqb_terms.h"
 
 namespace pqb {
 
+// Matrix `index` of p, by the whole block.
 template <int NS>
-__global__ __launch_bounds__(1024) void tiny_kernel(TinyParams p) {
-    extern __shared__ double2 lds[];
-    __shared__ ddc red[1024 / kWave];
+__device__ __forceinline__ void tiny_matrix(const TinyParams& p, int64_t index, double2* lds, ddc* red) {
     constexpr int pitch = NS | 1;
     const int R = p.R, P = p.P, T = P + p.S / P;  // T: rows of the two tables
     double2* const rows = lds;
     double2* const tab = rows + R * pitch;
     double* const wt = reinterpret_cast<double*>(tab + T * pitch);
-    const double2* const A = p.A + (int64_t)blockIdx.x * p.stride;
+    const double2* const A = p.A + index * p.stride;
     for (int e = threadIdx.x; e < R * NS; e += blockDim.x) rows[(e / NS) * pitch + e % NS] = A[e];
     __syncthreads();
     for (int e = threadIdx.x; e < T * NS; e += blockDim.x) {
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(1024) void tiny_kernel(TinyParams p) {
     }
     const ddc s = ddc_scale(block_reduce(ddc_from(ar, ai), red), p.scale);
     if (threadIdx.x == 0) {
-        double* const o = p.out + 6 * (int64_t)blockIdx.x;
+        double* const o = p.out + 6 * index;
         o[0] = s.hr + s.lr;
         o[1] = s.hi + s.li;
         o[2] = s.hr;
@@ -83,6 +84,32 @@ __global__ __launch_bounds__(1024) void tiny_kernel(TinyParams p) {
         o[5] = s.li;
         announce(p.done);
     }
+}
+
+template <int NS>
+__global__ __launch_bounds__(1024) void tiny_kernel(TinyParams p) {
+    extern __shared__ double2 lds[];
+    __shared__ ddc red[1024 / kWave];
+    tiny_matrix<NS>(p, blockIdx.x, lds, red);
+}
+
+template <int NS>
+__device__ __forceinline__ void tiny_dispatch(int ns, const TinyParams& p, int64_t index, double2* lds, ddc* red) {
+    if constexpr (NS >= 1) {
+        if (ns == NS) tiny_matrix<NS>(p, index, lds, red);
+        else tiny_dispatch<NS - 1>(ns, p, index, lds, red);
+    }
+}
+
+// The shapes of a list beside each other: seven launches of n = 5..11, each 5 to 10 us of
+// latency, took 60 us of a list's time.  Waves without terms add zeros, so a shape's sums do
+// not depend on the block's size.
+__global__ __launch_bounds__(1024) void tiny_mixed_kernel(TinyMixed m) {
+    extern __shared__ double2 lds[];
+    __shared__ ddc red[1024 / kWave];
+    int at = 0;
+    while (at + 1 < m.shapes && blockIdx.x >= m.first[at + 1]) ++at;
+    tiny_dispatch<kTinySlots>(m.ns[at], m.p[at], blockIdx.x - m.first[at], lds, red);
 }
 
 bool tiny_split(TinyParams& p, int NS, int R) {
@@ -109,10 +136,23 @@ bool tiny_split(TinyParams& p, int NS, int R) {
     return p.lds_bytes <= 60 * 1024;
 }
 
+static int tiny_threads(const TinyParams& p) { return p.S >= 1024 ? 1024 : (p.S + kWave - 1) / kWave * kWave; }
+
 template <int NS>
 static hipError_t launch_tiny_ns(const TinyParams& p, unsigned count, hipStream_t st) {
-    const int threads = p.S >= 1024 ? 1024 : (p.S + kWave - 1) / kWave * kWave;
-    hipLaunchKernelGGL(tiny_kernel<NS>, dim3(count), dim3(threads), p.lds_bytes, st, p);
+    hipLaunchKernelGGL(tiny_kernel<NS>, dim3(count), dim3(tiny_threads(p)), p.lds_bytes, st, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_tiny_mixed(const TinyMixed& m, hipStream_t st) {
+    if (m.shapes < 1 || m.shapes > kTinyShapes) return hipErrorInvalidValue;
+    int threads = 0;
+    unsigned lds = 0;
+    for (int k = 0; k < m.shapes; ++k) {
+        threads = std::max(threads, tiny_threads(m.p[k]));
+        lds = std::max(lds, m.p[k].lds_bytes);
+    }
+    hipLaunchKernelGGL(tiny_mixed_kernel, dim3(m.first[m.shapes]), dim3(threads), lds, st, m);
     return hipGetLastError();
 }
 

@@ -30,6 +30,17 @@ struct PlainParams {
     unsigned* done;      // host memory, set to 1 after `out` (NULL: not wanted)
 };
 
+// Several shapes in one launch of blocks of 256 threads (plain_mixed_kernel).
+constexpr int kMixedMinCols = 11, kMixedMaxCols = 21, kMixedShapes = 16;
+struct PlainMixed {
+    PlainParams p[kMixedShapes];
+    int nc[kMixedShapes];
+    unsigned blocks[kMixedShapes];     // per matrix
+    unsigned first[kMixedShapes + 1];  // first block of each shape, then their total
+    int shapes;
+};
+hipError_t launch_plain_mixed(const PlainMixed& m, hipStream_t st);
+
 // The same sum with products in exact doubles (perm_exact.hip).
 constexpr int kExactBlock = 1024;  // threads per block at most
 struct ExactF64Params {
@@ -77,6 +88,15 @@ struct TinyParams {
 // Fills the split of the digits whose radices are set; false: not for this kernel.
 bool tiny_split(TinyParams& p, int NS, int R);
 hipError_t launch_tiny(int ns, const TinyParams& p, int64_t count, hipStream_t st);
+// Several shapes in one launch.
+constexpr int kTinyShapes = 16;
+struct TinyMixed {
+    TinyParams p[kTinyShapes];
+    unsigned first[kTinyShapes + 1];  // first block of each shape, then their total
+    unsigned char ns[kTinyShapes];
+    int shapes;
+};
+hipError_t launch_tiny_mixed(const TinyMixed& m, hipStream_t st);
 
 // ---- repeated-row / batched sweep ----
 // A row of multiplicity D <= kMaxDegree may be expanded (plan_task): the columns are
