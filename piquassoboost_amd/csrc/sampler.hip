@@ -10,7 +10,7 @@
 // starts: the loop is a chain of launches on one stream, and the drawn modes are written to
 // host memory as they fall.  (With the host in the loop -- a copy each way, a wait and the
 // pmf in numpy per photon -- 8 samples of 20 photons in 60 modes took 5.28 ms, over 90% of it
-// outside the kernels; now 0.36 ms.)
+// outside the kernels; now 0.32 ms, 0.24 of it kernels.)
 //
 // * Photons 1..kHeadPhotons: one launch, a block per sample.  The minors come from the
 //   permanents of all column subsets, F[S] = perm(first |S| rows, columns S), kept in LDS:
@@ -44,8 +44,15 @@ namespace {
 constexpr int kHeadPhotons = 12;
 constexpr int kHeadThreads = 512;
 constexpr int kStepThreads = 256;
+// Columns of a mode's amplitude, and terms of a subset's permanent, that are loaded
+// together: the loops are short and a block is alone on its CU, so a step is latency.
+constexpr int kTogether = 4;
 // pmf of up to this many modes in LDS, of more in device memory
 constexpr int kLdsModes = 1024;
+
+constexpr int choose(int n, int k) { return k > n ? 0 : k == 0 ? 1 : choose(n - 1, k - 1) + choose(n - 1, k); }
+// a level's sets, and the whole, have a thread each
+static_assert(choose(kHeadPhotons - 1, (kHeadPhotons - 1) / 2) < kHeadThreads);
 
 struct SampleParams {
     const double2* Ut;    // columns x modes: the interferometer's entered columns
@@ -53,7 +60,7 @@ struct SampleParams {
     const double* draw;   // count x P: uniform number of each step
     const int* photons;   // count, descending
     int* drawn;           // count x P: output modes
-    int* host_drawn;      // the same in host memory
+    int* host_drawn;      // the same in host memory, of the finished samples
     double2* A;           // count x k x (k + 1): matrix of the next step, packed
     double* pmf;          // count x modes, for modes > kLdsModes
     const double2* partials;  // count x nblk x k (minors sweep)
@@ -69,28 +76,30 @@ __device__ __forceinline__ int draw_mode(const SampleParams& p, const double2* m
                                          double r, double* pm) {
     for (int m = threadIdx.x; m < p.modes; m += blockDim.x) {
         double ar = 0.0, ai = 0.0;
-        for (int j = 0; j < k; ++j) {
-            const double2 u = p.Ut[(int64_t)col[j] * p.modes + m], v = minors[j];
-            ar = fma(v.x, u.x, ar);
-            ar = fma(-v.y, u.y, ar);
-            ai = fma(v.x, u.y, ai);
-            ai = fma(v.y, u.x, ai);
+        for (int j = 0; j < k; j += kTogether) {
+            double2 u[kTogether];
+#pragma unroll
+            for (int q = 0; q < kTogether; ++q) u[q] = p.Ut[(int64_t)col[min(j + q, k - 1)] * p.modes + m];
+#pragma unroll
+            for (int q = 0; q < kTogether; ++q) {
+                const double2 v = j + q < k ? minors[j + q] : make_double2(0.0, 0.0);
+                ar = fma(v.x, u[q].x, ar);
+                ar = fma(-v.y, u[q].y, ar);
+                ai = fma(v.x, u[q].y, ai);
+                ai = fma(v.y, u[q].x, ai);
+            }
         }
         pm[m] = ar * ar + ai * ai;
     }
     __syncthreads();
     if (threadIdx.x >= kWave) return 0;
-    // a lane per run of consecutive modes
+    // a lane per run of consecutive modes; the running sums are compared with r times the
+    // total, not divided by it
     const int lane = threadIdx.x, per = (p.modes + kWave - 1) / kWave;
     const int m0 = min(lane * per, p.modes), m1 = min(m0 + per, p.modes);
     double sum = 0.0;
     for (int m = m0; m < m1; ++m) sum += pm[m];
-    double total = sum;
-#pragma unroll
-    for (int d = kWave / 2; d >= 1; d >>= 1) total += __shfl_xor(total, d, kWave);
-    double run = 0.0;
-    for (int m = m0; m < m1; ++m) run += pm[m] / total;
-    double incl = run;  // inclusive sums over the lanes
+    double incl = sum;  // inclusive sums over the lanes
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
         const double o = __shfl_up(incl, d, kWave);
@@ -98,26 +107,31 @@ __device__ __forceinline__ int draw_mode(const SampleParams& p, const double2* m
     }
     double before = __shfl_up(incl, 1, kWave);
     if (lane == 0) before = 0.0;
-    const unsigned long long hit = __ballot(m0 < m1 && incl >= r);
+    const double total = __shfl(incl, kWave - 1, kWave);
+    if (!(total > 0.0 && total <= 1.7976931348623157e308)) return 0;  // no weight, infinite, NaN
+    const double level = r * total;
+    const unsigned long long hit = __ballot(m0 < m1 && incl >= level);
     if (hit == 0) return 0;
     const int who = __builtin_ctzll(hit);
     int got = -1, last = m0;
     if (lane == who) {
         double at = 0.0;
         for (int m = m0; m < m1 && got < 0; ++m) {
-            const double w = pm[m] / total;
-            at += w;
-            if (w > 0.0) last = m;
-            if (before + at >= r) got = m;
+            at += pm[m];
+            if (pm[m] > 0.0) last = m;
+            if (before + at >= level) got = m;
         }
         if (got < 0) got = last;  // the lanes' sums round differently
     }
     return __shfl(got, who, kWave);
 }
 
-__device__ __forceinline__ void record_mode(const SampleParams& p, int s, int k, int mode) {
-    p.drawn[(int64_t)s * p.P + k - 1] = mode;
-    p.host_drawn[(int64_t)s * p.P + k - 1] = mode;
+// The modes drawn up to step k, for the next step or, after the sample's last, for the
+// host.  Written once per launch: a barrier waits for the stores before it, those over the
+// bus too.
+__device__ __forceinline__ void record_modes(const SampleParams& p, int s, int n, int k, const int* row) {
+    int* const to = (n == k ? p.host_drawn : p.drawn) + (int64_t)s * p.P;
+    if (threadIdx.x < (unsigned)k) to[threadIdx.x] = row[threadIdx.x];
 }
 
 // The k x (k + 1) matrix of step k + 1: rows the modes drawn so far, columns the entered ones.
@@ -135,11 +149,38 @@ __global__ __launch_bounds__(kHeadThreads) void sample_head_kernel(SampleParams 
     __shared__ double2 minors[kHeadPhotons];
     __shared__ double pm_lds[kLdsModes];
     __shared__ int col[kHeadPhotons + 1], row[kHeadPhotons];
+    __shared__ double draw[kHeadPhotons];
+    // the subsets of the earlier columns by size, then value: those of i of the first b
+    // columns are the first C(b, i) of their size's, so that a level's sets go to as many
+    // consecutive threads.  (With a test of every subset's size instead, a store of each
+    // mode to the host as it falls and a second scan over the normalised weights, the same
+    // run took 352 us against 318.)
+    __shared__ int binom[kHeadPhotons][kHeadPhotons + 1], first[kHeadPhotons + 1];
+    __shared__ unsigned short by_size[1 << (kHeadPhotons - 1)];
     const int s = blockIdx.x, tid = threadIdx.x;
     const int n = p.photons[s], last = min(n, kHeadPhotons);
     double* const pm = p.modes <= kLdsModes ? pm_lds : p.pmf + (int64_t)s * p.modes;
     if (tid <= kHeadPhotons && tid < n) col[tid] = p.enter[(int64_t)s * p.P + tid];
+    if (tid >= kWave && tid - kWave < last) draw[tid - kWave] = p.draw[(int64_t)s * p.P + tid - kWave];
     if (tid == 0) F[0] = make_double2(1.0, 0.0);
+    if (tid < kHeadPhotons * (kHeadPhotons + 1)) {
+        const int b = tid / (kHeadPhotons + 1), size = tid % (kHeadPhotons + 1);
+        int c = size > b ? 0 : 1;
+        for (int q = 1; q <= size; ++q) c = c * (b - size + q) / q;  // C(b, size)
+        binom[b][size] = c;
+    }
+    __syncthreads();
+    if (tid <= kHeadPhotons) {
+        int at = 0;
+        for (int q = 0; q < tid; ++q) at += binom[kHeadPhotons - 1][q];
+        first[tid] = at;
+    }
+    __syncthreads();
+    for (unsigned e = tid; e < (1u << (kHeadPhotons - 1)); e += blockDim.x) {
+        int at = first[__builtin_popcount(e)], size = 0;
+        for (unsigned left = e; left; left &= left - 1) at += binom[__builtin_ctz(left)][++size];
+        by_size[at] = (unsigned short)e;
+    }
     __syncthreads();
     for (int k = 1; k <= last; ++k) {
         // a[i][j], i < k - 1, j < k: the last row and the last column are new
@@ -149,22 +190,31 @@ __global__ __launch_bounds__(kHeadThreads) void sample_head_kernel(SampleParams 
                 a[tid - kWave][k - 1] = p.Ut[(int64_t)col[k - 1] * p.modes + row[tid - kWave]];
             __syncthreads();
         }
-        const unsigned old = 1u << (k - 1);  // subsets of the earlier columns; also the new column's bit
+        const unsigned old = 1u << (k - 1);  // the new column's bit
         for (int i = 1; i < k; ++i) {
             // sets of i columns, the new one among them; at the last level also the set of
             // all the earlier columns, whose row has just been drawn
-            for (unsigned e = tid; e < old; e += blockDim.x) {
-                const bool whole = i == k - 1 && e == old - 1;
-                if (__builtin_popcount(e) != i - 1 && !whole) continue;
-                const unsigned T = whole ? e : e | old;
+            const int sets = binom[k - 1][i - 1];
+            if (tid < sets + (i == k - 1)) {
+                const unsigned T = tid < sets ? by_size[first[i - 1] + tid] | old : old - 1;
                 double2 f = make_double2(0.0, 0.0);
-                for (unsigned left = T; left; left &= left - 1) {
-                    const int j = __builtin_ctz(left);
-                    const double2 c = a[i - 1][j], g = F[T ^ (1u << j)];
-                    f.x = fma(c.x, g.x, f.x);
-                    f.x = fma(-c.y, g.y, f.x);
-                    f.y = fma(c.x, g.y, f.y);
-                    f.y = fma(c.y, g.x, f.y);
+                unsigned left = T;  // i columns
+                for (int t = 0; t < i; t += kTogether) {
+                    double2 c[kTogether], g[kTogether];
+#pragma unroll
+                    for (int q = 0; q < kTogether; ++q) {
+                        const unsigned bit = left & (0u - left);
+                        left ^= bit;
+                        c[q] = bit ? a[i - 1][__builtin_ctz(bit | old << 1)] : make_double2(0.0, 0.0);
+                        g[q] = F[bit ? T ^ bit : 0u];
+                    }
+#pragma unroll
+                    for (int q = 0; q < kTogether; ++q) {
+                        f.x = fma(c[q].x, g[q].x, f.x);
+                        f.x = fma(-c[q].y, g[q].y, f.x);
+                        f.y = fma(c[q].x, g[q].y, f.y);
+                        f.y = fma(c[q].y, g[q].x, f.y);
+                    }
                 }
                 F[T] = f;
             }
@@ -172,13 +222,11 @@ __global__ __launch_bounds__(kHeadThreads) void sample_head_kernel(SampleParams 
         }
         if (tid < k) minors[tid] = F[(2 * old - 1) ^ (1u << tid)];
         __syncthreads();
-        const int mode = draw_mode(p, minors, col, k, p.draw[(int64_t)s * p.P + k - 1], pm);
-        if (tid == 0) {
-            row[k - 1] = mode;
-            record_mode(p, s, k, mode);
-        }
+        const int mode = draw_mode(p, minors, col, k, draw[k - 1], pm);
+        if (tid == 0) row[k - 1] = mode;
         __syncthreads();
     }
+    record_modes(p, s, n, last, row);
     if (n > kHeadPhotons) next_matrix(p, s, kHeadPhotons, row, col);
 }
 
@@ -206,18 +254,21 @@ __global__ __launch_bounds__(kStepThreads) void sample_step_kernel(SampleParams 
         red[tid] = v;
     }
     __syncthreads();
+    for (int left = slices; left > 1;) {
+        const int half = (left + 1) / 2;
+        if (slice < left - half) ddc_add(red[tid], red[tid + half * k]);
+        __syncthreads();
+        left = half;
+    }
     if (tid < k) {
-        for (int q = 1; q < slices; ++q) ddc_add(v, red[q * k + tid]);
-        v = ddc_scale(v, p.scale);
+        v = ddc_scale(red[tid], p.scale);
         minors[tid] = make_double2(v.hr + v.lr, v.hi + v.li);
     }
     __syncthreads();
     const int mode = draw_mode(p, minors, col, k, p.draw[(int64_t)s * p.P + k - 1], pm);
-    if (tid == 0) {
-        row[k - 1] = mode;
-        record_mode(p, s, k, mode);
-    }
+    if (tid == 0) row[k - 1] = mode;
     __syncthreads();
+    record_modes(p, s, n, k, row);
     if (n > k) next_matrix(p, s, k, row, col);
 }
 
