@@ -36,10 +36,10 @@ N = 30
 M_MODES = 60
 SEED = 1002
 FP64_PEAK_TFLOPS = 78.6  # MI355X FP64 vector (and matrix) peak
-# HBM bytes per launch of the n=30 sweep: FETCH_SIZE x 2.00 + WRITE_SIZE x 1.00 (factors from a
+# HBM bytes per n=30 permanent (table, both sweeps' launches): FETCH_SIZE x 2.00 + WRITE_SIZE x 1.00 (factors from a
 # 256 MiB copy kernel), measured with rocprofv3 --pmc on this workload
 # (profiles/plain_sweep_n30_counters.md).
-TRAFFIC_BYTES_N30 = 863296
+TRAFFIC_BYTES_N30 = 776672
 
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tests", "golden")
@@ -385,8 +385,8 @@ def grad_leg(reps: int = 10) -> dict:
 def sampling_leg(photons: int = 20, modes: int = 60, shots: int = 8) -> dict:
     """Seeded generalized-Clifford boson sampling (20 photons in modes 0..19 of a 60-mode
     Haar interferometer, seed 1010): time per sample with compute_pmf's permanents from one
-    column-minors sweep per photon step (the samples advanced together, one batched launch
-    per step), from the per-mode batched permanents (one sample at a time), and from the
+    column-minors sweep per photon step (the samples advanced together, the whole photon loop
+    on the GPU), from the per-mode batched permanents (one sample at a time), and from the
     oracle's restated reference sweep on the host (one call per mode, as the reference
     does).  All three draw the same samples.  Each GPU method runs once untimed first (the
     first launches of a process load the kernels)."""
