@@ -30,6 +30,7 @@
 
 #include "pqb_perm.h"
 #include "pqb_device.h"
+#include "pqb_exact_rule.h"
 #include "pqb_kernels.h"
 #include "pqb_engine.h"
 
@@ -412,18 +413,6 @@ static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 typedef __int128 i128;
 
 static double i128_to_double(i128 v) { return (double)v; }
-
-// Steps between flushes of the exact sweep on the FP64 pipe, 0: its group products may
-// exceed 46 bits (perm_exact.hip).
-static int exact_fp64_flush(int64_t cmax, int C) {
-    const int g = (C + 2) / 3;
-    int64_t q = 1;
-    for (int k = 0; k < g; ++k) {
-        q *= std::max<int64_t>(cmax, 1);
-        if (q > ((int64_t)1 << 46)) return 0;
-    }
-    return 1 << std::min(8, 140 - 3 * ceil_log2(q));
-}
 
 // Exact route: sum_delta (prod delta) prod_j c_j  (mod 2^128) on the GPU,
 // then divide by 2^(R-1).  The caller holds the lease of E.
