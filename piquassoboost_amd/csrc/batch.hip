@@ -562,6 +562,14 @@ struct BatchBuffers {
     bool last_is_direct = false;      // last_direct, of last_ntasks tasks
     RepBatchParams last_direct = {};
 
+    // Nothing to replay: before a buffer is written over, and until the batch it is written
+    // for has run (the last one's launches would read the new one's counts and tasks).
+    void forget_last() {
+        last_range = -1;
+        last_ntasks = 0;
+        last_tiny_ns = 0;
+    }
+
     void layout(size_t nt, size_t ni, size_t nd) {
         cap_tasks = nt;
         cap_items = ni;
@@ -596,9 +604,7 @@ void release_batch_locked(Engine& E) {
     B.dbuf = B.hbuf = nullptr;
     B.cap_tasks = B.cap_items = B.cap_data = 0;
     for (int& g : B.grid) g = 0;
-    B.last_range = -1;
-    B.last_ntasks = 0;
-    B.last_tiny_ns = 0;
+    B.forget_last();
 }
 
 // The context whose batch ran last: pqb_batch_replay replays it.
@@ -609,8 +615,7 @@ static int ensure_batch_buffers_locked(Engine& E, size_t nt, size_t ni, size_t n
     if (B.dbuf && nt <= B.cap_tasks && ni <= B.cap_items && nd <= B.cap_data) return PQB_OK;
     (void)hipStreamSynchronize(E.stream);
     B.drop_graphs();
-    B.last_range = -1;  // nothing to replay in the buffers that follow
-    B.last_tiny_ns = 0;
+    B.forget_last();
     if (B.dbuf) (void)hipFree(B.dbuf);
     if (B.hbuf) (void)hipHostFree(B.hbuf);
     B.dbuf = B.hbuf = nullptr;
@@ -922,6 +927,7 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     if (st) return st;
     BatchLayout at = B.at;
     if (direct) at.set(live.size(), items.size(), nd);
+    B.forget_last();
     char* h = static_cast<char*>(B.hbuf);
     char* d = static_cast<char*>(B.dbuf);
     // header: head counter (0), counts
@@ -1025,7 +1031,6 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
     for (size_t k = 0; k < live.size(); ++k) std::copy(&res[6 * k], &res[6 * k] + 6, &out6[6 * live[k]]);
     B.last_range = range;
     B.last_is_direct = direct;
-    B.last_tiny_ns = 0;
     B.last_ntasks = (int)live.size();
     g_last_batch.store(&E);
     return PQB_OK;
@@ -1042,6 +1047,7 @@ static int run_tiny_locked(Engine& E, const pqb_task& t, const SweepChoice& choi
     st = ensure_batch_buffers_locked(E, 1, 1, (size_t)P.R * P.NS * sizeof(double2));
     if (st) return st;
     BatchBuffers& B = batch_of(E);
+    B.forget_last();
     char* h = static_cast<char*>(B.hbuf);
     fill_rows(P, reinterpret_cast<double*>(h + B.at.data));
     p.A = reinterpret_cast<const double2*>(h + B.at.data);
@@ -1054,7 +1060,6 @@ static int run_tiny_locked(Engine& E, const pqb_task& t, const SweepChoice& choi
     if (e != hipSuccess) return drain_fail(E, e, "batch sweep");
     out[0] = p.out[0];
     out[1] = p.out[1];
-    B.last_range = -1;
     B.last_ntasks = 1;
     B.last_tiny_ns = P.NS;
     B.last_tiny = p;
