@@ -40,6 +40,7 @@
 #include "pqb_device.h"
 #include "pqb_engine.h"
 #include "pqb_kernels.h"
+#include "pqb_pivot.h"
 
 namespace pqb {
 
@@ -128,9 +129,7 @@ constexpr double kExpandMinSteps = 4096.0;
 // instead of 6 FP64 instructions per column -- of the D + 1 steps it replaces, 0.80, 0.72,
 // 0.67 of the instructions at D = 1, 2, 3 and 26 columns, 0.78, 0.68, 0.61 at 16.  The
 // cheapest orientation and multiplicity whose entries allow it is taken; the conditions
-// are those of the plain sweep (perm_expand.hip): a row without an entry below 2^-16 of
-// the matrix's largest, all of it inside [2^-20, 2^20], entries finite and not all whole
-// numbers.
+// are those of the plain sweep (pqb_pivot.h).
 static SweepChoice choose_sweep(const double* A, int64_t ld, const PlanScratch& sc, bool expand) {
     SweepChoice c;
     const double sr = sweep_steps(sc.rm), st = sweep_steps(sc.cm);
@@ -169,25 +168,23 @@ static SweepChoice choose_sweep(const double* A, int64_t ld, const PlanScratch& 
     if (nc == 0) return c;
     std::sort(cand, cand + nc, [](const Candidate& a, const Candidate& b) { return a.cost < b.cost; });
 
-    constexpr double kLargest = 0x1p20, kSmallest = 0x1p-20, kSpread = 0x1p-16;
     const size_t R = sc.ri.size(), C = sc.ci.size();
     double row_min[kMaxSlots], col_min[kMaxSlots], hi = 0.0;
     std::fill(row_min, row_min + R, HUGE_VAL);
     std::fill(col_min, col_min + C, HUGE_VAL);
-    bool frac = false;
+    int low = lowest_bit(0.0);
     for (size_t r = 0; r < R; ++r)
         for (size_t k = 0; k < C; ++k) {
             const double* a = A + 2 * (sc.ri[r] * ld + sc.ci[k]);
-            const double x = std::fabs(a[0]), y = std::fabs(a[1]);
-            if (!(x <= kLargest && y <= kLargest)) return c;
-            frac = frac || a[0] != std::rint(a[0]) || a[1] != std::rint(a[1]);
-            const double v = std::max(x, y);
+            if (!pivot_admits(a[0], a[1])) return c;
+            const double v = std::max(std::fabs(a[0]), std::fabs(a[1]));
             row_min[r] = std::min(row_min[r], v);
             col_min[k] = std::min(col_min[k], v);
             hi = std::max(hi, v);
+            if (!off_grid(low, hi)) low = std::min(low, lowest_bit(a[0], a[1]));  // off it, it stays off
         }
-    if (!frac) return c;
-    const double least = std::max(kSmallest, kSpread * hi);
+    if (!off_grid(low, hi)) return c;
+    const double least = pivot_least(hi);
     for (int q = 0; q < nc; ++q) {
         const std::vector<int64_t>& m = cand[q].transpose ? sc.cm : sc.rm;
         const double* mins = cand[q].transpose ? col_min : row_min;

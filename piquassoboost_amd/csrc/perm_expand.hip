@@ -17,8 +17,10 @@
 //    are then below 40 x 2^16.5, their products over 40 columns and the sum over
 //    2^39 vectors below 2^950, and the product of the scales is above 2^-800;
 //  * an entry is not finite or beyond 2^20;
-//  * every entry is a (Gaussian) integer: small integer matrices sum without
-//    rounding, which a division would lose.
+//  * every entry is a (Gaussian) whole number of up to 21 bits times a power of two that
+//    they share: small ones sum without rounding, which a division would lose (rows of
+//    +-1.5 among +-0.5 at n = 14: 1572.0000000000118 for 1572).
+// The rule itself is in pqb_pivot.h.
 // Repeated-row tasks (batch.hip plans them) are divided here too: a row of multiplicity D
 // contributes the coefficient of x^D, times D!.
 //
@@ -28,10 +30,12 @@
 // This unit is compiled without contraction: the exact product splits would
 // otherwise be fused away.
 
+#include <algorithm>
 #include <cmath>
 
 #include "pqb_device.h"
 #include "pqb_kernels.h"
+#include "pqb_pivot.h"
 
 namespace pqb {
 
@@ -89,15 +93,14 @@ __device__ __forceinline__ ddc wave_product(const double2* v, int n, int lane) {
     return f;
 }
 
-constexpr double kLargest = 0x1p20, kSmallest = 0x1p-20, kSpread = 0x1p-16;
-
 }  // namespace
 
 __global__ __launch_bounds__(256) void plain_expand_kernel(const double2* __restrict__ A, double2* __restrict__ M2,
                                                            int n, int64_t m2_stride, unsigned* counters) {
     __shared__ double row_min[kMaxCols];
     __shared__ double row_max[kMaxCols];
-    __shared__ int row_flags[kMaxCols];  // bit 0: an entry not finite or too large; bit 1: one not an integer
+    __shared__ int row_low[kMaxCols];   // lowest bit of the row's entries
+    __shared__ bool row_bad[kMaxCols];  // an entry not finite or too large
     __shared__ int pivot;
     const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     const int64_t task = blockIdx.x;
@@ -106,35 +109,40 @@ __global__ __launch_bounds__(256) void plain_expand_kernel(const double2* __rest
 
     for (int i = wid; i < n; i += 4) {  // a wave per row (n <= 40 <= 64 lanes)
         double lo = __builtin_inf(), hi = 0.0;
-        bool bad = false, frac = false;
+        int low = lowest_bit(0.0);
+        bool bad = false;
         if (lane < n) {
             const double2 v = A[i * n + lane];
             const double x = fabs(v.x), y = fabs(v.y);
-            bad = !(x <= kLargest && y <= kLargest);
-            frac = !(v.x == rint(v.x) && v.y == rint(v.y));
+            bad = !pivot_admits(v.x, v.y);
+            low = lowest_bit(v.x, v.y);
             lo = hi = x > y ? x : y;
         }
         for (int m = kWave / 2; m >= 1; m >>= 1) {
             lo = fmin(lo, __shfl_xor(lo, m, kWave));
             hi = fmax(hi, __shfl_xor(hi, m, kWave));
+            low = min(low, __shfl_xor(low, m, kWave));
         }
-        const bool any_bad = __any(bad), any_frac = __any(frac);
+        const bool any_bad = __any(bad);
         if (lane == 0) {
             row_min[i] = lo;
             row_max[i] = hi;
-            row_flags[i] = (any_bad ? 1 : 0) | (any_frac ? 2 : 0);
+            row_low[i] = low;
+            row_bad[i] = any_bad;
         }
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        int best = 0, flags = 0;
+        int best = 0, low = lowest_bit(0.0);
+        bool bad = false;
         double hi = 0.0;
         for (int i = 0; i < n; ++i) {
             if (row_min[i] > row_min[best]) best = i;
             hi = fmax(hi, row_max[i]);
-            flags |= row_flags[i];
+            low = min(low, row_low[i]);
+            bad = bad || row_bad[i];
         }
-        const bool fits = flags == 2 && row_min[best] >= kSmallest && row_min[best] >= kSpread * hi;
+        const bool fits = !bad && off_grid(low, hi) && row_min[best] >= pivot_least(hi);
         pivot = fits ? best : -1;
         counters[task] = fits ? kExpandedFlag : 0u;
     }
@@ -225,26 +233,24 @@ hipError_t launch_rep_layout(RepTask* tasks, int64_t ntasks, hipStream_t st) {
 }
 
 int plain_expand_row(const double* A, int n, int64_t ld) {
-    int best = -1;
+    int best = -1, low = lowest_bit(0.0);
     double best_min = -1.0, hi = 0.0;
-    bool frac = false;
     for (int i = 0; i < n; ++i) {
         double lo = __builtin_inf();
         for (int j = 0; j < n; ++j) {
             const double re = A[2 * (i * ld + j)], im = A[2 * (i * ld + j) + 1];
-            const double x = std::fabs(re), y = std::fabs(im);
-            if (!(x <= kLargest && y <= kLargest)) return -1;
-            frac = frac || re != std::rint(re) || im != std::rint(im);
-            const double v = x > y ? x : y;
+            if (!pivot_admits(re, im)) return -1;
+            const double x = std::fabs(re), y = std::fabs(im), v = x > y ? x : y;
             lo = v < lo ? v : lo;
             hi = v > hi ? v : hi;
+            if (!off_grid(low, hi)) low = std::min(low, lowest_bit(re, im));  // off it, it stays off
         }
         if (lo > best_min) {
             best_min = lo;
             best = i;
         }
     }
-    return frac && best_min >= kSmallest && best_min >= kSpread * hi ? best : -1;
+    return off_grid(low, hi) && best_min >= pivot_least(hi) ? best : -1;
 }
 
 hipError_t launch_plain_expand(const double2* A, double2* M2, int n, int64_t count, unsigned* counters,
