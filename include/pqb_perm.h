@@ -117,8 +117,8 @@ int pqb_perm(const double* A, int64_t rows, int64_t cols, int64_t ld, int algo,
  * of one shape on the FP64 route share one launch (a grid row per matrix, each
  * with the launch plan of a single call, so each value is bit-identical to
  * the pqb_perm call on that matrix), the double-double route (PQB_PREC_INF)
- * takes one batched launch (the correctly rounded sum, as per call, whenever
- * the sum cancels by less than ~2^45), exact-route integer matrices one sweep
+ * takes one or two batched launches (the correctly rounded sum, as per call,
+ * whenever the sum cancels by less than ~2^45), exact-route integer matrices one sweep
  * each.  A failing matrix fails the call; the message names its index.
  * Synchronous. */
 int pqb_perm_list(const double* const* A, const int64_t* rows, const int64_t* cols, const int64_t* ld,

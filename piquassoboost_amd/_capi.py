@@ -210,8 +210,9 @@ def permanent(A, algo: int = ALGO_BBFG, precision: int = PREC_DOUBLE) -> complex
 
 def permanent_list(mats, algo: int = ALGO_BBFG, precision: int = PREC_DOUBLE) -> list:
     """Plain permanents of a list of matrices (any shapes) in one call: each value
-    equals permanent(m, algo, precision) bit for bit; matrices of one shape share a
-    launch (pqb_perm_list)."""
+    equals permanent(m, algo, precision), bit for bit on the FP64 and exact routes; with
+    PREC_INF it is the same sum in another order, rounded once, which differs at most in
+    the last bits of a permanent that cancels by more than 2^45 (pqb_perm_list)."""
     mats = list(mats)
     n = len(mats)
     if n == 0:

@@ -24,6 +24,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <cmath>
 #include <condition_variable>
 #include <cstring>
@@ -201,6 +202,26 @@ static SweepChoice choose_sweep(const double* A, int64_t ld, const PlanScratch& 
     return c;
 }
 
+// Whether the double-double sweep may take the rows of a task (its occupied rows and columns
+// in `sc`) in two parts (RepTask::split), and E with entries below 2^E.  A column sum of at
+// most 40 rows is then below 2^(E+6), so parts on the grid of 2^(E-47) add up exactly in a
+// double; those below it add up to less than 2^(E-42), and are multiples of 2^(E-92) when no
+// entry but zeros is below 2^(E-40), so they do too.
+static bool split_exact(const double* A, int64_t ld, const PlanScratch& sc, int* E) {
+    double most = 0.0, least = HUGE_VAL;
+    for (int64_t r : sc.ri)
+        for (int64_t k : sc.ci)
+            for (int c = 0; c < 2; ++c) {
+                const double v = std::fabs(A[2 * (r * ld + k) + c]);
+                if (!(v <= 0x1p900)) return false;
+                most = std::max(most, v);
+                if (v > 0.0) least = std::min(least, v);
+            }
+    if (!(most >= 0x1p-900)) return false;
+    *E = std::ilogb(most) + 1;
+    return least >= std::ldexp(1.0, *E - 40);
+}
+
 // choice: the sweep (NULL: without expansion).
 int plan_task(const double* A, int64_t rows, int64_t cols, int64_t ld, const int64_t* rmult,
               const int64_t* cmult, uint64_t target_L, TaskPlan& P, const SweepChoice* choice, bool plain) {
@@ -343,26 +364,6 @@ static void fill_xrow(const TaskPlan& P, double* x) {
     }
 }
 
-// Whether the double-double sweep may take a plan's rows in two parts (RepTask::split), and
-// E with entries below 2^E.  A column sum of at most 40 rows is then below 2^(E+6), so parts
-// on the grid of 2^(E-47) add up exactly in a double; those below it add up to less than
-// 2^(E-42), and are multiples of 2^(E-92) when no entry but zeros is below 2^(E-40), so they
-// do too.
-static bool split_exact(const TaskPlan& P, int* E) {
-    double most = 0.0, least = HUGE_VAL;
-    for (int r = 0; r < P.R; ++r)
-        for (int s = 0; s < P.NS; ++s)
-            for (int c = 0; c < 2; ++c) {
-                const double v = std::fabs(P.entry(r, s)[c]);
-                if (!(v <= 0x1p900)) return false;
-                most = std::max(most, v);
-                if (v > 0.0) least = std::min(least, v);
-            }
-    if (!(most >= 0x1p-900)) return false;
-    *E = std::ilogb(most) + 1;
-    return least >= std::ldexp(1.0, *E - 40);
-}
-
 // The parts of the rows and of the base.  A chunk's `group` lanes have `own` slots each, lane
 // q from q * own on; a row holds the lanes' k-th slots side by side, (re_hi, re_lo) of each,
 // then (im_hi, im_lo), so that a load of the wave is one line.
@@ -371,9 +372,7 @@ static void fill_split(const TaskPlan& P, int group, double* out) {
     auto at = [&](int r, int s, int c) {
         return out + 2 * ((((size_t)r * own + s % own) * 2 + c) * group + s / own);
     };
-    int E = 0;
-    (void)split_exact(P, &E);
-    const double shift = std::ldexp(1.5, E + 5);  // ulp 2^(E-47)
+    const double shift = std::ldexp(1.5, P.split_top + 5);  // ulp 2^(E-47), E as in split_exact
     std::fill(out, out + (size_t)4 * (P.R + 1) * slots, 0.0);
     for (int s = P.NS; s < slots; ++s) at(P.R, s, 0)[0] = 1.0;  // a padding slot's factor
     for (int r = 0; r < P.R; ++r) {
@@ -745,6 +744,26 @@ static uint64_t choose_L(double S, double total, int64_t lanes, bool fp64, doubl
     return (uint64_t)L;
 }
 
+// Chunks of the double-double sweep in flight on the whole grid.
+static int64_t dd_chunks(Engine& E, int max_ns, bool split) {
+    const int range = rep_dd_range_for(max_ns, split);
+    return (int64_t)batch_grid_locked(E, range) * (kBlock / kWave) * rep_dd_walkers(range);
+}
+
+constexpr int kUnsplit = INT_MIN;  // in place of a task's split_top
+
+// Column sums of the tasks whose rows can be split from which on they are swept apart from
+// others that cannot: it saves them 5 of 11 instructions a component and costs a further
+// upload, sweep and wait.  Lists of some of the first kind and one of the second, together /
+// apart, us: 8 x 16 (4e6) 100 / 164, 200 and 3 x 12 (5e6) 345 / 485, 8 x 20 (8e7) 440 / 430,
+// 3 x 24 (6e8) 1803 / 1648, 32 x 22 (1.5e9) 4320 / 2970.
+constexpr double kApartWork = 0x1p26;
+
+static void set_split(TaskPlan& P, int top) {
+    P.split = true;
+    P.split_top = top;
+}
+
 // The matrix of every task of a batch, where they share one.
 struct SharedMatrix {
     const double* A = nullptr;
@@ -753,7 +772,7 @@ struct SharedMatrix {
 };
 
 // Run a list of planned tasks; results (6 doubles each) into out6.  dd: the
-// double-double sweep (a chunk per quad of lanes) instead of the FP64 one.
+// double-double sweep (a chunk per group of lanes) instead of the FP64 one.
 static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector<double>& out6, bool dd,
                             const SharedMatrix& shared = SharedMatrix()) {
     BatchBuffers& B = batch_of(E);
@@ -777,36 +796,30 @@ static int run_tasks_locked(Engine& E, std::vector<TaskPlan>& plans, std::vector
         max_ns = std::max(max_ns, plans[i].NS);
     }
     if (live.empty()) return PQB_OK;
-    std::atomic<bool> split{dd};
-    if (dd)
-        host_parallel((int64_t)live.size(), 256, [&](int64_t lo, int64_t hi) {
-            int E = 0;
-            for (int64_t k = lo; k < hi && split; ++k)
-                if (!split_exact(plans[live[(size_t)k]], &E)) split = false;
-        });
-    const int range = dd ? rep_dd_range_for(max_ns, split) : rep_range_for(min_ns, max_ns);
-    if (range < 0) {
-        // split at 32 slots and run the two halves
-        std::vector<TaskPlan> lo, hi;
-        std::vector<size_t> ilo, ihi;
+    // tasks that no launch takes together run one kind after the other: up to 32 slots and more;
+    // double-double, split rows and others
+    auto apart = [&](auto first) {
+        std::vector<TaskPlan> part[2];
+        std::vector<size_t> index[2];
         for (size_t i : live) {
-            if (plans[i].NS <= 32) {
-                lo.push_back(plans[i]);
-                ilo.push_back(i);
-            } else {
-                hi.push_back(plans[i]);
-                ihi.push_back(i);
-            }
+            const int which = first(plans[i]) ? 0 : 1;
+            part[which].push_back(plans[i]);
+            index[which].push_back(i);
         }
-        std::vector<double> olo, ohi;
-        int st = run_tasks_locked(E, lo, olo, dd, shared);
-        if (st) return st;
-        st = run_tasks_locked(E, hi, ohi, dd, shared);
-        if (st) return st;
-        for (size_t k = 0; k < ilo.size(); ++k) std::copy(&olo[6 * k], &olo[6 * k] + 6, &out6[6 * ilo[k]]);
-        for (size_t k = 0; k < ihi.size(); ++k) std::copy(&ohi[6 * k], &ohi[6 * k] + 6, &out6[6 * ihi[k]]);
-        return PQB_OK;
-    }
+        for (int which = 0; which < 2; ++which) {
+            std::vector<double> o;
+            const int st = run_tasks_locked(E, part[which], o, dd, shared);
+            if (st) return st;
+            for (size_t k = 0; k < index[which].size(); ++k)
+                std::copy(&o[6 * k], &o[6 * k] + 6, &out6[6 * index[which][k]]);
+        }
+        return (int)PQB_OK;
+    };
+    const bool split = plans[live[0]].split;
+    for (size_t i : live)
+        if (plans[i].split != split) return apart([](const TaskPlan& P) { return P.split; });
+    const int range = dd ? rep_dd_range_for(max_ns, split) : rep_range_for(min_ns, max_ns);
+    if (range < 0) return apart([](const TaskPlan& P) { return P.NS <= 32; });
 
     // ---- work items ----
     std::vector<RepItem> items;
@@ -1115,6 +1128,7 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
     std::vector<TaskPlan> plans((size_t)ntasks);
     std::vector<SweepChoice> choices((size_t)ntasks);
     std::vector<int> photons((size_t)ntasks, 0);
+    std::vector<int> tops(dd ? (size_t)ntasks : 0, kUnsplit);  // TaskPlan::split_top
     // Validation and planning are per task and independent: large batches run
     // them on host threads (4096 tasks are milliseconds of host work either
     // way).  Errors come back per task; the first one by task index is
@@ -1142,6 +1156,8 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
                 compact_occupations(tasks[i].rows, tasks[i].cols, tasks[i].row_mult, tasks[i].col_mult, sc, &n, &nc);
                 choices[(size_t)i] = choose_sweep(tasks[i].A, tasks[i].ld, sc, !dd);
                 photons[(size_t)i] = (int)n;
+                int top = 0;
+                if (dd && split_exact(tasks[i].A, tasks[i].ld, sc, &top)) tops[(size_t)i] = top;
             } catch (const std::exception& ex) {
                 pst[(size_t)i] = PQB_ERR_DEVICE;
                 perr[(size_t)i] = std::string("internal error: ") + ex.what();
@@ -1153,11 +1169,22 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
             t_err = (ntasks > 1 ? "task " + std::to_string(i) + ": " : std::string()) + perr[(size_t)i];
             return pst[(size_t)i];
         }
-    double total = 0.0;
-    int max_photons = 1;  // = the largest slot count of the batch
+    // of the tasks that run together: all of them; double-double, those whose rows are split
+    // [1] and those whose are not [0]
+    double total[2] = {0.0, 0.0};
+    int max_photons[2] = {1, 1};  // = their largest slot count
+    auto kind = [&](int64_t i) { return dd && tops[(size_t)i] != kUnsplit; };
+    if (dd) {
+        double work = 0.0;
+        bool others = false;
+        for (int64_t i = 0; i < ntasks; ++i)
+            if (kind(i)) work += choices[(size_t)i].steps * photons[(size_t)i];
+            else others = others || !plans[(size_t)i].trivial;
+        if (others && work < kApartWork) std::fill(tops.begin(), tops.end(), kUnsplit);
+    }
     for (int64_t i = 0; i < ntasks; ++i) {
-        total += choices[(size_t)i].steps;
-        max_photons = std::max(max_photons, photons[(size_t)i]);
+        total[kind(i)] += choices[(size_t)i].steps;
+        max_photons[kind(i)] = std::max(max_photons[kind(i)], photons[(size_t)i]);
     }
     bool any_sweep = false;
     for (const TaskPlan& P : plans) any_sweep = any_sweep || !P.trivial;
@@ -1178,10 +1205,10 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
         if (st || done) return st;
     }
     // chunks in flight: a lane each (FP64), a group of lanes each (double-double)
-    const int dd_range = rep_dd_range_for(max_photons, true);
-    const int64_t lanes = dd ? (int64_t)batch_grid_locked(E, dd_range) * (kBlock / kWave) * rep_dd_walkers(dd_range)
-                             : (int64_t)batch_grid_locked(E, 2) * kBlock;
-    const bool large_batch = total >= 1024.0 * (double)lanes;  // steps per lane
+    int64_t lanes[2];
+    for (int k = 0; k < 2; ++k)
+        lanes[k] = dd ? dd_chunks(E, max_photons[k], k == 1) : (int64_t)batch_grid_locked(E, 2) * kBlock;
+    const bool large_batch = total[0] >= 1024.0 * (double)lanes[0];  // steps per lane
     auto plan_range = [&](int64_t lo, int64_t hi) {
         for (int64_t i = lo; i < hi; ++i) {
             if (plans[(size_t)i].trivial) continue;
@@ -1195,13 +1222,14 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
                 (!dd && large_batch && photons >= 0 && photons <= PQB_MAX_COLS) ? g_walk[photons].load() : 0;
             const uint64_t L = L_override > 0 ? (uint64_t)L_override
                                : tuned > 0    ? (uint64_t)tuned
-                                              : choose_L(choices[(size_t)i].steps, total, lanes, !dd,
+                                              : choose_L(choices[(size_t)i].steps, total[kind(i)], lanes[kind(i)], !dd,
                                                          step_cost(choices[(size_t)i].degree, (int)photons) /
                                                              step_cost(0, (int)photons));
             try {  // nothing may escape a worker thread
                 pst[(size_t)i] = plan_task(tasks[i].A, tasks[i].rows, tasks[i].cols, tasks[i].ld,
                                            tasks[i].row_mult, tasks[i].col_mult, L, plans[(size_t)i], &choices[(size_t)i]);
                 if (pst[(size_t)i]) perr[(size_t)i] = t_err;  // t_err is per thread
+                if (kind(i)) set_split(plans[(size_t)i], tops[(size_t)i]);
             } catch (const std::exception& ex) {
                 pst[(size_t)i] = PQB_ERR_DEVICE;
                 perr[(size_t)i] = std::string("internal error: ") + ex.what();
@@ -1232,13 +1260,28 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
 int run_plain_dd_list_locked(Engine& E, const double* const* A, const int* R, const int* C, const int64_t* ld,
                              int64_t n, double* out) {
     std::vector<TaskPlan> plans((size_t)n);
+    std::vector<int> tops((size_t)n, kUnsplit);
+    const std::vector<int64_t> ones(PQB_MAX_COLS + 1, 1);
+    double work = 0.0;
+    bool others = false;
     for (int64_t k = 0; k < n; ++k) {
-        const std::vector<int64_t> rm((size_t)R[k], 1), cm((size_t)C[k], 1);
+        int64_t rows = 0, cols = 0;
+        compact_occupations(R[k], C[k], ones.data(), ones.data(), plan_scratch(), &rows, &cols);
+        if (split_exact(A[k], ld[k], plan_scratch(), &tops[(size_t)k])) {
+            work += std::ldexp((double)C[k], R[k] - 1);
+        } else {
+            tops[(size_t)k] = kUnsplit;
+            others = true;
+        }
+    }
+    if (others && work < kApartWork) std::fill(tops.begin(), tops.end(), kUnsplit);
+    for (int64_t k = 0; k < n; ++k) {
         const double S = std::ldexp(1.0, R[k] - 1);
-        const int range = rep_dd_range_for(C[k], true);  // the slots are the columns
-        const int64_t walkers = (int64_t)batch_grid_locked(E, range) * (kBlock / kWave) * rep_dd_walkers(range);
-        const int st = plan_task(A[k], R[k], C[k], ld[k], rm.data(), cm.data(), choose_L(S, S, walkers, false),
+        const bool split = tops[(size_t)k] != kUnsplit;
+        const int64_t chunks = dd_chunks(E, C[k], split);  // the slots are the columns
+        const int st = plan_task(A[k], R[k], C[k], ld[k], ones.data(), ones.data(), choose_L(S, S, chunks, false),
                                  plans[(size_t)k], nullptr, true);
+        if (split) set_split(plans[(size_t)k], tops[(size_t)k]);
         if (st) return n > 1 ? fail(st, "matrix " + std::to_string(k) + ": " + t_err) : st;
     }
     std::vector<double> out6;

@@ -620,10 +620,12 @@ int plain_entry(const double* A, int64_t rows, int64_t cols, int64_t ld, int alg
 // ------------------------------------------------------------- list entry --
 //
 // Plain permanents of a list of host matrices (any mix of shapes).  Each
-// matrix gets the value pqb_perm gives it; the work is regrouped:
+// matrix gets the value pqb_perm gives it (double-double: the same sum, in another
+// order before it is rounded); the work is regrouped:
 //  * exact-route integer matrices: one exact sweep each (as per call);
 //  * double-double route: every matrix planned as a single call would plan it,
-//    all of them in one batched launch;
+//    all of them in one batched launch (in two, where many matrices whose rows
+//    are split stand beside others, see kApartWork in batch.hip);
 //  * FP64 route: one launch for all the shapes that are small, else one per
 //    distinct shape with one grid row (blockIdx.y) per matrix, each matrix
 //    with the single-call launch plan -- so every value is bit-identical to

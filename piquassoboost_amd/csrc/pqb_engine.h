@@ -67,6 +67,8 @@ struct TaskPlan {
     uint64_t L = 1;            // walk length
     uint64_t nchunks = 1;
     int degree = 0;            // RepTask::degree
+    bool split = false;        // double-double sweep over split rows (RepTask::split):
+    int split_top = 0;         // entries below 2^split_top
     uint32_t xrow = 0;         // expanded: the expanded row (column when transposed)
     double scale = 1.0;        // 2^-(N-1); expanded: D! 2^-(N-D-1)
     uint32_t row[kMaxRepRows];    // R rows of the matrix (columns when transposed)
@@ -89,7 +91,7 @@ struct Engine;
 // Plain permanent (1 <= rows <= cols + 1) by the double-double sweep; context locked.
 int run_plain_dd_locked(Engine& E, const double* A, int R, int C, int64_t ld, double* out);
 // `n` such permanents (matrix k: A[k], R[k] x C[k], stride ld[k]), each planned as
-// run_plain_dd_locked plans it, in one batched launch; out: 2 doubles each.
+// run_plain_dd_locked plans it, in one or two batched launches; out: 2 doubles each.
 int run_plain_dd_list_locked(Engine& E, const double* const* A, const int* R, const int* C, const int64_t* ld,
                              int64_t n, double* out);
 int list_entry(const double* const* A, const int64_t* rows, const int64_t* cols, const int64_t* ld,

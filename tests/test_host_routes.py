@@ -85,3 +85,40 @@ assert launched() == []
 {first}
 assert C.batch_replay_ms(2) > 0.0
 """)
+
+
+DOUBLE_DOUBLE = """
+def wide(n, seed):
+    A = matrix(n, seed)
+    A[1, 2] = 1e-17  # a rounding residue
+    return A
+def sweeps(calls):
+    return [k[k.index("rep_dd_kernel"):].split("EEEv")[0] for k in calls if "rep_dd_kernel" in k]
+SPLIT, WHOLE = "rep_dd_kernelILi2ELi12ELb1", "rep_dd_kernelILi4ELi8ELb0"  # up to 24 slots
+"""
+
+
+def test_split_and_whole_rows_of_a_list_are_swept_apart(runtime):
+    """In the double-double sweeps a matrix whose entries are too far apart to be split does
+    not take many others of its list or batch along; a few small ones stay with it."""
+    run(runtime, DOUBLE_DOUBLE + """
+near, far, small = [matrix(22, k) for k in range(2)], [wide(22, k) for k in range(2)], [matrix(20, k) for k in range(6)]
+C.permanent(near[0], precision=C.PREC_INF), C.permanent(far[0], precision=C.PREC_INF)
+assert sweeps(launched()) == [SPLIT, WHOLE]
+for mats, want in ((near, [SPLIT]), (far, [WHOLE]), ([near[0], far[0], near[1], far[1]], [SPLIT, WHOLE]),
+                   (small, [SPLIT]), (small + far, [WHOLE])):
+    C.permanent_list(mats, precision=C.PREC_INF)
+    assert sweeps(launched()) == want
+    ones = np.ones(22, np.int64)
+    C.permanent_batch([(A, ones[:len(A)], ones[:len(A)]) for A in mats], precision=C.PREC_INF)
+    assert sweeps(launched()) == want
+""")
+
+
+def test_repeated_tasks_of_more_than_32_slots_are_swept_apart(runtime):
+    run(runtime, """
+def task(m): return (matrix(6, m), [m] * 6, [m] * 6)
+C.permanent_batch([task(3), task(6), task(4)])
+calls = [k[k.index("rep_batch_kernel"):].split("EEEv")[0] for k in launched() if "rep_batch_kernel" in k]
+assert calls == ["rep_batch_kernelILi1ELi26", "rep_batch_kernelILi33ELi40"]
+""")
