@@ -1,5 +1,5 @@
 // Permanents of at most kTinySteps signed terms, one block per matrix: plain ones of up
-// to 12 rows and repeated-row ones of few steps (the sums of BBFGPermanentCalculator.hpp:
+// to 11 rows and repeated-row ones of few steps (the sums of BBFGPermanentCalculator.hpp:
 // 87-235 and BBFGPermanentCalculatorRepeated.hpp:116-307).
 //
 // Such a call is latency: copies, launches and their gaps, not arithmetic.  Everything is

@@ -122,3 +122,20 @@ C.permanent_batch([task(3), task(6), task(4)])
 calls = [k[k.index("rep_batch_kernel"):].split("EEEv")[0] for k in launched() if "rep_batch_kernel" in k]
 assert calls == ["rep_batch_kernelILi1ELi26", "rep_batch_kernelILi33ELi40"]
 """)
+
+
+def test_limits_of_the_one_block_kernel(runtime):
+    run(runtime, """
+def kernels():
+    return [next(k for k in ("tiny_kernel", "tiny_mixed", "plain_sweep", "plain_prep", "plain_mixed") if k in name)
+            for name in launched()]
+for rows, cols, want in ((11, 11, ["tiny_kernel"]), (11, 24, ["tiny_kernel"]), (11, 25, ["plain_sweep"]),
+                         (12, 11, ["plain_sweep"]), (12, 12, ["plain_sweep"])):
+    C.permanent(matrix(rows, 1, cols), precision=C.PREC_FP64)
+    assert kernels() == want, (rows, cols)
+for count, want in ((256, ["tiny_kernel"]), (257, ["plain_prep", "plain_sweep"])):
+    buffers = [np.zeros(n) for n in (2 * 25 * count, 6 * count, C.batch_device_workspace_bytes(count, 5, 5) // 8 + 1)]
+    A, out, work = (b.ctypes.data for b in buffers)
+    C.permanent_batch_device(A, count, 5, 5, out, work, buffers[2].nbytes, 0)
+    assert kernels() == want, count
+""")
