@@ -213,15 +213,8 @@ __global__ __launch_bounds__(256) void rep_layout_kernel(RepTask* tasks) {
         for (int d = 0; d < T.nlow; ++d) {
             const double m = (double)(T.lrad[d] - 1);
             const double2 a = A[(1 + d) * NS + lane];
-            if (expand) {
-                b.x += m * a.x;
-                b.y += m * a.y;
-            } else {  // rounded as on the host (fill_base in batch.hip)
-                double px = m * a.x, py = m * a.y;
-                asm volatile("" : "+v"(px), "+v"(py));
-                b.x += px;
-                b.y += py;
-            }
+            b.x += m * a.x;  // two roundings, as on the host (fill_base in batch.hip)
+            b.y += m * a.y;
         }
         const_cast<double2*>(T.base)[lane] = b;
     }
