@@ -9,7 +9,8 @@ device-pointer entry point of libpqb_perm.so on torch's current stream.
 
 Prints one JSON line with the throughput, the FP64 roofline fraction of the
 sweep kernel (algorithmic flops (8n-4) 2^(n-1) per permanent over the mean
-launch time measured with HIP events on the launch stream), and a CPU
+launch time measured with HIP events on the launch stream; the expansion along
+one row does fewer, so it is a speed in units of the plain sum), and a CPU
 baseline: the restated reference TBB sweep (double, std::thread, one chunk per
 4 x threads as BBFGPermanentCalculator.hpp:120-134) timed on this host.  The same
 line carries the other workloads' legs: the 30-photon repeated-row permanent, the
@@ -152,7 +153,9 @@ def cpu_baseline(A: np.ndarray, budget_s: float = 20.0) -> dict:
 def batched_leg() -> dict:
     """4096 uneven repeated-row permanents (n in [8, 26], output
     multiplicities 1/2/3 with p = .7/.2/.1) from one 100-mode Haar unitary, as
-    one batched launch against 4096 per-call launches on the same GPU."""
+    one batched launch against 4096 per-call launches on the same GPU.  Steps and
+    operations are those of the sweep over all rows; tasks that are expanded along
+    a row do fewer, so `replay_tflops` compares speeds and is not a utilisation."""
     from piquassoboost_amd import _capi as C
     from piquassoboost_amd.sampling.utilities import adapt_interferometer, uneven_batch
 
@@ -214,8 +217,8 @@ def thirty_photon_task():
 
 def walk_sweep(walks=(24, 48, 72, 144, 216, 432), reps: int = 30) -> dict:
     """The 30-photon transition at several walk lengths (Gray steps per chunk): the
-    walk the digit packing gives for each target, the chunk count, and the best of two
-    averages of `reps` replays of the captured launch."""
+    walk the digit packing gives for each target and the chunk count (of the sweep over
+    all rows), and the best of two averages of `reps` replays of the captured launch."""
     from piquassoboost_amd import _capi as C
 
     A, rows, cols = thirty_photon_task()
@@ -236,7 +239,8 @@ def repeated_leg(reps: int = 10) -> dict:
     0..29, 18 distinct output modes with multiplicities 1 + Multinomial(12, 1/18), seeded
     60-mode Haar unitary (seed 1004); the compact 18 x 30 matrix.  GPU per call (host API,
     wall) and per replay of the captured launch; the restated reference sweep (double,
-    std::thread) on the host cores beside it."""
+    std::thread) on the host cores beside it.  Steps and operations are those of the
+    sweep over all rows (the task is expanded along a row and does fewer)."""
     from piquassoboost_amd import _capi as C
 
     sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))

@@ -113,10 +113,10 @@ int pqb_perm(const double* A, int64_t rows, int64_t cols, int64_t ld, int algo,
  * permanent.  Replaces the list surface of the plain Python calculator
  * (GlynnPermanentCalculator_Wrapper.hpp:204-293: a list of matrices in, a list
  * of permanents out, one calculator call per matrix).  Same algo and precision
- * codes, edge rules and routes as pqb_perm; the work is regrouped: matrices
- * of one shape on the FP64 route share one launch (a grid row per matrix, each
- * with the launch plan of a single call, so each value is bit-identical to
- * the pqb_perm call on that matrix), the double-double route (PQB_PREC_INF)
+ * codes, edge rules and routes as pqb_perm; the work is regrouped: on the
+ * FP64 route the small shapes share launches and the matrices of each larger
+ * shape share one (each matrix with the launch plan of a single call, so each
+ * value is bit-identical to the pqb_perm call on that matrix), the double-double route (PQB_PREC_INF)
  * takes one or two batched launches (the correctly rounded sum, as per call,
  * whenever the sum cancels by less than ~2^45), exact-route integer matrices one sweep
  * each.  A failing matrix fails the call; the message names its index.
@@ -205,9 +205,11 @@ int pqb_set_walk_lengths(const int64_t* walk, int64_t count);
  * HIP events around the replays.  No reference counterpart (measurement). */
 int pqb_batch_replay(int iters, double* ms);
 
-/* Host-only plan of one repeated task (no device needed): info[0] = column
- * slots, [1] = rows incl. anchor, [2] = low digits, [3] = high digits,
- * [4] = walk length, [5] = chunks.  All zero when no sweep is needed. */
+/* Host-only plan of the sweep over all rows of one repeated task (no device
+ * needed; a task that is expanded along a row walks the others only, and a
+ * single one of few steps is evaluated by one block): info[0] = column slots,
+ * [1] = rows incl. anchor, [2] = low digits, [3] = high digits, [4] = walk
+ * length, [5] = chunks.  All zero when no sweep is needed. */
 int pqb_repeated_plan(const double* A, int64_t rows, int64_t cols, int64_t ld,
                       const int64_t* row_mult, const int64_t* col_mult,
                       int64_t walk_length, int64_t* info);
@@ -254,10 +256,12 @@ int pqb_perm_batch_device(const double* dA, int64_t count, int64_t rows, int64_t
                           void* d_work, size_t work_bytes, void* stream);
 
 /* ---- launch plan introspection (host only, no device needed) --------------
- * Writes the sweep decomposition chosen for a rows x cols plain permanent:
- * plan[0] = K (Gray bits walked per group), plan[1] = B (lane bits),
- * plan[2] = H (group bits), plan[3] = launched waves, plan[4] = threads per
- * block, plan[5] = blocks.  `waves_resident` = waves the device keeps
+ * Writes the decomposition of the sweep over all rows of a rows x cols plain
+ * permanent (a square matrix that is expanded along a row, from 2^24 sign
+ * vectors on, is swept over one row fewer with its own waves; a matrix of up to
+ * 11 rows is evaluated by one block): plan[0] = K (Gray bits walked per
+ * group), plan[1] = B (lane bits), plan[2] = H (group bits), plan[3] =
+ * launched waves, plan[4] = threads per block, plan[5] = blocks.  `waves_resident` = waves the device keeps
  * resident for this kernel (0 = ask the device). */
 int pqb_plain_plan(int64_t rows, int64_t cols, int64_t waves_resident, int64_t* plan);
 

@@ -1217,7 +1217,10 @@ int batch_entry(const pqb_task* tasks, int64_t ntasks, int algo, int precision, 
             // The autotuned walk lengths are measured for the FP64 sweep on a large batch
             // (thousands of steps per lane); a small batch, a single task above all, keeps
             // the automatic rule (a 6e6-step task at the tuned 1024-step walk left all but
-            // ~6000 lanes idle: 0.32 ms against 0.10 ms).
+            // ~6000 lanes idle: 0.32 ms against 0.10 ms).  They were measured on the sweep over
+            // all rows and hold for expanded tasks as they are: replays of 4096 tasks of 8..26 /
+            // 18..26 / 14..22 photons 6.78 / 12.78 / 1.09 ms, with walks half as long 6.76 / 12.88 /
+            // 1.08, with the automatic rule (which scales by the step's cost) 6.73 / 12.93 / 1.09.
             const int64_t tuned =
                 (!dd && large_batch && photons >= 0 && photons <= PQB_MAX_COLS) ? g_walk[photons].load() : 0;
             const uint64_t L = L_override > 0 ? (uint64_t)L_override

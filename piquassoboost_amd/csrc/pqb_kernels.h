@@ -30,7 +30,8 @@ struct PlainParams {
     unsigned* done;      // host memory, set to 1 after `out` (NULL: not wanted)
 };
 
-// Several shapes in one launch of blocks of 256 threads (plain_mixed_kernel).
+// Several shapes in one launch of blocks of 256 threads (plain_mixed_kernel).  The upper
+// limit was measured on one list (see there), not over many.
 constexpr int kMixedMinCols = 11, kMixedMaxCols = 21, kMixedShapes = 16;
 struct PlainMixed {
     PlainParams p[kMixedShapes];

@@ -125,7 +125,7 @@ class GlynnPermanentCalculator_wrapper:
         algo, prec = PLAIN_LIBS[self.lib]
         if isinstance(self._matrix, list):
             # one call for the whole list (the reference loops over the matrices,
-            # GlynnPermanentCalculator_Wrapper.hpp:210-237): one launch per shape
+            # GlynnPermanentCalculator_Wrapper.hpp:210-237): few launches, not one per matrix
             return _run(C.permanent_list, self._matrix, algo, prec)
         return _run(C.permanent, self._matrix, algo, prec)
 
